@@ -92,7 +92,7 @@ struct ProfCall {
 struct Layout {
   size_t w8_xq, w8_xs, w8_act, w8_acts, w8_aq, w8_as, w8_aqs, w8_ass, w8_o;
   size_t stack_flags, stack_cap, stack_end;
-  size_t sync, sync_words, slots, tiles2, n_tiles2, logits, sg_logit, idx, w, sg, xperm, chunk_counts, chunk_masks, rank, counts, offsets, perm, inv,
+  size_t sync, sync_words, slots, logits, sg_logit, idx, w, sg, xperm, chunk_counts, chunk_masks, rank, counts, offsets, perm, inv,
       ptok, tiles, n_tiles, ticket, act, act_s, o, h, wnorm, xsum, asum, asum_s, total;
 };
 
@@ -150,16 +150,14 @@ Layout layout_of(const ainfer_moe_shape &s, int Tm) {
   L.tiles = take((size_t)max_tiles_bound(s, (int)T, DEC_MT) * 16);  // >= every other bound
   L.n_tiles = take(4);
   L.ticket = take(4);
-  L.tiles2 = take((E * ((GEMM_SMALL_MAX + SMALL_MT - 1) / SMALL_MT) + 1) * 16);
-  L.n_tiles2 = take(4);
   L.act = take(T * k * s.inter * 2);
   L.act_s = take(T * (size_t)(s.shared_inter > 0 ? s.shared_inter : 1) * 2);
   L.o = take(T * (k + 1) * H * 2);
   L.h = take(T * H * 2);
   L.wnorm = take(E * 4);
   L.xsum = take(T * (H / 128) * 4);
-  L.asum = take(T * k * (s.inter / 32) * 4);
-  L.asum_s = take(T * (size_t)(s.shared_inter > 0 ? s.shared_inter / 32 : 1) * 4);
+  L.asum = take(T * k * (s.inter / 128) * 4);
+  L.asum_s = take(T * (size_t)(s.shared_inter > 0 ? s.shared_inter / 128 : 1) * 4);
   L.w8_xq = L.w8_xs = L.w8_act = L.w8_acts = L.w8_aq = L.w8_as = L.w8_aqs = L.w8_ass = L.w8_o = 0;
   if (s.precision == AINFER_PRECISION_W4A8) {
     const size_t Is = s.shared_inter > 0 ? s.shared_inter : 128, I = s.inter;
@@ -234,9 +232,6 @@ DispatchOut dispatch_out(const ainfer_moe_shape *s, const Layout &L, void *ws, i
   d.tiles = at<int4>(ws, L.tiles);
   d.n_tiles = at<int32_t>(ws, L.n_tiles);
   d.ticket = at<int32_t>(ws, L.ticket);
-  d.tiles2 = at<int4>(ws, L.tiles2);
-  d.n_tiles2 = at<int32_t>(ws, L.n_tiles2);
-  d.small_max = 0;
   d.mt = SMALL_MT;
   return d;
 }
@@ -281,18 +276,6 @@ ExpertArgs expert_args(const ainfer_moe_shape *s, const ainfer_moe_weights *w, c
   return a;
 }
 
-#ifndef SGU_KBW
-#define SGU_KBW 4
-#endif
-#ifndef SGU_RG
-#define SGU_RG RG_GATE_UP
-#endif
-#ifndef SDN_KBW
-#define SDN_KBW 2
-#endif
-#ifndef SDN_RG
-#define SDN_RG RG_DOWN
-#endif
 // norm (decode path only, ainfer_moe_block_forward): x is the residual stream and
 // the routing kernel applies the RMSNorm itself
 int down_kbw(const ainfer_moe_shape &s) { return down_kbw_of(s); }
@@ -394,9 +377,8 @@ int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, cons
 }
 
 // The expert stage on the dispatch d in the workspace, x in MFMA order
-// written (and its group sums at T >= GEMM_MIN_T): the grouped GEMM there
-// (with the small experts' 16-token tiles), else the streaming items over
-// tiles of DEC_MT tokens.  Leaves o in the workspace: dispatch-position rows,
+// written (and its group sums at T >= GEMM_MIN_T): the grouped GEMM there,
+// else the streaming items over tiles of DEC_MT tokens.  Leaves o in the workspace: dispatch-position rows,
 // the shared expert's at rows T * k + t.
 int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const Layout &L,
                 void *ws, DispatchOut &d, int T, bool gemm, hipStream_t st, ProfCall *pc) {
@@ -429,22 +411,6 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
     g.act = at<uint16_t>(ws, L.act);
     g.act_s = at<uint16_t>(ws, L.act_s);
     HIP_TRY(launch_expert_gemm(0, s->scale_dtype, g, gtiles, st));
-    ExpertArgs sgu, sdn;
-    int small_bound = 0;
-    if (d.small_max > 0) {
-      DispatchOut d2 = d;
-      d2.tiles = d.tiles2;
-      d2.n_tiles = d.n_tiles2;
-      sgu = expert_args(s, w, L, ws, d2, T, 0);
-      sdn = expert_args(s, w, L, ws, d2, T, 1);
-      // tiles2 holds at most E * ceil(small_max / SMALL_MT) tiles, and at
-      // most one partial tile per expert beyond T * k / SMALL_MT full ones
-      const long b1 = (long)E * ((GEMM_SMALL_MAX + SMALL_MT - 1) / SMALL_MT);
-      const long b2 = (long)T * k / SMALL_MT + E;
-      small_bound = (int)(b1 < b2 ? b1 : b2);
-      HIP_TRY(launch_expert_stream(0, s->scale_dtype, sgu, small_bound, SGU_KBW, SGU_RG, SMALL_MT,
-                                   st));
-    }
     pc->end(4);
     g.w0 = w->w_down;
     g.s0 = (const uint16_t *)w->s_down;
@@ -458,10 +424,6 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
     g.a_shared = at<uint16_t>(ws, L.act_s);
     g.o = at<uint16_t>(ws, L.o);
     HIP_TRY(launch_expert_gemm(1, s->scale_dtype, g, gtiles, st));
-    if (d.small_max > 0) {
-      HIP_TRY(launch_expert_stream(1, s->scale_dtype, sdn, small_bound, SDN_KBW, SDN_RG, SMALL_MT,
-                                   st));
-    }
     pc->end(5);
     return AINFER_OK;
   }
@@ -493,7 +455,7 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
   a.a_shared = at<uint16_t>(ws, L.xperm);
   a.act = at<uint16_t>(ws, L.act);
   a.act_s = at<uint16_t>(ws, L.act_s);
-  HIP_TRY(launch_expert_stream(0, s->scale_dtype, a, max_tiles, kbw, RG_GATE_UP, smt, st));
+  HIP_TRY(launch_expert_stream(0, s->scale_dtype, a, max_tiles, kbw, RG_GATE_UP, st));
   pc->end(4);
   // down + combine
   a.w0 = w->w_down;
@@ -507,7 +469,7 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
   a.a_routed = at<uint16_t>(ws, L.act);
   a.a_shared = at<uint16_t>(ws, L.act_s);
   a.o = at<uint16_t>(ws, L.o);
-  HIP_TRY(launch_expert_stream(1, s->scale_dtype, a, max_tiles, kbw_down, RG_DOWN, smt, st));
+  HIP_TRY(launch_expert_stream(1, s->scale_dtype, a, max_tiles, kbw_down, RG_DOWN, st));
   pc->end(5);
   return AINFER_OK;
 }
@@ -562,7 +524,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
       if (T == 1) {
         pc->kernel_events();
         HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, max_tiles_bound(*s, T, DEC_MT), 4,
-                                     DEC_RG_GATE_UP, DEC_MT, st));
+                                     DEC_RG_GATE_UP, st));
         pc->end(4);
       }
       HIP_TRY(launch_experts_decode(s->scale_dtype, dg, gu, dn, at<float>(ws, L.w),
@@ -573,9 +535,9 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
       // bandwidth-bound: three launches whose items hold no waits
       const int mtb = max_tiles_bound(*s, T, DEC_MT);
       pc->kernel_events();
-      HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, mtb, 4, DEC_RG_GATE_UP, DEC_MT, st));
+      HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, mtb, 4, DEC_RG_GATE_UP, st));
       pc->end(4);
-      HIP_TRY(launch_expert_stream(1, s->scale_dtype, dn, mtb, down_kbw(*s), DEC_RG_DOWN, DEC_MT, st));
+      HIP_TRY(launch_expert_stream(1, s->scale_dtype, dn, mtb, down_kbw(*s), DEC_RG_DOWN, st));
       pc->end(5);
       HIP_TRY(combine(d, L));
       pc->end(6);
@@ -602,10 +564,6 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
                                T, H, E, k, has_shared, fused ? &d : nullptr, st,
                                cmask ? at<int32_t>(ws, L.chunk_counts) : nullptr, cmask));
   pc->end(2);
-  // prefill: experts with at most SMALL_MT tokens skip the GEMM (a 128-token
-  // tile costs about half a full one however few tokens it holds) for one
-  // 16-token tile of the streaming kernels, which read their weights once
-  if (gemm) d.small_max = GEMM_SMALL_MAX;
   if (!fused)
     HIP_TRY(launch_dispatch(at<int32_t>(ws, L.idx), T, k, E, mt, has_shared,
                             at<int32_t>(ws, L.chunk_counts), at<int32_t>(ws, L.rank), d, st,
@@ -1072,7 +1030,6 @@ int ainfer_moe_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, c
   const bool gemm = T >= GEMM_MIN_T;
   DispatchOut d = dispatch_out(s, L, ws, T);
   d.mt = gemm ? GEMM_MT : DEC_MT;
-  if (gemm) d.small_max = GEMM_SMALL_MAX;
   ProfCall pc(st);
   pc.start();
   HIP_TRY(launch_xperm(x, at<uint16_t>(ws, L.xperm), gemm ? at<float>(ws, L.xsum) : nullptr, T,

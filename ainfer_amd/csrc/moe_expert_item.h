@@ -39,31 +39,6 @@ __device__ __forceinline__ u32x4 ldg_stream(const void *p) {
   return __builtin_nontemporal_load((const u32x4 *)p);
 }
 
-// Four bf16 pairs (136 + q) for MFMA k-slice j of a 16-byte chunk already
-// xor'ed with 0x88888888.  `magic` is 0x43004300 held in a register so the
-// AND-OR is a single instruction.
-__device__ __forceinline__ u32x4 nib_slice(u32x4 b, int j, uint32_t magic) {
-  const uint32_t mask = 0x000F000Fu;
-  return u32x4{((b[0] >> (4 * j)) & mask) | magic, ((b[1] >> (4 * j)) & mask) | magic,
-               ((b[2] >> (4 * j)) & mask) | magic, ((b[3] >> (4 * j)) & mask) | magic};
-}
-
-// The KBW scales of one row and k-range in one load (KB is a multiple of
-// KBW, so the address is KBW * 2-byte aligned).
-template <int KBW>
-__device__ __forceinline__ void load_scales(const uint16_t *p, uint16_t (&S)[KBW]) {
-  if constexpr (KBW == 4) {
-    const uint2 v = *(const uint2 *)p;
-    S[0] = (uint16_t)v.x; S[1] = (uint16_t)(v.x >> 16);
-    S[2] = (uint16_t)v.y; S[3] = (uint16_t)(v.y >> 16);
-  } else if constexpr (KBW == 2) {
-    const uint32_t v = *(const uint32_t *)p;
-    S[0] = (uint16_t)v; S[1] = (uint16_t)(v >> 16);
-  } else {
-    S[0] = *p;
-  }
-}
-
 __device__ __forceinline__ float silu_mul(float g, float u) {
   return g / (1.0f + expf(-g)) * u;
 }

@@ -7,26 +7,34 @@
 // Restates the reference's INT4 GEMM (ChunkGemm, tools/cmdlist/kernels.cpp:
 // 691-785; gemmMT4, tools/prefill/prefill.cpp:46-129) for bf16 MFMA.
 //
-// Block tile: 128 tokens (one expert tile of the dispatch) x 64 * GEMM_WN
-// weight rows (GEMM_WN = 4: MODE 0 takes 128 gate rows and the matching 128
-// up rows, MODE 1 256 down rows), K in 128-wide groups.  2 x GEMM_WN waves
-// as 2 (tokens) x GEMM_WN (rows); a wave owns 64 x 64 = 4 x 4 tiles of
-// v_mfma_f32_16x16x32_bf16.  Token subtiles past the tile's count skip
-// their MFMAs and A reads.
+// Block tile: at most 64 tokens (one expert tile of the dispatch) x 256
+// weight rows (MODE 0 takes 128 gate rows and the matching 128 up rows, MODE
+// 1 256 down rows), K in 128-wide groups.  4 waves along the rows; a wave
+// owns 64 x 64 = 4 x 4 tiles of v_mfma_f32_16x16x32_bf16.  16-token subtiles
+// past the tile's count cost no MFMA, A read or A copy, so one kernel serves
+// experts of one token (bound by streaming their weights) and of thousands
+// (bound by the loop's issue).
 //
-// Data movement: a 3-stage LDS ring per block (2 stages where K > 2048
-// leaves no room), one barrier per group.  Each
-// stage holds one group of the token rows (128 x 256 B, already in MFMA
+// Why 64 tokens and 4 waves: two such blocks fit a CU (76 KB of LDS each, 2
+// waves per SIMD together), so one block's table loads, barriers and epilogue
+// run under the other's main loop, and a tile holds little padding.  Against
+// one block of 8 waves on 128-token tiles with the experts of at most 32
+// tokens in a 16-token streaming kernel (whole layer, H2048 E512 k10 I512):
+// T = 1500 576 -> 319 us, T = 4096 Zipf 578 -> 477, 4 x 4096 2822 -> 2209;
+// H2560 E96 k6 I896 T = 301 381 -> 191 us.
+//
+// Data movement: a 2-stage LDS ring per block, one barrier per group.  Each
+// stage holds one group of the token rows (64 x 256 B, already in MFMA
 // order) and of the raw INT4 weight rows (64 B each).  Both arrive by
 // global->LDS DMA (global_load_lds_dwordx4: lane i of a wave lands at
-// M0 + 16 i), two groups ahead of the math, with no staging registers.  The
+// M0 + 16 i), one group ahead of the math, with no staging registers.  The
 // DMA is issued from inline asm and its completion tracked with explicit
 // vmcnt waits, so the compiler's conservative waits do not serialise the
 // ring.  Rows are swizzled in 16-byte chunks (A: chunk c of row r at
 // c ^ aswz(r); B: chunk q at q ^ bswz(r)) so that the lanes reading 16 rows
 // at one column hit distinct bank groups.  Scales and the group sums
 // sum_{k in g} a (for x from k_select, for act from this kernel's MODE 0
-// epilogue) are copied to LDS once per block.
+// epilogue) are copied to LDS tables 16 groups at a time.
 #include <type_traits>
 
 #include "moe_common.h"
@@ -47,12 +55,12 @@ extern "C" int ainfer_debug_gemm_trace(void *host) {
 
 namespace {
 
-constexpr int BM = 128;  // tokens per tile
+constexpr int BM = GEMM_MT;  // tokens per tile: one token wave of 64
 
-// Block geometry: 2 x WN waves; BN = 64 * WN weight rows per block.
+// Block geometry: WN waves along the weight rows; BN = 64 * WN rows per block.
 template <int WN, int STAGES_>
 struct Geo {
-  static constexpr int NW = 2 * WN;                  // waves
+  static constexpr int NW = WN;                      // waves
   static constexpr int THREADS = 64 * NW;
   static constexpr int BN = 64 * WN;                 // weight rows
   static constexpr int STAGES = STAGES_;
@@ -63,7 +71,10 @@ struct Geo {
   static constexpr int B_DMA = B_STAGE / (THREADS * 16);
   static constexpr int DMA = A_DMA + B_DMA;
   static constexpr int COLS = 32 * WN;               // MODE 0: act columns per block
+  static_assert(BN == THREADS, "a thread loads the table scales of one weight row");
 };
+// k-groups whose scales and group sums the LDS tables hold at once
+constexpr int TG = 16;
 
 __device__ __forceinline__ void dma16(const void *g, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
@@ -151,14 +162,13 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
-// One item: expert tile lb / n_nblk (its entry t, loaded by the caller one
-// item ahead), column block lb % n_nblk.
+// One item: expert tile lb / n_nblk (its entry t), column block lb % n_nblk.
 template <int SD, int MODE, int WN, int STAGES_>
 __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const int4 t) {
   using Gm = Geo<WN, STAGES_>;
   constexpr int BN = Gm::BN, STAGES = Gm::STAGES, A_STAGE = Gm::A_STAGE, STAGE = Gm::STAGE;
   constexpr int NW = Gm::NW, THREADS = Gm::THREADS, COLS = Gm::COLS;
-  // dynamic LDS: STAGES x (A | B) ring, scales[G][BN] fp16, xs[G][BM] fp32
+  // dynamic LDS: STAGES x (A | B) ring, scales[TG][BN] fp16, xs[TG][BM] fp32
   // (group-major: a lane's 4 rows are one 16-byte read); the epilogue's
   // staging and row sums reuse the idle ring
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -166,7 +176,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   const int nb = lb % n_nb;
   const int e = t.x, pos0 = t.y, mcnt = t.z;
   const bool shared = e == a.E;
-  // MODE 0: N = act columns (I or Is), block covers 64 of them; MODE 1: N = H, 128 rows
+  // MODE 0: N = act columns (I or Is), block covers COLS of them; MODE 1: N = H, BN rows
   const int N = MODE == 0 ? (shared ? a.Is : a.I) : a.H;
   const int K = MODE == 0 ? a.H : (shared ? a.Is : a.I);
   const int G = K >> 7;
@@ -174,16 +184,13 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
   uint16_t *sc_lds = (uint16_t *)(lds + STAGES * STAGE);
-  float *xs_lds = (float *)(lds + STAGES * STAGE + ((BN * G * 2 + 15) & ~15));
+  float *xs_lds = (float *)(lds + STAGES * STAGE + BN * TG * 2);
 
   GTRACE(const unsigned long long t0 = __builtin_amdgcn_s_memtime());
   const int tid = tid_opaque();  // per item: nothing lane-dependent is hoisted across items
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
-  // 2 token waves x WN row waves; wave w runs on SIMD w % 4, so each SIMD
-  // hosts waves of both token halves (a tile of <= 64 tokens keeps every
-  // SIMD busy)
-  const int wn = wave % WN, wm = wave / WN;
+  const int wn = wave;
   const int m16 = lane & 15, q = lane >> 4;
 
   // ---- per-thread DMA sources: A_DMA A slots and B_DMA B slots per stage ---
@@ -226,85 +233,77 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     row = min(row, N - 1);
     boff[i] = (uint32_t)row * (uint32_t)rowb + (uint32_t)qq * 16u;
   }
-  // DMA of group g into stage st (normally g % STAGES)
-  auto issue_to = [&](int g, int st) {
-    const uint32_t base = lds0 + (uint32_t)st * STAGE;
+  // 16-token subtiles that hold tokens (block-uniform): A slot i of a stage is
+  // subtile i's rows, so the subtiles past the count are not copied
+  const int nms = __builtin_amdgcn_readfirstlane(min(4, (mcnt + 15) >> 4));
+  static_assert(Gm::A_DMA == 4 && NW == 4, "A slot i holds the rows of token subtile i");
+  // DMA of group g into its ring stage
+  auto issue = [&](int g) {
+    const uint32_t base = lds0 + (uint32_t)(g % STAGES) * STAGE;
 #pragma unroll
     for (int i = 0; i < Gm::A_DMA; ++i)
-      dma16s(aoff[i], abase + g * 256, base + (uint32_t)((i * NW + wave) * 1024));
+      if (i < nms) dma16s(aoff[i], abase + g * 256, base + (uint32_t)((i * NW + wave) * 1024));
 #pragma unroll
     for (int i = 0; i < Gm::B_DMA; ++i)
       dma16s(boff[i], bbase[i] + g * 64, base + A_STAGE + (uint32_t)((i * NW + wave) * 1024));
   };
-  auto issue = [&](int g) { issue_to(g, g % STAGES); };
-
-  // ---- prologue: tables to LDS; groups 0 .. STAGES-2 in flight -------------
-  // Tables: every load is issued before the first use (unrolled, clamped
-  // indices, no per-lane branches), so the block pays one latency, not one
-  // per element.  G <= 32.  Entry idx is (g = idx / rows, row = idx % rows):
-  // consecutive threads write consecutive LDS words (the global reads
-  // gather instead), so the LDS stores are free of bank conflicts.  The
-  // first groups' DMA is issued after the table loads: loads complete in
-  // issue order, so a wait for a table value never waits for the DMA.
-  {
-    constexpr int SC_IT = BN * 32 / THREADS;
-    uint16_t scv[SC_IT];
-#pragma unroll
-    for (int i = 0; i < SC_IT; ++i) {
-      const int idx = tid + i * THREADS;
-      const int r = idx % BN, g = min(idx / BN, G - 1);
-      const uint16_t *sc;
-      int row;
-      if (MODE == 0) {
-        sc = r < COLS ? (shared ? a.ss0 : a.s0 + (size_t)e * N * G)
-                      : (shared ? a.ss1 : a.s1 + (size_t)e * N * G);
-        row = nb * COLS + (r % COLS);
-      } else {
-        sc = shared ? a.ss0 : a.s0 + (size_t)e * N * G;
-        row = nb * BN + r;
-      }
-      scv[i] = sc[(size_t)min(row, N - 1) * G + g];
-    }
-    constexpr int XS_IT = BM * 32 / THREADS;
-    float xv[XS_IT];
+  // ---- tables of groups [g0, g0 + TG): scales [group][B-row] and -136 x the
+  // group sums [group][token row] in LDS.  A thread reads one weight row's
+  // scales (contiguous: 8 bytes per load where G allows it) and four groups
+  // of one token row; all loads are issued before the first LDS store.
+  auto load_tables = [&](int g0) {
+    const int ng = min(TG, G - g0);
+    const int r = tid;  // B-row (BN == THREADS)
+    const uint16_t *sc;
+    int row;
     if (MODE == 0) {
-      int tok[XS_IT];
+      sc = r < COLS ? (shared ? a.ss0 : a.s0 + (size_t)e * N * G)
+                    : (shared ? a.ss1 : a.s1 + (size_t)e * N * G);
+      row = nb * COLS + (r % COLS);
+    } else {
+      sc = shared ? a.ss0 : a.s0 + (size_t)e * N * G;
+      row = nb * BN + r;
+    }
+    sc += (size_t)min(row, N - 1) * G + g0;
+    uint32_t sv[TG / 2];  // packed pairs
+    if ((G & 3) == 0) {
 #pragma unroll
-      for (int i = 0; i < XS_IT; ++i) {
-        const int row = min((tid + i * THREADS) % BM, mcnt - 1);
-        tok[i] = shared ? pos0 + row : a.ptok[pos0 + row];
-      }
-#pragma unroll
-      for (int i = 0; i < XS_IT; ++i) {
-        const int g = min((tid + i * THREADS) / BM, G - 1);
-        xv[i] = a.xsum[(size_t)tok[i] * G + g];
+      for (int j = 0; j < TG / 4; ++j) {
+        const uint2 v = *(const uint2 *)(sc + min(4 * j, ng - 4));
+        sv[2 * j] = v.x;
+        sv[2 * j + 1] = v.y;
       }
     } else {
-      // act partial sums: a.aslots per 128-wide group, added in order
-      const float *asb = shared ? a.asum_s : a.asum;
 #pragma unroll
-      for (int i = 0; i < XS_IT; ++i) {
-        const int idx = tid + i * THREADS;
-        const int row = min(idx % BM, mcnt - 1), g = min(idx / BM, G - 1);
-        const float *as = asb + (size_t)(pos0 + row) * (a.aslots * G) + a.aslots * g;
-        float v = as[0];
-        for (int j = 1; j < a.aslots; ++j) v += as[j];
-        xv[i] = v;
-      }
+      for (int j = 0; j < TG / 2; ++j)
+        sv[j] = (uint32_t)sc[min(2 * j, ng - 1)] | ((uint32_t)sc[min(2 * j + 1, ng - 1)] << 16);
     }
-    issue(0);
-    if (STAGES > 2) issue_to(min(1, G - 1), 1);  // group 1, or a dummy into idle stage 1
+    // thread: token row tid / 4, groups g0 + 4 * (tid % 4) + [0, 4)
+    static_assert(BM * 4 == THREADS && TG == 16, "one thread per (token row, 4 groups)");
+    const int xr = tid >> 2, xg = 4 * (tid & 3);
+    const int rr = min(xr, mcnt - 1);
+    const float *xsrc = MODE == 0 ? a.xsum : (shared ? a.asum_s : a.asum);
+    const int xrow = MODE == 0 && !shared ? a.ptok[pos0 + rr] : pos0 + rr;
+    xsrc += (size_t)xrow * G + g0;
+    float xv[4];
+    if ((G & 3) == 0) {
+      const float4 v = *(const float4 *)(xsrc + min(xg, ng - 4));
+      xv[0] = v.x; xv[1] = v.y; xv[2] = v.z; xv[3] = v.w;
+    } else {
 #pragma unroll
-    for (int i = 0; i < SC_IT; ++i) {
-      const int idx = tid + i * THREADS;
-      if (idx < BN * G) sc_lds[idx] = scv[i];  // [g][r]
+      for (int j = 0; j < 4; ++j) xv[j] = xsrc[min(xg + j, ng - 1)];
     }
 #pragma unroll
-    for (int i = 0; i < XS_IT; ++i) {
-      const int idx = tid + i * THREADS;
-      if (idx < BM * G) xs_lds[idx] = idx % BM < mcnt ? -136.0f * xv[i] : 0.0f;  // [g][row]
+    for (int j = 0; j < TG / 2; ++j) {
+      if (2 * j < ng) sc_lds[2 * j * BN + r] = (uint16_t)sv[j];
+      if (2 * j + 1 < ng) sc_lds[(2 * j + 1) * BN + r] = (uint16_t)(sv[j] >> 16);
     }
-  }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (xg + j < ng) xs_lds[(xg + j) * BM + xr] = xr < mcnt ? -136.0f * xv[j] : 0.0f;
+  };
+  issue(0);
+  load_tables(0);
 
   // B rows of this wave's 4 N-subtiles
   int brow[4];
@@ -336,7 +335,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     // scales of group g.
     auto part_v = [&](int g) {
 #pragma unroll
-      for (int ns = 0; ns < 4; ++ns) sg[ns] = scale_to_f32<SD>(sc_lds[g * BN + brow[ns]]);
+      for (int ns = 0; ns < 4; ++ns) sg[ns] = scale_to_f32<SD>(sc_lds[(g % TG) * BN + brow[ns]]);
 #pragma unroll
       for (int ns = 0; ns < 4; ++ns)
 #pragma unroll
@@ -353,12 +352,12 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     };
     auto part_m = [&](int g, const u32x4 (&bx)[4]) {
       const uint8_t *sa = lds + (g % STAGES) * STAGE;
-      const uint8_t *arow = sa + (wm * 64 + m16) * 256;
+      const uint8_t *arow = sa + m16 * 256;
       // group sums (-136 sum_k a): the first k-slice accumulates onto them
       f32x4 c0[4];
 #pragma unroll
       for (int ms = 0; ms < NMS; ++ms)
-        c0[ms] = *(const f32x4 *)(xs_lds + g * BM + wm * 64 + ms * 16 + 4 * q);
+        c0[ms] = *(const f32x4 *)(xs_lds + (g % TG) * BM + ms * 16 + 4 * q);
       // A fragments one k-slice ahead; the scheduling barrier after each
       // slice keeps the compiler from hoisting all 16 reads (64 VGPRs) to
       // the top, which spills at this register budget
@@ -432,40 +431,23 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     };
 
     u32x4 bx[4];
-    if constexpr (STAGES == 2) {
-      // One barrier per group.  At the top of iteration g every wave has
-      // issued all its MFMAs of group g-1 (they may still be executing) and
-      // has read its last fragment of stage g-1, so after the barrier the DMA
-      // of group g+1 may overwrite that stage.
-      for (int g = 0; g < G; ++g) {
-        wait_vm<0>();  // this thread's DMA of group g (issued one group ago)
-        // stage g complete for every thread (and, at g = 0, the LDS tables)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        block_barrier();
-        if (g + 1 < G) issue(g + 1);
-        load_bx(g, bx);
-        part_v(g);
-        part_m(g, bx);
-      }
-    } else {
-      // Three stages; the barrier that ends iteration g-1 also makes group
-      // g+1 visible, so each wave reads its B chunks of the next group into
-      // registers at the end of a group, and a group starts with the scale
-      // step (VALU) that hides its first LDS reads, then unpacks at once.
-      // The DMA of group g+2 is issued after that barrier into stage
-      // (g+2) % 3, which held group g-1, and every thread waits for it
-      // before the next barrier: one iteration of latency per DMA.
-      asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)" ::: "memory");
-      block_barrier();  // groups 0 and 1 and the LDS tables complete
-      for (int g = 0; g < G; ++g) {
-        if (g + 2 < G) issue(g + 2);
-        load_bx(g, bx);
-        part_v(g);
-        part_m(g, bx);
-        wait_vm<0>();
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    // One barrier per group.  At the top of iteration g every wave has
+    // issued all its MFMAs of group g-1 (they may still be executing) and
+    // has read its last fragment of stage g-1 and its table entries, so after
+    // the barrier the DMA of group g+1 may overwrite that stage and, every TG
+    // groups, the tables may be rewritten.
+    for (int g = 0; g < G; ++g) {
+      wait_vm<0>();  // this thread's DMA of group g (issued one group ago)
+      // stage g complete for every thread (and, at g = 0, the LDS tables)
+      block_barrier();
+      if (g + 1 < G) issue(g + 1);
+      if (g > 0 && g % TG == 0) {
+        load_tables(g);
         block_barrier();
       }
+      load_bx(g, bx);
+      part_v(g);
+      part_m(g, bx);
     }
 #pragma unroll
     for (int ns = 0; ns < 4; ++ns)
@@ -474,13 +456,14 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   };
   // token subtiles of this wave holding tokens of the tile (wave-uniform)
   GTRACE(const unsigned long long t1 = __builtin_amdgcn_s_memtime());
-  const int nms = __builtin_amdgcn_readfirstlane(max(0, min(4, (mcnt - wm * 64 + 15) >> 4)));
-  if (nms > 2)
+  if (nms > 3)
     main_loop(std::integral_constant<int, 4>());
-  else if (nms > 0)
+  else if (nms > 2)
+    main_loop(std::integral_constant<int, 3>());
+  else if (nms > 1)
     main_loop(std::integral_constant<int, 2>());
   else
-    main_loop(std::integral_constant<int, 0>());
+    main_loop(std::integral_constant<int, 1>());
   wait_vm<0>();  // no DMA into the ring remains in flight
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   block_barrier();  // every wave's last read of the ring precedes the staging below
@@ -492,7 +475,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   });
 
   // ---- epilogue -------------------------------------------------------
-  // lane (q, m16) of tile (ms, ns) holds rows wm*64 + ms*16 + 4q + r, column
+  // lane (q, m16) of tile (ms, ns) holds rows ms*16 + 4q + r, column
   // m16.  Results are staged in the (now idle) LDS ring and leave as 16-byte
   // row chunks.
   if (MODE == 0) {
@@ -532,7 +515,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
         const uint32_t send = hi4 ? p01 : p23, own = hi4 ? p23 : p01;
         // lane ^ 4 inside each group of 32 lanes (ds_swizzle bit mode)
         const uint32_t recv = (uint32_t)__builtin_amdgcn_ds_swizzle((int)send, 0x101F);
-        const int row0 = wm * 64 + ms * 16 + 4 * q + (hi4 ? 2 : 0);
+        const int row0 = ms * 16 + 4 * q + (hi4 ? 2 : 0);
         *(uint32_t *)(lds + row0 * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel0);
         *(uint32_t *)(lds + (row0 + 1) * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel1);
       }
@@ -546,7 +529,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
 #pragma unroll
       for (int ms = 0; ms < 4; ++ms)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red_sum[wn * BM + wm * 64 + ms * 16 + 4 * q + r] = rowsum[ms][r];
+        for (int r = 0; r < 4; ++r) red_sum[wn * BM + ms * 16 + 4 * q + r] = rowsum[ms][r];
     __syncthreads();
     uint16_t *dst = shared ? a.act_s : a.act;
     constexpr int CPR = COLS / 8;  // 16-byte chunks per row
@@ -589,7 +572,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
         const uint32_t send = odd ? p01 : p23, own = odd ? p23 : p01;
         const uint32_t recv =
             (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xF, 0xF, false);  // lane ^ 1
-        const int row0 = wm * 64 + ms * 16 + 4 * q + (odd ? 2 : 0);
+        const int row0 = ms * 16 + 4 * q + (odd ? 2 : 0);
         *(uint32_t *)(lds + row0 * OST + cl * 2) = __builtin_amdgcn_perm(recv, own, sel0);
         *(uint32_t *)(lds + (row0 + 1) * OST + cl * 2) = __builtin_amdgcn_perm(recv, own, sel1);
       }
@@ -615,30 +598,19 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   }
 }
 
-// Persistent grid: one block per resident slot (occupancy x CUs) walks the
-// items in rounds of gridDim.x.  Within a round the items a block takes are
-// XCD-contiguous (xcd_remap), so the column blocks of one expert tile run on
-// one XCD at the same time and share its A rows through that L2.  The item
-// count comes from the dispatch on the device; the host sizes the grid from
-// its upper bound.
+// One block per item.  The items a launch's blocks take are XCD-contiguous
+// (xcd_remap over the device's item count, so every XCD gets an equal share
+// whatever the host's tile bound), which keeps the column blocks of one
+// expert tile, and the tiles of one expert, on one XCD: they share A rows and
+// weights through that L2.
 template <int SD, int MODE, int WN, int STAGES_>
-__global__ __launch_bounds__(128 * WN) void k_expert_gemm(GemmArgs a) {
+__global__ __launch_bounds__(64 * WN, 2) void k_expert_gemm(GemmArgs a) {
   const int n_items = *a.n_tiles * a.n_nblk;
-  const int P = gridDim.x, me = xcd_remap(blockIdx.x, P);
-  // the tile entry of the next item is loaded while this one runs (it is a
-  // global load the item's whole prologue would otherwise wait on)
-  int4 t = me < n_items ? a.tiles[me / a.n_nblk] : int4{0, 0, 0, 0};
-  for (int base = 0; base < n_items; base += P) {
-    const int lb = base + me;
-    if (lb >= n_items) break;  // later rounds only hold larger items
-    const int ln = lb + P;
-    const int4 tn = ln < n_items ? a.tiles[ln / a.n_nblk] : t;
-    gemm_item<SD, MODE, WN, STAGES_>(a, lb, t);
-    t = tn;
-    __syncthreads();  // the epilogue's LDS reads precede the next item's DMA
-    GTRACE(if (threadIdx.x == 0 && lb < 16384) g_gtrace[(MODE * 16384 + lb) * 4 + 3] =
-               __builtin_amdgcn_s_memtime());
-  }
+  if ((int)blockIdx.x >= n_items) return;
+  const int lb = xcd_remap(blockIdx.x, n_items);
+  gemm_item<SD, MODE, WN, STAGES_>(a, lb, a.tiles[lb / a.n_nblk]);
+  GTRACE(__syncthreads(); if (threadIdx.x == 0 && lb < 16384) g_gtrace[(MODE * 16384 + lb) * 4 + 3] =
+             __builtin_amdgcn_s_memtime());
 }
 
 // ---------------------------------------------------------------------------
@@ -777,27 +749,17 @@ __global__ __launch_bounds__(256) void k_router_gemm(const uint16_t *__restrict_
   }
 }
 
-constexpr size_t GEMM_LDS_MAX = 160 * 1024;  // LDS per workgroup on gfx950
-
-template <int WN>
-size_t gemm_lds_bytes(int stages, int Gmax) {
-  using Gm = Geo<WN, 2>;
-  return (size_t)stages * Gm::STAGE + (((size_t)Gm::BN * Gmax * 2 + 15) & ~(size_t)15) +
-         sizeof(float) * (size_t)BM * Gmax;
-}
-
 template <int WN, int STAGES_>
 hipError_t launch_geo(int mode, int scale_dtype, GemmArgs a, int max_tiles, hipStream_t s) {
   using Gm = Geo<WN, STAGES_>;
   const int Nmax = mode == 0 ? (a.I > a.Is ? a.I : a.Is) : a.H;
   a.n_nblk = mode == 0 ? (Nmax + Gm::COLS - 1) / Gm::COLS : (Nmax + Gm::BN - 1) / Gm::BN;
-  a.aslots = 128 / Gm::COLS;  // act partial sums per 128-wide group (MODE 0 writes them)
   const long grid = (long)max_tiles * a.n_nblk;
   if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
-  const int Gmax = (mode == 0 ? a.H : (a.I > a.Is ? a.I : a.Is)) / 128;
-  if (Gmax > 32) return hipErrorInvalidValue;  // table loads assume K <= 4096
-  const size_t lds = gemm_lds_bytes<WN>(Gm::STAGES, Gmax);
-  if (lds > GEMM_LDS_MAX) return hipErrorInvalidValue;
+  // the group sums of act: MODE 0 writes one per COLS = 128 columns
+  static_assert(Gm::COLS == 128, "one act sum per k-group");
+  constexpr size_t lds = (size_t)STAGES_ * Gm::STAGE + Gm::BN * TG * 2 + BM * TG * 4;
+  static_assert(2 * lds <= 160 * 1024, "two blocks per CU");
   void (*kern)(GemmArgs);
   if (mode == 0)
     kern = scale_dtype == AINFER_SCALE_FP16 ? k_expert_gemm<AINFER_SCALE_FP16, 0, WN, STAGES_>
@@ -805,16 +767,7 @@ hipError_t launch_geo(int mode, int scale_dtype, GemmArgs a, int max_tiles, hipS
   else
     kern = scale_dtype == AINFER_SCALE_FP16 ? k_expert_gemm<AINFER_SCALE_FP16, 1, WN, STAGES_>
                                             : k_expert_gemm<AINFER_SCALE_BF16, 1, WN, STAGES_>;
-  // resident blocks per CU for this kernel and LDS size, times the CUs
-  int dev = 0, cus = 0, per_cu = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, Gm::THREADS, lds);
-  if (e != hipSuccess) return e;
-  if (per_cu < 1) return hipErrorInvalidConfiguration;
-  const long resident = (long)per_cu * cus;
-  kern<<<(unsigned)(grid < resident ? grid : resident), Gm::THREADS, lds, s>>>(a);
+  kern<<<(unsigned)grid, Gm::THREADS, lds, s>>>(a);
   return hipGetLastError();
 }
 
@@ -840,10 +793,6 @@ hipError_t launch_router_gemm(const void *x, const void *rw, const float *bias, 
 hipError_t launch_expert_gemm(int mode, int scale_dtype, GemmArgs a, int max_tiles,
                               hipStream_t s) {
   if (max_tiles <= 0) return hipSuccess;
-  // the 3-stage ring where its LDS fits (K <= 2048 at GEMM_WN = 4)
-  const int Gmax = (mode == 0 ? a.H : (a.I > a.Is ? a.I : a.Is)) / 128;
-  if (gemm_lds_bytes<GEMM_WN>(3, Gmax) <= GEMM_LDS_MAX)
-    return launch_geo<GEMM_WN, 3>(mode, scale_dtype, a, max_tiles, s);
   return launch_geo<GEMM_WN, 2>(mode, scale_dtype, a, max_tiles, s);
 }
 

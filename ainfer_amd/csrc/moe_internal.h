@@ -37,12 +37,12 @@ struct GemmArgs {
   uint16_t *act, *act_s;      // MODE 0 out
   uint16_t *o;                // MODE 1 out: [Tk + T][H] bf16
   const float *xsum;          // [T][H/128] group sums of x
-  float *asum, *asum_s;       // [Tk][I/32], [T][Is/32] (max) partial sums of act
+  float *asum, *asum_s;       // [Tk][I/128], [T][Is/128] group sums of act (MODE 0 out)
   const int32_t *ptok;
   const int4 *tiles;
   const int32_t *n_tiles;
   int T, k, E, H, I, Is;
-  int n_nblk, aslots;         // set by the launcher
+  int n_nblk;                 // set by the launcher
 };
 // Prefill router: approximate logits (+ bias) and router row norms, tiled bf16 MFMA GEMM.
 // zbuf: zwords 32-bit words zeroed by the kernel (the dispatch counts and
@@ -53,13 +53,9 @@ hipError_t launch_router_gemm(const void *x, const void *rw, const float *bias, 
 hipError_t launch_expert_gemm(int mode, int scale_dtype, GemmArgs a, int max_tiles,
                               hipStream_t s);
 // token-tile height of the prefill GEMM and the T above which it is used
-constexpr int GEMM_MT = 128;
-// experts with at most this many tokens leave the prefill GEMM (0: none)
-#ifndef GEMM_SMALL_MAX
-#define GEMM_SMALL_MAX 32
-#endif
+constexpr int GEMM_MT = 64;
 #ifndef GEMM_WN
-#define GEMM_WN 4       // row waves per GEMM block (2 x GEMM_WN waves)
+#define GEMM_WN 4       // waves per GEMM block, 64 weight rows each
 #endif
 constexpr int GEMM_MIN_T = 256;
 
@@ -73,11 +69,6 @@ struct DispatchOut {
   int4 *tiles;
   int32_t *n_tiles;
   int32_t *ticket;
-  // experts with 1..small_max tokens get SMALL_MT-token tiles in tiles2
-  // instead of tiles (small_max 0: no split)
-  int4 *tiles2;
-  int32_t *n_tiles2;
-  int small_max;
   int mt;  // tokens per tile of dispatch_small_block
 };
 
@@ -158,14 +149,13 @@ bool expert_geometry(int mode, int H, int I, int Is, int pref_kbw, int *KBW, int
 #define DEC_KBW_DOWN 2
 #endif
 // rg: 16-row groups per wave (1, 2 or 4) sharing one load of the token rows;
-// mt: tokens per tile the dispatch produced (DEC_MT: A staged in LDS, or SMALL_MT)
 // The next decode gate/up launch of launch_expert_stream (the DEC_MT items)
 // goes through hipExtLaunchKernel with these start/stop events (one shot).
 void set_expert_launch_events(hipEvent_t start, hipEvent_t stop);
 hipError_t launch_expert_stream(int mode, int scale_dtype, ExpertArgs a, int max_tiles,
-                                int pref_kbw, int rg, int mt, hipStream_t s);
+                                int pref_kbw, int rg, hipStream_t s);
 
-// tile height of the small-M expert kernels
+// most tokens the small selection (k_select_small) takes
 constexpr int SMALL_MT = 16;
 // LDS bytes per wave of a decode expert item (moe_expert_item.h): its A
 // rows (MT x KBW * 256 B), its scales (KBW >= 2: one dword DMA per 256 B),

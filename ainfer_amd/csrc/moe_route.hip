@@ -339,10 +339,7 @@ __global__ __launch_bounds__(64) void k_dispatch_count(const int32_t *__restrict
 // blockDim = NT >= E (512 when E <= 512: twice the registers per thread
 // for the chunk counts).  Also emits the tile list: for each expert with
 // tokens, ceil(count / mt) tiles (expert, first row), experts ascending,
-// then ceil(T / mt) shared-expert tiles (expert id E) when has_shared.  With
-// ds.small_max > 0, an expert with 1..small_max tokens instead gets
-// ceil(count / SMALL_MT) tiles in ds.tiles2 (experts ascending), counted in
-// ds.n_tiles2.
+// then ceil(T / mt) shared-expert tiles (expert id E) when has_shared.
 constexpr int DISPATCH_MAX_CHUNKS = 64;  // 64-token chunks: T <= 4096 per call
 
 template <int NT>
@@ -367,15 +364,10 @@ __global__ __launch_bounds__(NT) void k_dispatch_scan(int32_t *__restrict__ chun
   }
 #pragma unroll
   for (int j = 0; j < DISPATCH_MAX_CHUNKS; ++j) total += u[j];
-  const bool small = ds.small_max > 0 && total > 0 && total <= ds.small_max;
-  const int ntile = (ds.tiles && e < E && !small) ? (total + mt - 1) / mt : 0;
-  const int nsmall = small ? (total + SMALL_MT - 1) / SMALL_MT : 0;
-  // two block scans (integers: exact): token counts, and the big tile count
-  // (low 16 bits) with the small tile count (high bits).  Where tiles are
-  // written (T * k / mt + E tiles at most, mt = 16 only below 256 tokens)
-  // both counts stay below 2^15.
+  const int ntile = (ds.tiles && e < E) ? (total + mt - 1) / mt : 0;
+  // two block scans (integers: exact): token counts and tile counts
   const int ic = wave_scan_incl(total);
-  const int it = wave_scan_incl(ntile | (nsmall << 16));
+  const int it = wave_scan_incl(ntile);
   if (lane == 63) {
     wsum[0][wv] = ic;
     wsum[1][wv] = it;
@@ -391,8 +383,7 @@ __global__ __launch_bounds__(NT) void k_dispatch_scan(int32_t *__restrict__ chun
     tt += a1;
   }
   const int base = bc + ic - total;
-  const int tb = bt + it - (ntile | (nsmall << 16));
-  const int tbase = tb & 0xFFFF, sbase = tb >> 16;
+  const int tbase = bt + it - ntile;
   if (e < E) {
     ds.counts[e] = total;
     ds.offsets[e] = base;
@@ -406,12 +397,9 @@ __global__ __launch_bounds__(NT) void k_dispatch_scan(int32_t *__restrict__ chun
     if (ds.tiles)
       for (int i = 0; i < ntile; ++i)
         ds.tiles[tbase + i] = make_int4(e, base + i * mt, min(mt, total - i * mt), 0);
-    for (int i = 0; i < nsmall; ++i)
-      ds.tiles2[sbase + i] = make_int4(e, base + i * SMALL_MT, min(SMALL_MT, total - i * SMALL_MT), 0);
   }
   if (e == 0) ds.offsets[E] = tc;
-  if (e == 0 && ds.small_max > 0) *ds.n_tiles2 = tt >> 16;
-  const int routed_tiles = tt & 0xFFFF;
+  const int routed_tiles = tt;
   const int nsh = has_shared ? (T + mt - 1) / mt : 0;
   if (ds.tiles)
     for (int i = e; i < nsh; i += blockDim.x)

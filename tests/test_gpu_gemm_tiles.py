@@ -1,0 +1,90 @@
+"""The prefill expert GEMM at the edges of its tiles: experts of 1 to 300
+tokens (every 16-token subtile count, full and partial 64-token tiles), K of
+1, 7, 15, 18 and 32 quantization groups (one and two table windows, odd and
+4-divisible group counts), rows that do not fill a block.
+
+Each expert row is compared with the float64 MLP of the dequantised weights.
+The bound per element is what the arithmetic states: fp32 sums of n exact
+products (n * 2^-24 of the sum of magnitudes), the activation rounded to bf16 (8
+significant bits: half a unit in the last place is at most 2^-8 of the value;
+and 2^-20 for the exp2 / rcp SiLU), the output rounded to bf16 (2^-8).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+COUNTS = {"low": [1, 15, 16, 17, 31, 32, 33, 47, 48, 60], "high": [49, 63, 64, 65, 59]}
+T = 300
+
+
+def routing(counts):
+    """Slot 0: expert i gets counts[i] tokens, scattered; slot 1: expert E - 1 all of them."""
+    rng = np.random.default_rng(5)
+    first = np.repeat(np.arange(len(counts)), counts)
+    assert first.size == T
+    rng.shuffle(first)
+    return first
+
+
+@pytest.mark.parametrize("scales", ["fp16", "bf16"])
+@pytest.mark.parametrize("which", ["low", "high"])
+@pytest.mark.parametrize("H,I,Is", [(4096, 128, 128), (2304, 256, 128), (1920, 896, 0),
+                                    (128, 128, 1920)])
+def test_expert_rows_at_tile_edges(torch, oracle, H, I, Is, which, scales):
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    print(f"[case] gemm tiles H={H} I={I} Is={Is} {which} {scales}", flush=True)
+    E = 12
+    cfg = MoeConfig("tiles", H, E, 2, I, Is, (T,), seed=77)
+    sd = L.SCALE_FP16 if scales == "fp16" else L.SCALE_BF16
+    ly = MoeLayer(cfg, scale_dtype=sd)
+    first = routing(COUNTS[which])
+    idx = np.stack([first, np.full(T, E - 1)], 1).astype(np.int32)
+    x = make_input(cfg, T)
+    o = ly.experts(x, torch.from_numpy(idx).cuda(), ly.workspace(T))
+    torch.cuda.synchronize()
+    got = o.double().cpu()
+    xd = x.double().cpu()
+
+    def mat(pre, name, e, rows, K):
+        w = ly.t[pre[0] + name].cpu().numpy().reshape(-1, rows, K // 2)[e]
+        s = ly.t[pre[1] + name].view(torch.int16).cpu().numpy().view(np.uint16)
+        w = oracle.dequant(w, s.reshape(-1, rows, K // 128)[e], sd, rows, K)
+        return torch.from_numpy(np.asarray(w, np.float64).reshape(rows, K))
+
+    def check(rows, tok, pre, e, inter):
+        g, u, d = mat(pre, "gate", e, inter, H), mat(pre, "up", e, inter, H), mat(pre, "down", e, H, inter)
+        xi = xd[tok]
+        vg, vu = xi @ g.t(), xi @ u.t()
+        eps = 2.0 ** -24
+        dg, du = (H + 300) * eps * (xi.abs() @ g.abs().t()), (H + 300) * eps * (xi.abs() @ u.abs().t())
+        sil = vg / (1 + torch.exp(-vg))
+        act = sil * vu
+        # |silu'| <= 1.1
+        dact = 1.1 * dg * (vu.abs() + du) + sil.abs() * du + act.abs() * (2.0 ** -8 + 2.0 ** -20)
+        ref = act @ d.t()
+        mag = (act.abs() + dact) @ d.abs().t()
+        bound = dact @ d.abs().t() + (inter + 300) * eps * mag
+        bound = bound + 2.0 ** -8 * (ref.abs() + bound) + 1e-30
+        err = (got[rows] - ref).abs()
+        worst = float((err / bound).max())
+        assert worst <= 1.0, (e, len(tok), worst)
+
+    for e in range(len(COUNTS[which])):
+        tok = np.nonzero(first == e)[0]
+        check(tok * 2, tok, ("w_", "s_"), e, I)
+    every = np.arange(T)
+    check(every * 2 + 1, every, ("w_", "s_"), E - 1, I)
+    if Is:
+        check(2 * T + every, every, ("ws_", "ss_"), 0, Is)
