@@ -58,23 +58,24 @@ namespace {
 constexpr int BM = GEMM_MT;  // tokens per tile: one token wave of 64
 
 // Block geometry: WN waves along the weight rows; BN = 64 * WN rows per block.
-template <int WN, int STAGES_>
+template <int WN>
 struct Geo {
   static constexpr int NW = WN;                      // waves
   static constexpr int THREADS = 64 * NW;
   static constexpr int BN = 64 * WN;                 // weight rows
-  static constexpr int STAGES = STAGES_;
-  static constexpr int A_STAGE = BM * 256;           // bytes per group
+  static constexpr int A_SUB = 16 * 256;             // bytes of a 16-token subtile per group
   static constexpr int B_STAGE = BN * 64;            // bytes per group
-  static constexpr int STAGE = A_STAGE + B_STAGE;
-  static constexpr int A_DMA = A_STAGE / (THREADS * 16);  // DMA per thread per stage
+  // one ring stage at NMS token subtiles: A rows, B rows, a dword per B row
+  // holding its scale, the group sums of 64 token rows
+  static constexpr int stage(int nms) { return nms * A_SUB + B_STAGE + BN * 4 + BM * 4; }
+  // two groups in flight where three stages fit (two blocks per CU, 80 KB each)
+  static constexpr int stages(int nms) { return nms <= 2 ? 3 : 2; }
+  static constexpr int RING = 3 * stage(2) > 2 * stage(4) ? 3 * stage(2) : 2 * stage(4);
+  static constexpr int A_DMA = BM * 256 / (THREADS * 16);  // DMA per thread per group
   static constexpr int B_DMA = B_STAGE / (THREADS * 16);
-  static constexpr int DMA = A_DMA + B_DMA;
   static constexpr int COLS = 32 * WN;               // MODE 0: act columns per block
-  static_assert(BN == THREADS, "a thread loads the table scales of one weight row");
+  static_assert(BN == THREADS, "one lane per weight row copies its scales");
 };
-// k-groups whose scales and group sums the LDS tables hold at once
-constexpr int TG = 16;
 
 __device__ __forceinline__ void dma16(const void *g, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
@@ -83,17 +84,25 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds_addr) {
                : "memory", "m0");
 }
 
-// The same with a scalar base address and a 32-bit per-lane offset.  The
-// base must be wave-uniform; it is moved to SGPRs explicitly, since the
-// compiler cannot always prove the uniformity of values loaded per item.
-__device__ __forceinline__ void dma16s(uint32_t off, const void *base, uint32_t lds_addr) {
-  const uint64_t b = (uint64_t)(uintptr_t)base;
-  const uint64_t sb = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
-                      ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32);
+// The same with a scalar base address (sbase64) and a 32-bit per-lane offset.
+__device__ __forceinline__ void dma16s(uint32_t off, uint64_t base, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :
-               : "v"(off), "s"(sb), "s"(lds_addr)
+               : "v"(off), "s"(base), "s"(lds_addr)
                : "memory", "m0");
+}
+// one dword per lane
+__device__ __forceinline__ void dma4s(uint32_t off, uint64_t base, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+               :
+               : "v"(off), "s"(base), "s"(lds_addr)
+               : "memory", "m0");
+}
+// a wave-uniform address in SGPRs
+__device__ __forceinline__ uint64_t sbase64(const void *p) {
+  const uint64_t b = (uint64_t)(uintptr_t)p;
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
+         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32);
 }
 
 template <int N>
@@ -127,10 +136,15 @@ __device__ __forceinline__ int bswz(int r) {
   return (((r >> 1) ^ (r >> 3)) & 1) | (((r >> 2) & 1) << 1);
 }
 
+// Four bf16 pairs 136 + q of k-slice j of a packed 16-byte chunk.  A nibble's
+// two's complement value q is (nibble ^ 8) - 8, and bf16 0x43NN is exactly
+// 128 + NN, so the shifted and masked nibble pair xor'ed with `magic` =
+// 0x43084308 (held in a register) is the pair 136 + q: one v_bitop3_b32 after
+// the shift.
 __device__ __forceinline__ u32x4 nib_slice3(u32x4 b, int j, uint32_t magic) {
   const uint32_t mask = 0x000F000Fu;
-  return u32x4{((b[0] >> (4 * j)) & mask) | magic, ((b[1] >> (4 * j)) & mask) | magic,
-               ((b[2] >> (4 * j)) & mask) | magic, ((b[3] >> (4 * j)) & mask) | magic};
+  return u32x4{((b[0] >> (4 * j)) & mask) ^ magic, ((b[1] >> (4 * j)) & mask) ^ magic,
+               ((b[2] >> (4 * j)) & mask) ^ magic, ((b[3] >> (4 * j)) & mask) ^ magic};
 }
 
 // silu(g) * u for the prefill epilogue: the hardware exp2 and reciprocal
@@ -163,14 +177,11 @@ __device__ __forceinline__ float row16_sum(float v) {
 }
 
 // One item: expert tile lb / n_nblk (its entry t), column block lb % n_nblk.
-template <int SD, int MODE, int WN, int STAGES_>
+template <int SD, int MODE, int WN>
 __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const int4 t) {
-  using Gm = Geo<WN, STAGES_>;
-  constexpr int BN = Gm::BN, STAGES = Gm::STAGES, A_STAGE = Gm::A_STAGE, STAGE = Gm::STAGE;
-  constexpr int NW = Gm::NW, THREADS = Gm::THREADS, COLS = Gm::COLS;
-  // dynamic LDS: STAGES x (A | B) ring, scales[TG][BN] fp16, xs[TG][BM] fp32
-  // (group-major: a lane's 4 rows are one 16-byte read); the epilogue's
-  // staging and row sums reuse the idle ring
+  using Gm = Geo<WN>;
+  constexpr int BN = Gm::BN, NW = Gm::NW, THREADS = Gm::THREADS, COLS = Gm::COLS;
+  // dynamic LDS: the ring; the epilogue's staging and row sums reuse it
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int n_nb = a.n_nblk;
   const int nb = lb % n_nb;
@@ -183,9 +194,6 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   if (nb * (MODE == 0 ? COLS : BN) >= N) return;
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
-  uint16_t *sc_lds = (uint16_t *)(lds + STAGES * STAGE);
-  float *xs_lds = (float *)(lds + STAGES * STAGE + BN * TG * 2);
-
   GTRACE(const unsigned long long t0 = __builtin_amdgcn_s_memtime());
   const int tid = tid_opaque();  // per item: nothing lane-dependent is hoisted across items
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -237,80 +245,67 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   // subtile i's rows, so the subtiles past the count are not copied
   const int nms = __builtin_amdgcn_readfirstlane(min(4, (mcnt + 15) >> 4));
   static_assert(Gm::A_DMA == 4 && NW == 4, "A slot i holds the rows of token subtile i");
-  // DMA of group g into its ring stage
-  auto issue = [&](int g) {
-    const uint32_t base = lds0 + (uint32_t)(g % STAGES) * STAGE;
-#pragma unroll
-    for (int i = 0; i < Gm::A_DMA; ++i)
-      if (i < nms) dma16s(aoff[i], abase + g * 256, base + (uint32_t)((i * NW + wave) * 1024));
-#pragma unroll
-    for (int i = 0; i < Gm::B_DMA; ++i)
-      dma16s(boff[i], bbase[i] + g * 64, base + A_STAGE + (uint32_t)((i * NW + wave) * 1024));
-  };
-  // ---- tables of groups [g0, g0 + TG): scales [group][B-row] and -136 x the
-  // group sums [group][token row] in LDS.  A thread reads one weight row's
-  // scales (contiguous: 8 bytes per load where G allows it) and four groups
-  // of one token row; all loads are issued before the first LDS store.
-  auto load_tables = [&](int g0) {
-    const int ng = min(TG, G - g0);
-    const int r = tid;  // B-row (BN == THREADS)
-    const uint16_t *sc;
+  // scales: wave w copies B rows [64 w, +64), lane l the aligned dword that
+  // holds row 64 w + l's scale of the group (the tensor's rows are a multiple
+  // of 128, so the dword never ends past it); group sums: lane l token row l
+  const uint16_t *sbase;
+  uint32_t soff, xoff;
+  const float *xbase;
+  {
+    const int r = wave * 64 + lane;
     int row;
     if (MODE == 0) {
-      sc = r < COLS ? (shared ? a.ss0 : a.s0 + (size_t)e * N * G)
-                    : (shared ? a.ss1 : a.s1 + (size_t)e * N * G);
+      sbase = wave * 64 < COLS ? (shared ? a.ss0 : a.s0 + (size_t)e * N * G)
+                               : (shared ? a.ss1 : a.s1 + (size_t)e * N * G);
       row = nb * COLS + (r % COLS);
     } else {
-      sc = shared ? a.ss0 : a.s0 + (size_t)e * N * G;
+      sbase = shared ? a.ss0 : a.s0 + (size_t)e * N * G;
       row = nb * BN + r;
     }
-    sc += (size_t)min(row, N - 1) * G + g0;
-    uint32_t sv[TG / 2];  // packed pairs
-    if ((G & 3) == 0) {
-#pragma unroll
-      for (int j = 0; j < TG / 4; ++j) {
-        const uint2 v = *(const uint2 *)(sc + min(4 * j, ng - 4));
-        sv[2 * j] = v.x;
-        sv[2 * j + 1] = v.y;
-      }
+    soff = (uint32_t)(min(row, N - 1) * G) * 2u;
+    const int rr = min(lane, mcnt - 1);
+    if (MODE == 0) {
+      xbase = a.xsum + (shared ? (size_t)pos0 * G : 0);
+      xoff = (uint32_t)((shared ? rr : a.ptok[pos0 + rr]) * G) * 4u;
     } else {
-#pragma unroll
-      for (int j = 0; j < TG / 2; ++j)
-        sv[j] = (uint32_t)sc[min(2 * j, ng - 1)] | ((uint32_t)sc[min(2 * j + 1, ng - 1)] << 16);
+      xbase = (shared ? a.asum_s : a.asum) + (size_t)pos0 * G;
+      xoff = (uint32_t)(rr * G) * 4u;
     }
-    // thread: token row tid / 4, groups g0 + 4 * (tid % 4) + [0, 4)
-    static_assert(BM * 4 == THREADS && TG == 16, "one thread per (token row, 4 groups)");
-    const int xr = tid >> 2, xg = 4 * (tid & 3);
-    const int rr = min(xr, mcnt - 1);
-    const float *xsrc = MODE == 0 ? a.xsum : (shared ? a.asum_s : a.asum);
-    const int xrow = MODE == 0 && !shared ? a.ptok[pos0 + rr] : pos0 + rr;
-    xsrc += (size_t)xrow * G + g0;
-    float xv[4];
-    if ((G & 3) == 0) {
-      const float4 v = *(const float4 *)(xsrc + min(xg, ng - 4));
-      xv[0] = v.x; xv[1] = v.y; xv[2] = v.z; xv[3] = v.w;
-    } else {
+  }
+  const uint64_t abase_s = sbase64(abase), sbase_s = sbase64(sbase), xbase_s = sbase64(xbase);
+  uint64_t bbase_s[Gm::B_DMA];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) xv[j] = xsrc[min(xg + j, ng - 1)];
-    }
+  for (int i = 0; i < Gm::B_DMA; ++i) bbase_s[i] = sbase64(bbase[i]);
+  // DMA of group g into the ring stage at `base`, NMS token subtiles
+  // (NMS + B_DMA + 2 instructions per wave)
+  auto issue = [&](auto nms_c, int g, uint32_t base) {
+    constexpr int NMS = decltype(nms_c)::value;
+    constexpr uint32_t BO = NMS * Gm::A_SUB, SO = BO + Gm::B_STAGE, XO = SO + BN * 4;
 #pragma unroll
-    for (int j = 0; j < TG / 2; ++j) {
-      if (2 * j < ng) sc_lds[2 * j * BN + r] = (uint16_t)sv[j];
-      if (2 * j + 1 < ng) sc_lds[(2 * j + 1) * BN + r] = (uint16_t)(sv[j] >> 16);
-    }
+    for (int i = 0; i < Gm::B_DMA; ++i)
+      dma16s(boff[i], bbase_s[i] + (uint32_t)g * 64u, base + BO + (uint32_t)((i * NW + wave) * 1024));
+    dma4s((soff + 2u * (uint32_t)g) & ~3u, sbase_s, base + SO + (uint32_t)(wave * 256));
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (xg + j < ng) xs_lds[(xg + j) * BM + xr] = xr < mcnt ? -136.0f * xv[j] : 0.0f;
+    for (int i = 0; i < NMS; ++i)
+      dma16s(aoff[i], abase_s + (uint32_t)g * 256u, base + (uint32_t)((i * NW + wave) * 1024));
+    // (every wave copies the same 64 sums: equal instruction counts)
+    dma4s(xoff, xbase_s + (uint32_t)g * 4u, base + XO);
   };
-  issue(0);
-  load_tables(0);
 
-  // B rows of this wave's 4 N-subtiles
-  int brow[4];
+  // B rows of this wave's 4 N-subtiles: m16 + brow(ns); the subtiles' LDS
+  // addresses differ by constants (bswz depends on the row's low 4 bits)
+  auto brow = [](int ns) {
+    return MODE == 0 ? (ns < 2 ? ns * 16 : COLS + (ns - 2) * 16) : ns * 16;
+  };
+  const int brow0 = (MODE == 0 ? wn * 32 : wn * 64) + m16;
+  const uint32_t soffl = (uint32_t)(brow0 * 4);
+  const uint32_t boffl = (uint32_t)(brow0 * 64 + ((q ^ bswz(m16)) << 4));
+  uint32_t aoffl[4];  // this lane's A chunk of k-slice j in a 16-row subtile
 #pragma unroll
-  for (int ns = 0; ns < 4; ++ns)
-    brow[ns] = MODE == 0 ? (ns < 2 ? wn * 32 + ns * 16 : COLS + wn * 32 + (ns - 2) * 16) + m16
-                         : wn * 64 + ns * 16 + m16;
+  for (int j = 0; j < 4; ++j) aoffl[j] = (uint32_t)(m16 * 256 + (((4 * q + j) ^ aswz(m16)) << 4));
+  // the half of a row's scale dword that holds group 0's scale (odd G: every
+  // other row; the same for the 4 subtiles, whose rows differ by even numbers)
+  uint32_t ssh = ((uint32_t)(brow0 * G) & 1u) * 16u;
 
   // The main loop, for NMS of this wave's 4 token subtiles (16 tokens each):
   // subtiles past the tile's token count cost no MFMA or A read.
@@ -321,8 +316,13 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     for (int ns = 0; ns < 4; ++ns) tot[ms][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
   auto main_loop = [&](auto nms_c) {
     constexpr int NMS = decltype(nms_c)::value;
+    constexpr int STAGE = Gm::stage(NMS), STAGES = Gm::stages(NMS);
+    constexpr uint32_t BO = NMS * Gm::A_SUB, SO = BO + Gm::B_STAGE, XO = SO + BN * 4;
+    constexpr int PER = NMS + Gm::B_DMA + 2;  // DMA instructions per wave and group
+    issue(nms_c, 0, lds0);
+    if (STAGES > 2 && G > 1) issue(nms_c, 1, lds0 + STAGE);
     uint32_t magic;
-    asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    asm volatile("v_mov_b32 %0, 0x43084308" : "=v"(magic));
     // acc and sprev start at zero, so the scale step of "group -1" adds
     // +0 * +0 to tot's +0 and leaves it unchanged (no branch in the loop)
     f32x4 acc[4][4];
@@ -333,9 +333,13 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     float sg[4], sprev[4] = {0.f, 0.f, 0.f, 0.f};
     // Group g, part 1: the scale step of group g-1 (VALU only) and the
     // scales of group g.
-    auto part_v = [&](int g) {
+    auto part_v = [&](const uint8_t *st) {
 #pragma unroll
-      for (int ns = 0; ns < 4; ++ns) sg[ns] = scale_to_f32<SD>(sc_lds[(g % TG) * BN + brow[ns]]);
+      for (int ns = 0; ns < 4; ++ns) {
+        const uint32_t v = *(const uint32_t *)(st + soffl + SO + brow(ns) * 4);
+        sg[ns] = scale_to_f32<SD>((uint16_t)(v >> ssh));
+      }
+      ssh ^= 16u;
 #pragma unroll
       for (int ns = 0; ns < 4; ++ns)
 #pragma unroll
@@ -343,28 +347,25 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     };
     // Group g, part 2: group sums and A fragments from LDS, B unpacked per
     // k-slice, and the 4 x NMS MFMAs of each of the 4 k-slices.
-    // this wave's raw B chunks of group g (sign bits flipped: 8 + q)
-    auto load_bx = [&](int g, u32x4 (&bx)[4]) {
-      const uint8_t *sb = lds + (g % STAGES) * STAGE + A_STAGE;
+    // this wave's raw B chunks of the stage
+    auto load_bx = [&](const uint8_t *st, u32x4 (&bx)[4]) {
 #pragma unroll
       for (int ns = 0; ns < 4; ++ns)
-        bx[ns] = *(const u32x4 *)(sb + brow[ns] * 64 + ((q ^ bswz(brow[ns])) << 4)) ^ 0x88888888u;
+        bx[ns] = *(const u32x4 *)(st + boffl + BO + brow(ns) * 64);
     };
-    auto part_m = [&](int g, const u32x4 (&bx)[4]) {
-      const uint8_t *sa = lds + (g % STAGES) * STAGE;
-      const uint8_t *arow = sa + m16 * 256;
+    auto part_m = [&](const uint8_t *st, const u32x4 (&bx)[4]) {
       // group sums (-136 sum_k a): the first k-slice accumulates onto them
       f32x4 c0[4];
 #pragma unroll
       for (int ms = 0; ms < NMS; ++ms)
-        c0[ms] = *(const f32x4 *)(xs_lds + (g % TG) * BM + ms * 16 + 4 * q);
+        c0[ms] = *(const f32x4 *)(st + XO + (ms * 16 + 4 * q) * 4);
       // A fragments one k-slice ahead; the scheduling barrier after each
       // slice keeps the compiler from hoisting all 16 reads (64 VGPRs) to
       // the top, which spills at this register budget
       u32x4 af[2][4];
 #pragma unroll
       for (int ms = 0; ms < NMS; ++ms)
-        af[0][ms] = *(const u32x4 *)(arow + ms * 16 * 256 + (((4 * q) ^ aswz(m16)) << 4));
+        af[0][ms] = *(const u32x4 *)(st + aoffl[0] + ms * 16 * 256);
       if constexpr (MODE == 0) {
         // k-slice j's MFMAs run column subtile by column subtile, and each
         // subtile's B operand for slice j+1 is unpacked right after its last
@@ -379,10 +380,9 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if (j < 3) {
-            const int chunk = ((4 * q + j + 1) ^ aswz(m16)) << 4;
 #pragma unroll
             for (int ms = 0; ms < NMS; ++ms)
-              af[(j + 1) & 1][ms] = *(const u32x4 *)(arow + ms * 16 * 256 + chunk);
+              af[(j + 1) & 1][ms] = *(const u32x4 *)(st + aoffl[j + 1] + ms * 16 * 256);
           }
 #pragma unroll
           for (int ns = 0; ns < 4; ++ns) {
@@ -410,10 +410,9 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           if (j < 3) {
-            const int chunk = ((4 * q + j + 1) ^ aswz(m16)) << 4;
 #pragma unroll
             for (int ms = 0; ms < NMS; ++ms)
-              af[(j + 1) & 1][ms] = *(const u32x4 *)(arow + ms * 16 * 256 + chunk);
+              af[(j + 1) & 1][ms] = *(const u32x4 *)(st + aoffl[j + 1] + ms * 16 * 256);
           }
           u32x4 bf[4];
 #pragma unroll
@@ -433,21 +432,24 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     u32x4 bx[4];
     // One barrier per group.  At the top of iteration g every wave has
     // issued all its MFMAs of group g-1 (they may still be executing) and
-    // has read its last fragment of stage g-1 and its table entries, so after
-    // the barrier the DMA of group g+1 may overwrite that stage and, every TG
-    // groups, the tables may be rewritten.
+    // has read its last fragment of stage g-1, so after the barrier a DMA may
+    // overwrite that stage: group g+1 (2 stages) or g+2 (3 stages).
+    int st = 0, sf = STAGES - 1;  // stages of group g and of the group to fill
     for (int g = 0; g < G; ++g) {
-      wait_vm<0>();  // this thread's DMA of group g (issued one group ago)
-      // stage g complete for every thread (and, at g = 0, the LDS tables)
-      block_barrier();
-      if (g + 1 < G) issue(g + 1);
-      if (g > 0 && g % TG == 0) {
-        load_tables(g);
-        block_barrier();
-      }
-      load_bx(g, bx);
-      part_v(g);
-      part_m(g, bx);
+      // this thread's DMA of group g has landed (at 3 stages group g+1's,
+      // issued after it, may be in flight)
+      if (STAGES > 2 && g + 1 < G)
+        wait_vm<PER>();
+      else
+        wait_vm<0>();
+      block_barrier();  // and every thread's
+      if (g + STAGES - 1 < G) issue(nms_c, g + STAGES - 1, lds0 + (uint32_t)(sf * STAGE));
+      const uint8_t *sp = lds + st * STAGE;
+      load_bx(sp, bx);
+      part_v(sp);
+      part_m(sp, bx);
+      st = st + 1 == STAGES ? 0 : st + 1;
+      sf = sf + 1 == STAGES ? 0 : sf + 1;
     }
 #pragma unroll
     for (int ns = 0; ns < 4; ++ns)
@@ -482,7 +484,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     constexpr int OST = COLS * 2 + 16;  // staged row stride, bytes
     // staged rows, then red_sum[WN][BM] fp32 (per row-wave row sums)
     float *red_sum = (float *)(lds + BM * OST);
-    static_assert(BM * OST + WN * BM * 4 <= STAGES * STAGE, "staging exceeds the ring");
+    static_assert(BM * OST + WN * BM * 4 <= Gm::RING, "staging exceeds the ring");
     float rowsum[4][4];
 #pragma unroll
     for (int ms = 0; ms < 4; ++ms)
@@ -551,11 +553,11 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
       float v = 0.0f;
 #pragma unroll
       for (int w = 0; w < WN; ++w) v += red_sum[w * BM + tid];
-      as[(size_t)(pos0 + tid) * (N / COLS) + nb] = v;
+      as[(size_t)(pos0 + tid) * (N / COLS) + nb] = -136.0f * v;
     }
   } else {
     constexpr int OST = BN * 2 + 16;
-    static_assert(BM * OST <= STAGES * STAGE, "staging exceeds the ring");
+    static_assert(BM * OST <= Gm::RING, "staging exceeds the ring");
     // Neighbouring columns live in lanes m16 and m16 ^ 1: the pair trades
     // halves so that each lane stores whole dwords (even lane: rows r = 0,
     // 1; odd lane: rows 2, 3).  With the 528-byte row stride the 32 lanes of
@@ -603,12 +605,12 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
 // whatever the host's tile bound), which keeps the column blocks of one
 // expert tile, and the tiles of one expert, on one XCD: they share A rows and
 // weights through that L2.
-template <int SD, int MODE, int WN, int STAGES_>
+template <int SD, int MODE, int WN>
 __global__ __launch_bounds__(64 * WN, 2) void k_expert_gemm(GemmArgs a) {
   const int n_items = *a.n_tiles * a.n_nblk;
   if ((int)blockIdx.x >= n_items) return;
   const int lb = xcd_remap(blockIdx.x, n_items);
-  gemm_item<SD, MODE, WN, STAGES_>(a, lb, a.tiles[lb / a.n_nblk]);
+  gemm_item<SD, MODE, WN>(a, lb, a.tiles[lb / a.n_nblk]);
   GTRACE(__syncthreads(); if (threadIdx.x == 0 && lb < 16384) g_gtrace[(MODE * 16384 + lb) * 4 + 3] =
              __builtin_amdgcn_s_memtime());
 }
@@ -749,24 +751,24 @@ __global__ __launch_bounds__(256) void k_router_gemm(const uint16_t *__restrict_
   }
 }
 
-template <int WN, int STAGES_>
+template <int WN>
 hipError_t launch_geo(int mode, int scale_dtype, GemmArgs a, int max_tiles, hipStream_t s) {
-  using Gm = Geo<WN, STAGES_>;
+  using Gm = Geo<WN>;
   const int Nmax = mode == 0 ? (a.I > a.Is ? a.I : a.Is) : a.H;
   a.n_nblk = mode == 0 ? (Nmax + Gm::COLS - 1) / Gm::COLS : (Nmax + Gm::BN - 1) / Gm::BN;
   const long grid = (long)max_tiles * a.n_nblk;
   if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
   // the group sums of act: MODE 0 writes one per COLS = 128 columns
   static_assert(Gm::COLS == 128, "one act sum per k-group");
-  constexpr size_t lds = (size_t)STAGES_ * Gm::STAGE + Gm::BN * TG * 2 + BM * TG * 4;
+  constexpr size_t lds = Gm::RING;
   static_assert(2 * lds <= 160 * 1024, "two blocks per CU");
   void (*kern)(GemmArgs);
   if (mode == 0)
-    kern = scale_dtype == AINFER_SCALE_FP16 ? k_expert_gemm<AINFER_SCALE_FP16, 0, WN, STAGES_>
-                                            : k_expert_gemm<AINFER_SCALE_BF16, 0, WN, STAGES_>;
+    kern = scale_dtype == AINFER_SCALE_FP16 ? k_expert_gemm<AINFER_SCALE_FP16, 0, WN>
+                                            : k_expert_gemm<AINFER_SCALE_BF16, 0, WN>;
   else
-    kern = scale_dtype == AINFER_SCALE_FP16 ? k_expert_gemm<AINFER_SCALE_FP16, 1, WN, STAGES_>
-                                            : k_expert_gemm<AINFER_SCALE_BF16, 1, WN, STAGES_>;
+    kern = scale_dtype == AINFER_SCALE_FP16 ? k_expert_gemm<AINFER_SCALE_FP16, 1, WN>
+                                            : k_expert_gemm<AINFER_SCALE_BF16, 1, WN>;
   kern<<<(unsigned)grid, Gm::THREADS, lds, s>>>(a);
   return hipGetLastError();
 }
@@ -793,7 +795,7 @@ hipError_t launch_router_gemm(const void *x, const void *rw, const float *bias, 
 hipError_t launch_expert_gemm(int mode, int scale_dtype, GemmArgs a, int max_tiles,
                               hipStream_t s) {
   if (max_tiles <= 0) return hipSuccess;
-  return launch_geo<GEMM_WN, 2>(mode, scale_dtype, a, max_tiles, s);
+  return launch_geo<GEMM_WN>(mode, scale_dtype, a, max_tiles, s);
 }
 
 // ---------------------------------------------------------------------------
