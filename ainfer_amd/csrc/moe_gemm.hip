@@ -55,6 +55,8 @@ extern "C" int ainfer_debug_gemm_trace(void *host) {
 
 namespace {
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
 constexpr int BM = GEMM_MT;  // tokens per tile: one token wave of 64
 
 // Block geometry: WN waves along the weight rows; BN = 64 * WN rows per block.
@@ -147,6 +149,16 @@ __device__ __forceinline__ u32x4 nib_slice3(u32x4 b, int j, uint32_t magic) {
                ((b[2] >> (4 * j)) & mask) ^ magic, ((b[3] >> (4 * j)) & mask) ^ magic};
 }
 
+// D (TM x TM) += A B: 16 x 16 over 32 k, or 32 x 32 over 16 k
+template <int TM, typename V>
+__device__ __forceinline__ V mfma_bf16(u32x4 a, u32x4 b, V c) {
+  if constexpr (TM == 16)
+    return mfma_bf16_16x16x32(a, b, c);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
 // silu(g) * u for the prefill epilogue: the hardware exp2 and reciprocal
 // (about 1 ulp each) instead of expf and an IEEE division, which made the
 // epilogue several times longer than a group of the main loop.  The result is
@@ -199,7 +211,6 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int wn = wave;
-  const int m16 = lane & 15, q = lane >> 4;
 
   // ---- per-thread DMA sources: A_DMA A slots and B_DMA B slots per stage ---
   // slot s = (i*NW + wave)*64 + lane, 16 bytes each.  The block-uniform part
@@ -277,7 +288,8 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
 #pragma unroll
   for (int i = 0; i < Gm::B_DMA; ++i) bbase_s[i] = sbase64(bbase[i]);
   // DMA of group g into the ring stage at `base`, NMS token subtiles
-  // (NMS + B_DMA + 2 instructions per wave)
+  // (NMS + B_DMA + 2 instructions per wave; at NMS = 4 one fewer for a tile
+  // of three subtiles)
   auto issue = [&](auto nms_c, int g, uint32_t base) {
     constexpr int NMS = decltype(nms_c)::value;
     constexpr uint32_t BO = NMS * Gm::A_SUB, SO = BO + Gm::B_STAGE, XO = SO + BN * 4;
@@ -287,154 +299,72 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     dma4s((soff + 2u * (uint32_t)g) & ~3u, sbase_s, base + SO + (uint32_t)(wave * 256));
 #pragma unroll
     for (int i = 0; i < NMS; ++i)
-      dma16s(aoff[i], abase_s + (uint32_t)g * 256u, base + (uint32_t)((i * NW + wave) * 1024));
+      if (NMS < 4 || i < nms) dma16s(aoff[i], abase_s + (uint32_t)g * 256u, base + (uint32_t)((i * NW + wave) * 1024));
     // (every wave copies the same 64 sums: equal instruction counts)
     dma4s(xoff, xbase_s + (uint32_t)g * 4u, base + XO);
   };
 
-  // B rows of this wave's 4 N-subtiles: m16 + brow(ns); the subtiles' LDS
-  // addresses differ by constants (bswz depends on the row's low 4 bits)
-  auto brow = [](int ns) {
-    return MODE == 0 ? (ns < 2 ? ns * 16 : COLS + (ns - 2) * 16) : ns * 16;
-  };
-  const int brow0 = (MODE == 0 ? wn * 32 : wn * 64) + m16;
-  const uint32_t soffl = (uint32_t)(brow0 * 4);
-  const uint32_t boffl = (uint32_t)(brow0 * 64 + ((q ^ bswz(m16)) << 4));
-  uint32_t aoffl[4];  // this lane's A chunk of k-slice j in a 16-row subtile
+  // The main loop and epilogue on token tiles of TM: MS tiles of TM tokens
+  // x NS tiles of TM weight rows per wave (TM * NS = 64), NSUB = MS * TM / 16
+  // subtiles in the ring.
+  auto run = [&](auto tm_c, auto ms_c) {
+    constexpr int TM = decltype(tm_c)::value, MS = decltype(ms_c)::value;
+    constexpr int NS = 64 / TM, NSUB = MS * TM / 16, NSL = TM / 4;  // k-slices per group
+    constexpr int NP = TM / 16;  // 32-k blocks of a row per lane
+    constexpr int NQ = TM == 16 ? 1 : 4;  // row quads a lane holds of a tile
+    using acc_t = typename std::conditional<TM == 16, f32x4, f32x16>::type;
+    using nsub_t = std::integral_constant<int, NSUB>;
+    constexpr int STAGE = Gm::stage(NSUB), STAGES = Gm::stages(NSUB);
+    constexpr uint32_t BO = NSUB * Gm::A_SUB, SO = BO + Gm::B_STAGE, XO = SO + BN * 4;
+    constexpr int PER = NSUB + Gm::B_DMA + 2;  // DMA instructions per wave and group
+    issue(nsub_t(), 0, lds0);
+    if (STAGES > 2 && G > 1) issue(nsub_t(), 1, lds0 + STAGE);
+    // lane (Q, rl): row rl of a tile, 32-k blocks NP * Q'.. of the group: slice
+    // s of TM = 16 is nibble pair s of block Q; slice s = 4 p + j of TM = 32
+    // is nibble pair j of block 2 p + Q
+    const int rl = lane & (TM - 1), Q = lane / TM;
+    auto blk = [&](int p) { return TM == 16 ? Q : 2 * p + Q; };
+    // B-rows of the wave's NS row tiles: brow0 + brow(ns); the tiles' LDS
+    // addresses differ by constants (bswz depends on the row's low 4 bits)
+    auto brow = [](int ns) {
+      return MODE == 0 ? (ns < NS / 2 ? ns * TM : COLS + (ns - NS / 2) * TM) : ns * TM;
+    };
+    const int brow0 = (MODE == 0 ? wn * 32 : wn * 64) + rl;
+    const uint32_t soffl = (uint32_t)(brow0 * 4);
+    uint32_t boffl[NP], aoffl[NSL];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) aoffl[j] = (uint32_t)(m16 * 256 + (((4 * q + j) ^ aswz(m16)) << 4));
-  // the half of a row's scale dword that holds group 0's scale (odd G: every
-  // other row; the same for the 4 subtiles, whose rows differ by even numbers)
-  uint32_t ssh = ((uint32_t)(brow0 * G) & 1u) * 16u;
-
-  // The main loop, for NMS of this wave's 4 token subtiles (16 tokens each):
-  // subtiles past the tile's token count cost no MFMA or A read.
-  f32x4 tot[4][4];
+    for (int p = 0; p < NP; ++p) boffl[p] = (uint32_t)(brow0 * 64 + ((blk(p) ^ bswz(rl)) << 4));
 #pragma unroll
-  for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-    for (int ns = 0; ns < 4; ++ns) tot[ms][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto main_loop = [&](auto nms_c) {
-    constexpr int NMS = decltype(nms_c)::value;
-    constexpr int STAGE = Gm::stage(NMS), STAGES = Gm::stages(NMS);
-    constexpr uint32_t BO = NMS * Gm::A_SUB, SO = BO + Gm::B_STAGE, XO = SO + BN * 4;
-    constexpr int PER = NMS + Gm::B_DMA + 2;  // DMA instructions per wave and group
-    issue(nms_c, 0, lds0);
-    if (STAGES > 2 && G > 1) issue(nms_c, 1, lds0 + STAGE);
+    for (int s = 0; s < NSL; ++s)
+      aoffl[s] = (uint32_t)(rl * 256 + (((4 * blk(s >> 2) + (s & 3)) ^ aswz(rl)) << 4));
+    // the half of a row's scale dword that holds group 0's scale (odd G: every
+    // other row; the same for all row tiles, whose rows differ by even numbers)
+    uint32_t ssh = ((uint32_t)(brow0 * G) & 1u) * 16u;
     uint32_t magic;
     asm volatile("v_mov_b32 %0, 0x43084308" : "=v"(magic));
     // acc and sprev start at zero, so the scale step of "group -1" adds
     // +0 * +0 to tot's +0 and leaves it unchanged (no branch in the loop)
-    f32x4 acc[4][4];
+    acc_t tot[MS][NS], acc[MS][NS];
+    float sg[NS], sprev[NS];
 #pragma unroll
-    for (int ms = 0; ms < 4; ++ms)
+    for (int ns = 0; ns < NS; ++ns) {
+      sprev[ns] = 0.f;
 #pragma unroll
-      for (int ns = 0; ns < 4; ++ns) acc[ms][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float sg[4], sprev[4] = {0.f, 0.f, 0.f, 0.f};
-    // Group g, part 1: the scale step of group g-1 (VALU only) and the
-    // scales of group g.
-    auto part_v = [&](const uint8_t *st) {
+      for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-      for (int ns = 0; ns < 4; ++ns) {
-        const uint32_t v = *(const uint32_t *)(st + soffl + SO + brow(ns) * 4);
-        sg[ns] = scale_to_f32<SD>((uint16_t)(v >> ssh));
-      }
-      ssh ^= 16u;
+        for (int i = 0; i < 4 * NQ; ++i) tot[ms][ns][i] = acc[ms][ns][i] = 0.f;
+    }
+    auto scale_step = [&]() {
 #pragma unroll
-      for (int ns = 0; ns < 4; ++ns)
+      for (int ns = 0; ns < NS; ++ns)
 #pragma unroll
-        for (int ms = 0; ms < NMS; ++ms) tot[ms][ns] += sprev[ns] * acc[ms][ns];
+        for (int ms = 0; ms < MS; ++ms) tot[ms][ns] += sprev[ns] * acc[ms][ns];
     };
-    // Group g, part 2: group sums and A fragments from LDS, B unpacked per
-    // k-slice, and the 4 x NMS MFMAs of each of the 4 k-slices.
-    // this wave's raw B chunks of the stage
-    auto load_bx = [&](const uint8_t *st, u32x4 (&bx)[4]) {
-#pragma unroll
-      for (int ns = 0; ns < 4; ++ns)
-        bx[ns] = *(const u32x4 *)(st + boffl + BO + brow(ns) * 64);
-    };
-    auto part_m = [&](const uint8_t *st, const u32x4 (&bx)[4]) {
-      // group sums (-136 sum_k a): the first k-slice accumulates onto them
-      f32x4 c0[4];
-#pragma unroll
-      for (int ms = 0; ms < NMS; ++ms)
-        c0[ms] = *(const f32x4 *)(st + XO + (ms * 16 + 4 * q) * 4);
-      // A fragments one k-slice ahead; the scheduling barrier after each
-      // slice keeps the compiler from hoisting all 16 reads (64 VGPRs) to
-      // the top, which spills at this register budget
-      u32x4 af[2][4];
-#pragma unroll
-      for (int ms = 0; ms < NMS; ++ms)
-        af[0][ms] = *(const u32x4 *)(st + aoffl[0] + ms * 16 * 256);
-      if constexpr (MODE == 0) {
-        // k-slice j's MFMAs run column subtile by column subtile, and each
-        // subtile's B operand for slice j+1 is unpacked right after its last
-        // use, so the unpacking issues between MFMAs instead of as a block
-        // before them; slices 1-3 are pinned to one MFMA, 32 / (4 NMS) VALU
-        // and (first NMS) one LDS read per step.  Gate/up 1% faster (c2).
-        // The down kernel keeps the form below: with this one its K = 512
-        // items spill registers.
-        u32x4 bf[4];
-#pragma unroll
-        for (int ns = 0; ns < 4; ++ns) bf[ns] = nib_slice3(bx[ns], 0, magic);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j < 3) {
-#pragma unroll
-            for (int ms = 0; ms < NMS; ++ms)
-              af[(j + 1) & 1][ms] = *(const u32x4 *)(st + aoffl[j + 1] + ms * 16 * 256);
-          }
-#pragma unroll
-          for (int ns = 0; ns < 4; ++ns) {
-#pragma unroll
-            for (int ms = 0; ms < NMS; ++ms)
-              acc[ms][ns] = mfma_bf16_16x16x32(af[j & 1][ms], bf[ns], j == 0 ? c0[ms] : acc[ms][ns]);
-            if (j < 3) bf[ns] = nib_slice3(bx[ns], j + 1, magic);
-          }
-          // slice 0 also holds the scale step's 16 NMS fmas: left to the
-          // compiler (a fixed pattern there spills)
-          if (NMS > 0 && j > 0) {
-#pragma unroll
-            for (int i = 0; i < 4 * NMS; ++i) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-              if (j < 3)
-                __builtin_amdgcn_sched_group_barrier(0x002, 32 / (4 * (NMS > 0 ? NMS : 1)), 0);  // VALU
-              else
-                __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
-              if (i < NMS && j < 3) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j < 3) {
-#pragma unroll
-            for (int ms = 0; ms < NMS; ++ms)
-              af[(j + 1) & 1][ms] = *(const u32x4 *)(st + aoffl[j + 1] + ms * 16 * 256);
-          }
-          u32x4 bf[4];
-#pragma unroll
-          for (int ns = 0; ns < 4; ++ns) bf[ns] = nib_slice3(bx[ns], j, magic);
-#pragma unroll
-          for (int ms = 0; ms < NMS; ++ms)
-#pragma unroll
-            for (int ns = 0; ns < 4; ++ns)
-              acc[ms][ns] = mfma_bf16_16x16x32(af[j & 1][ms], bf[ns], j == 0 ? c0[ms] : acc[ms][ns]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-#pragma unroll
-      for (int ns = 0; ns < 4; ++ns) sprev[ns] = sg[ns];
-    };
-
-    u32x4 bx[4];
     // One barrier per group.  At the top of iteration g every wave has
     // issued all its MFMAs of group g-1 (they may still be executing) and
     // has read its last fragment of stage g-1, so after the barrier a DMA may
     // overwrite that stage: group g+1 (2 stages) or g+2 (3 stages).
-    int st = 0, sf = STAGES - 1;  // stages of group g and of the group to fill
+    int si = 0, sf = STAGES - 1;  // stages of group g and of the group to fill
     for (int g = 0; g < G; ++g) {
       // this thread's DMA of group g has landed (at 3 stages group g+1's,
       // issued after it, may be in flight)
@@ -443,161 +373,198 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
       else
         wait_vm<0>();
       block_barrier();  // and every thread's
-      if (g + STAGES - 1 < G) issue(nms_c, g + STAGES - 1, lds0 + (uint32_t)(sf * STAGE));
-      const uint8_t *sp = lds + st * STAGE;
-      load_bx(sp, bx);
-      part_v(sp);
-      part_m(sp, bx);
-      st = st + 1 == STAGES ? 0 : st + 1;
+      if (g + STAGES - 1 < G) issue(nsub_t(), g + STAGES - 1, lds0 + (uint32_t)(sf * STAGE));
+      const uint8_t *st = lds + si * STAGE;
+      // this wave's raw B chunks and scales, and the scale step of group g-1
+      u32x4 bx[NS][NP];
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int ns = 0; ns < NS; ++ns)
+          bx[ns][p] = *(const u32x4 *)(st + boffl[p] + BO + brow(ns) * 64);
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns)
+        sg[ns] = scale_to_f32<SD>((uint16_t)(*(const uint32_t *)(st + soffl + SO + brow(ns) * 4) >> ssh));
+      ssh ^= 16u;
+      scale_step();
+      // group sums (-136 sum_k a): the first k-slice accumulates onto them
+      acc_t c0[MS];
+#pragma unroll
+      for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) {
+          const f32x4 v = *(const f32x4 *)(st + XO + (ms * TM + 8 * i + 4 * Q) * 4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) c0[ms][4 * i + r] = v[r];
+        }
+      // A fragments one k-slice ahead, and each row tile's B operand of slice
+      // s+1 unpacked right after its last use in slice s, so the unpacking
+      // issues between MFMAs; the scheduling barrier after each slice keeps
+      // the compiler from hoisting all reads to the top (spills)
+      u32x4 af[2][MS], bf[NS];
+#pragma unroll
+      for (int ms = 0; ms < MS; ++ms) af[0][ms] = *(const u32x4 *)(st + aoffl[0] + ms * TM * 256);
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns) bf[ns] = nib_slice3(bx[ns][0], 0, magic);
+#pragma unroll
+      for (int s = 0; s < NSL; ++s) {
+        if (s + 1 < NSL) {
+#pragma unroll
+          for (int ms = 0; ms < MS; ++ms)
+            af[(s + 1) & 1][ms] = *(const u32x4 *)(st + aoffl[(s + 1) % NSL] + ms * TM * 256);
+        }
+#pragma unroll
+        for (int ns = 0; ns < NS; ++ns) {
+#pragma unroll
+          for (int ms = 0; ms < MS; ++ms)
+            acc[ms][ns] = mfma_bf16<TM>(af[s & 1][ms], bf[ns], s == 0 ? c0[ms] : acc[ms][ns]);
+          if (s + 1 < NSL) bf[ns] = nib_slice3(bx[ns][((s + 1) / 4) % NP], (s + 1) & 3, magic);
+        }
+        // slice 0 also holds the scale step's fmas: left to the compiler
+        if (s > 0) {
+#pragma unroll
+          for (int i = 0; i < NS * MS; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            if (s + 1 < NSL) {
+              __builtin_amdgcn_sched_group_barrier(0x002, 8 / MS, 0);  // VALU
+              if (i < MS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+            } else {
+              __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns) sprev[ns] = sg[ns];
+      si = si + 1 == STAGES ? 0 : si + 1;
       sf = sf + 1 == STAGES ? 0 : sf + 1;
     }
-#pragma unroll
-    for (int ns = 0; ns < 4; ++ns)
-#pragma unroll
-      for (int ms = 0; ms < NMS; ++ms) tot[ms][ns] += sprev[ns] * acc[ms][ns];
-  };
-  // token subtiles of this wave holding tokens of the tile (wave-uniform)
-  GTRACE(const unsigned long long t1 = __builtin_amdgcn_s_memtime());
-  if (nms > 3)
-    main_loop(std::integral_constant<int, 4>());
-  else if (nms > 2)
-    main_loop(std::integral_constant<int, 3>());
-  else if (nms > 1)
-    main_loop(std::integral_constant<int, 2>());
-  else
-    main_loop(std::integral_constant<int, 1>());
-  wait_vm<0>();  // no DMA into the ring remains in flight
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  block_barrier();  // every wave's last read of the ring precedes the staging below
-  GTRACE(if (tid == 0 && lb < 16384) {
-    const int o = (MODE * 16384 + lb) * 4;
-    g_gtrace[o] = t0;
-    g_gtrace[o + 1] = t1;
-    g_gtrace[o + 2] = __builtin_amdgcn_s_memtime();
-  });
+    scale_step();
+    wait_vm<0>();  // no DMA into the ring remains in flight
+    block_barrier();  // every wave's last read of the ring precedes the staging below
+    GTRACE(if (tid == 0 && lb < 16384) {
+      const int o = (MODE * 16384 + lb) * 4;
+      g_gtrace[o] = t0;
+      g_gtrace[o + 1] = t1;
+      g_gtrace[o + 2] = __builtin_amdgcn_s_memtime();
+    });
 
-  // ---- epilogue -------------------------------------------------------
-  // lane (q, m16) of tile (ms, ns) holds rows ms*16 + 4q + r, column
-  // m16.  Results are staged in the (now idle) LDS ring and leave as 16-byte
-  // row chunks.
-  if (MODE == 0) {
-    constexpr int OST = COLS * 2 + 16;  // staged row stride, bytes
-    // staged rows, then red_sum[WN][BM] fp32 (per row-wave row sums)
-    float *red_sum = (float *)(lds + BM * OST);
-    static_assert(BM * OST + WN * BM * 4 <= Gm::RING, "staging exceeds the ring");
-    float rowsum[4][4];
+    // ---- epilogue -------------------------------------------------------
+    // A lane holds quad i (4 consecutive tokens) of tile (ms, ns): rows
+    // ms * TM + 8 i + 4 Q + [0, 4), column ns * TM + rl.  Results are staged
+    // in the (now idle) LDS ring and leave as 16-byte row chunks.  The lanes
+    // of a column pair trade halves so that each stores whole dwords (the
+    // lower lane tokens 0 and 1 of the quad, the upper 2 and 3): 2-byte LDS
+    // stores cost several times a dword store.  Branch-free: the selects are
+    // plain values and v_perm_b32 takes a per-lane selector.
+    if constexpr (MODE == 0) {
+      constexpr int OST = COLS * 2 + 16;  // staged row stride, bytes
+      static_assert(BM * OST <= Gm::RING, "staging exceeds the ring");
+      // columns k and k + 4 of a 32-column block are neighbours in MFMA order
+      // (perm32_pos), and live in lanes rl and rl ^ 4
+      const bool hi4 = (rl & 4) != 0;
+      const uint32_t sel0 = pair_sel(hi4, 0), sel1 = pair_sel(hi4, 1);
 #pragma unroll
-    for (int ms = 0; ms < 4; ++ms)
+      for (int ns = 0; ns < NS / 2; ++ns) {
+        // within a 32-aligned block of columns, MFMA order is block-local
+        const int p = perm32_pos(wn * 32 + ns * TM + (rl & ~4));  // the pair's even position
 #pragma unroll
-      for (int r = 0; r < 4; ++r) rowsum[ms][r] = 0.0f;
-    // Columns k and k + 4 of a 32-column block are neighbours in MFMA order
-    // (perm32_pos), and live in lanes m16 and m16 ^ 4: the pair trades
-    // halves so that each lane stores whole dwords (lane bit 2 clear: rows
-    // r = 0, 1; set: rows 2, 3).  2-byte LDS stores cost several times a
-    // dword store.
-    // Branch-free: the selects below are plain values and v_perm_b32 takes
-    // a per-lane selector (ternaries over expressions became divergent
-    // branches around every store).
-    const bool hi4 = (m16 & 4) != 0;
-    const uint32_t sel0 = pair_sel(hi4, 0), sel1 = pair_sel(hi4, 1);
+        for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      // within a 32-aligned block of columns, MFMA order is block-local
-      const int p = perm32_pos(wn * 32 + h * 16 + (m16 & ~4));  // the pair's even position
+          for (int i = 0; i < NQ; ++i) {
+            float f[4];
 #pragma unroll
-      for (int ms = 0; ms < 4; ++ms) {
-        float f[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) f[r] = silu_mul_fast(tot[ms][h][r], tot[ms][h + 2][r]);
-        const uint32_t p01 = bf16x2_bits(f[0], f[1]), p23 = bf16x2_bits(f[2], f[3]);
-        rowsum[ms][0] += __uint_as_float(p01 << 16);
-        rowsum[ms][1] += __uint_as_float(p01 & 0xFFFF0000u);
-        rowsum[ms][2] += __uint_as_float(p23 << 16);
-        rowsum[ms][3] += __uint_as_float(p23 & 0xFFFF0000u);
-        const uint32_t send = hi4 ? p01 : p23, own = hi4 ? p23 : p01;
-        // lane ^ 4 inside each group of 32 lanes (ds_swizzle bit mode)
-        const uint32_t recv = (uint32_t)__builtin_amdgcn_ds_swizzle((int)send, 0x101F);
-        const int row0 = ms * 16 + 4 * q + (hi4 ? 2 : 0);
-        *(uint32_t *)(lds + row0 * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel0);
-        *(uint32_t *)(lds + (row0 + 1) * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel1);
+            for (int r = 0; r < 4; ++r)
+              f[r] = silu_mul_fast(tot[ms][ns][4 * i + r], tot[ms][ns + NS / 2][4 * i + r]);
+            const uint32_t p01 = bf16x2_bits(f[0], f[1]), p23 = bf16x2_bits(f[2], f[3]);
+            const uint32_t send = hi4 ? p01 : p23, own = hi4 ? p23 : p01;
+            // lane ^ 4 inside each group of 32 lanes (ds_swizzle bit mode)
+            const uint32_t recv = (uint32_t)__builtin_amdgcn_ds_swizzle((int)send, 0x101F);
+            const int row0 = ms * TM + 8 * i + 4 * Q + (hi4 ? 2 : 0);
+            *(uint32_t *)(lds + row0 * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel0);
+            *(uint32_t *)(lds + (row0 + 1) * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel1);
+          }
       }
-    }
-    // per-row sum over this wave's 32 columns: reduce over the 16 lanes m16
-#pragma unroll
-    for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) rowsum[ms][r] = row16_sum(rowsum[ms][r]);
-    if (m16 == 0)
-#pragma unroll
-      for (int ms = 0; ms < 4; ++ms)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) red_sum[wn * BM + ms * 16 + 4 * q + r] = rowsum[ms][r];
-    __syncthreads();
-    uint16_t *dst = shared ? a.act_s : a.act;
-    constexpr int CPR = COLS / 8;  // 16-byte chunks per row
-    constexpr int NST = BM * CPR / THREADS;
-    u32x4 out[NST];  // every LDS read before the (predicated) stores
-#pragma unroll
-    for (int i = 0; i < NST; ++i) {
-      const int idx = tid + i * THREADS;
-      out[i] = *(const u32x4 *)(lds + (idx / CPR) * OST + (idx % CPR) * 16);
-    }
-#pragma unroll
-    for (int i = 0; i < NST; ++i) {
-      const int idx = tid + i * THREADS, row = idx / CPR, c = idx % CPR;
-      if (row < mcnt) *(u32x4 *)(dst + (size_t)(pos0 + row) * N + nb * COLS + c * 8) = out[i];
-    }
-    if (tid < BM && tid < mcnt) {
+      __syncthreads();
+      uint16_t *dst = shared ? a.act_s : a.act;
       float *as = shared ? a.asum_s : a.asum;
-      // one partial per COLS act columns (slot nb), row waves summed in order
-      float v = 0.0f;
+      constexpr int CPR = COLS / 8;  // 16-byte chunks per row
+      static_assert(CPR == 16, "a DPP row of lanes holds one act row");
+      constexpr int NST = NSUB * 16 * CPR / THREADS;
+      u32x4 out[NST];  // every LDS read before the (predicated) stores
 #pragma unroll
-      for (int w = 0; w < WN; ++w) v += red_sum[w * BM + tid];
-      as[(size_t)(pos0 + tid) * (N / COLS) + nb] = -136.0f * v;
-    }
-  } else {
-    constexpr int OST = BN * 2 + 16;
-    static_assert(BM * OST <= Gm::RING, "staging exceeds the ring");
-    // Neighbouring columns live in lanes m16 and m16 ^ 1: the pair trades
-    // halves so that each lane stores whole dwords (even lane: rows r = 0,
-    // 1; odd lane: rows 2, 3).  With the 528-byte row stride the 32 lanes of
-    // one store hit 32 distinct banks.
-    const bool odd = (m16 & 1) != 0;
-    const uint32_t sel0 = pair_sel(odd, 0), sel1 = pair_sel(odd, 1);
+      for (int i = 0; i < NST; ++i) {
+        const int idx = tid + i * THREADS;
+        out[i] = *(const u32x4 *)(lds + (idx / CPR) * OST + (idx % CPR) * 16);
+      }
 #pragma unroll
-    for (int ns = 0; ns < 4; ++ns) {
-      const int cl = wn * 64 + 16 * ns + (m16 & ~1);
+      for (int i = 0; i < NST; ++i) {
+        const int idx = tid + i * THREADS, row = idx / CPR, c = idx % CPR;
+        if (row < mcnt) *(u32x4 *)(dst + (size_t)(pos0 + row) * N + nb * COLS + c * 8) = out[i];
+        // the row's sum over this block's 128 columns (one k-group of down)
+        float v = 0.f;
 #pragma unroll
-      for (int ms = 0; ms < 4; ++ms) {
-        const uint32_t p01 = bf16x2_bits(tot[ms][ns][0], tot[ms][ns][1]);
-        const uint32_t p23 = bf16x2_bits(tot[ms][ns][2], tot[ms][ns][3]);
-        const uint32_t send = odd ? p01 : p23, own = odd ? p23 : p01;
-        const uint32_t recv =
-            (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xF, 0xF, false);  // lane ^ 1
-        const int row0 = ms * 16 + 4 * q + (odd ? 2 : 0);
-        *(uint32_t *)(lds + row0 * OST + cl * 2) = __builtin_amdgcn_perm(recv, own, sel0);
-        *(uint32_t *)(lds + (row0 + 1) * OST + cl * 2) = __builtin_amdgcn_perm(recv, own, sel1);
+        for (int d = 0; d < 4; ++d)
+          v += __uint_as_float(out[i][d] << 16) + __uint_as_float(out[i][d] & 0xFFFF0000u);
+        v = row16_sum(v);
+        if (c == 0 && row < mcnt) as[(size_t)(pos0 + row) * (N / COLS) + nb] = -136.0f * v;
+      }
+    } else {
+      constexpr int OST = BN * 2 + 16;
+      static_assert(BM * OST <= Gm::RING, "staging exceeds the ring");
+      // neighbouring columns live in lanes rl and rl ^ 1
+      const bool odd = (rl & 1) != 0;
+      const uint32_t sel0 = pair_sel(odd, 0), sel1 = pair_sel(odd, 1);
+#pragma unroll
+      for (int ns = 0; ns < NS; ++ns) {
+        const int cl = wn * 64 + TM * ns + (rl & ~1);
+#pragma unroll
+        for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+          for (int i = 0; i < NQ; ++i) {
+            const acc_t &v = tot[ms][ns];
+            const uint32_t p01 = bf16x2_bits(v[4 * i], v[4 * i + 1]);
+            const uint32_t p23 = bf16x2_bits(v[4 * i + 2], v[4 * i + 3]);
+            const uint32_t send = odd ? p01 : p23, own = odd ? p23 : p01;
+            const uint32_t recv =
+                (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+            const int row0 = ms * TM + 8 * i + 4 * Q + (odd ? 2 : 0);
+            *(uint32_t *)(lds + row0 * OST + cl * 2) = __builtin_amdgcn_perm(recv, own, sel0);
+            *(uint32_t *)(lds + (row0 + 1) * OST + cl * 2) = __builtin_amdgcn_perm(recv, own, sel1);
+          }
+      }
+      __syncthreads();
+      constexpr int CPR = BN / 8;
+      constexpr int NST = NSUB * 16 * CPR / THREADS;
+      u32x4 out[NST];  // every LDS read before the (predicated) stores
+#pragma unroll
+      for (int i = 0; i < NST; ++i) {
+        const int idx = tid + i * THREADS;
+        out[i] = *(const u32x4 *)(lds + (idx / CPR) * OST + (idx % CPR) * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < NST; ++i) {
+        const int idx = tid + i * THREADS, row = idx / CPR, c = idx % CPR;
+        const int col = nb * BN + c * 8;
+        if (row < mcnt && col < N) {
+          const size_t orow = shared ? (size_t)a.T * a.k + pos0 + row : (size_t)(pos0 + row);
+          *(u32x4 *)(a.o + orow * a.H + col) = out[i];
+        }
       }
     }
-    __syncthreads();
-    constexpr int CPR = BN / 8;
-    constexpr int NST = BM * CPR / THREADS;
-    u32x4 out[NST];  // every LDS read before the (predicated) stores
-#pragma unroll
-    for (int i = 0; i < NST; ++i) {
-      const int idx = tid + i * THREADS;
-      out[i] = *(const u32x4 *)(lds + (idx / CPR) * OST + (idx % CPR) * 16);
-    }
-#pragma unroll
-    for (int i = 0; i < NST; ++i) {
-      const int idx = tid + i * THREADS, row = idx / CPR, c = idx % CPR;
-      const int col = nb * BN + c * 8;
-      if (row < mcnt && col < N) {
-        const size_t orow = shared ? (size_t)a.T * a.k + pos0 + row : (size_t)(pos0 + row);
-        *(u32x4 *)(a.o + orow * a.H + col) = out[i];
-      }
-    }
-  }
+  };
+  GTRACE(const unsigned long long t1 = __builtin_amdgcn_s_memtime());
+  // 33 to 64 tokens: 2 x 2 tiles of 32 (a third subtile's missing partner
+  // costs MFMAs but no copy; its rows are never stored); 17 to 32: 1 x 2; up
+  // to 16: the 16-wide tiles
+  using std::integral_constant;
+  if (nms > 2)
+    run(integral_constant<int, 32>(), integral_constant<int, 2>());
+  else if (nms > 1)
+    run(integral_constant<int, 32>(), integral_constant<int, 1>());
+  else
+    run(integral_constant<int, 16>(), integral_constant<int, 1>());
 }
 
 // One block per item.  The items a launch's blocks take are XCD-contiguous
