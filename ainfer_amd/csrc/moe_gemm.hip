@@ -308,6 +308,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
   // x NS tiles of TM weight rows per wave (TM * NS = 64), NSUB = MS * TM / 16
   // subtiles in the ring.
   auto run = [&](auto tm_c, auto ms_c) {
+    GTRACE(const unsigned long long t1 = __builtin_amdgcn_s_memtime());
     constexpr int TM = decltype(tm_c)::value, MS = decltype(ms_c)::value;
     constexpr int NS = 64 / TM, NSUB = MS * TM / 16, NSL = TM / 4;  // k-slices per group
     constexpr int NP = TM / 16;  // 32-k blocks of a row per lane
@@ -554,7 +555,6 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
       }
     }
   };
-  GTRACE(const unsigned long long t1 = __builtin_amdgcn_s_memtime());
   // 33 to 64 tokens: 2 x 2 tiles of 32 (a third subtile's missing partner
   // costs MFMAs but no copy; its rows are never stored); 17 to 32: 1 x 2; up
   // to 16: the 16-wide tiles
