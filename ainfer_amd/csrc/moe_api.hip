@@ -377,8 +377,8 @@ int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, cons
 }
 
 // The expert stage on the dispatch d in the workspace, x in MFMA order
-// written (and its group sums at T >= GEMM_MIN_T): the grouped GEMM there,
-// else the streaming items over tiles of DEC_MT tokens.  Leaves o in the workspace: dispatch-position rows,
+// written (and its group sums where gemm): the grouped GEMM, else the
+// streaming items over tiles of DEC_MT tokens.  Leaves o in the workspace: dispatch-position rows,
 // the shared expert's at rows T * k + t.
 int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const Layout &L,
                 void *ws, DispatchOut &d, int T, bool gemm, hipStream_t st, ProfCall *pc) {
@@ -496,9 +496,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
   const int E = s->n_experts, k = s->top_k, H = s->hidden;
   const int has_shared = s->shared_inter > 0;
   const bool fused = T <= FUSED_DISPATCH_MAX_T;
-  const bool gemm = T >= GEMM_MIN_T;
-  // below GEMM_MIN_T most experts get at most 4 tokens: tiles of DEC_MT for
-  // the LDS-staged items (c3 T=64: 629 -> 477 us against 16-token tiles)
+  const bool gemm = expert_gemm_at(*s, T);
   const int mt = gemm ? GEMM_MT : DEC_MT;
   DispatchOut d = dispatch_out(s, L, ws, T);
   d.mt = mt;
@@ -555,7 +553,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
   // prefill (T >= GEMM_MIN_T, unfused dispatch): the selection builds the
   // dispatch's per-chunk token masks itself, so the dispatch needs no counting launch
   unsigned long long *cmask =
-      gemm && !fused ? at<unsigned long long>(ws, L.chunk_masks) : nullptr;
+      T >= GEMM_MIN_T ? at<unsigned long long>(ws, L.chunk_masks) : nullptr;
   if (T > EXACT_ROUTER_MAX_T)
     HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
                                at<float>(ws, L.logits), at<float>(ws, L.wnorm),
@@ -1027,7 +1025,7 @@ int ainfer_moe_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, c
   hipStream_t st = (hipStream_t)stream;
   const Layout L = layout_of(*s, T);
   const int H = s->hidden, k = s->top_k, has_shared = s->shared_inter > 0;
-  const bool gemm = T >= GEMM_MIN_T;
+  const bool gemm = expert_gemm_at(*s, T);
   DispatchOut d = dispatch_out(s, L, ws, T);
   d.mt = gemm ? GEMM_MT : DEC_MT;
   ProfCall pc(st);

@@ -52,12 +52,30 @@ hipError_t launch_router_gemm(const void *x, const void *rw, const float *bias, 
                               hipStream_t s);
 hipError_t launch_expert_gemm(int mode, int scale_dtype, GemmArgs a, int max_tiles,
                               hipStream_t s);
-// token-tile height of the prefill GEMM and the T above which it is used
+// token-tile height of the prefill GEMM
 constexpr int GEMM_MT = 64;
 #ifndef GEMM_WN
 #define GEMM_WN 4       // waves per GEMM block, 64 weight rows each
 #endif
+// from this many tokens on the router's approximate logits come from the
+// tiled GEMM (k_router_gemm), k_select runs one wave per token, and the
+// experts always run as the grouped GEMM
 constexpr int GEMM_MIN_T = 256;
+// Experts as the grouped GEMM (64-token tiles) or as streaming items of at
+// most DEC_MT tokens, for 16 < T.  The items re-read an expert's weights for
+// every 4 of its tokens; the GEMM reads them once but needs enough items to
+// fill the chip.  Measured crossover in tokens per expert (T k / E): 2.6 at
+// H2048 E512 k10 I512 (T=160: 225 us items, 210 GEMM; T=96: 175, 188), 1.9 at
+// H4096 I1024, 3 at E64 k8 and E32 k4, 3.2 at E128 k8, 3.5 at H3072 E324 k5
+// I256.  With fewer than 128 GEMM items in a stage a launch leaves half the
+// CUs idle and the crossover is 12 to 14 (E8 k2 I1024, E66 k5 I128).
+inline bool expert_gemm_at(const ainfer_moe_shape &s, int T) {
+  if (T >= GEMM_MIN_T) return true;
+  if (T <= 16) return false;
+  const long E = s.n_experts, slots = (long)T * s.top_k;
+  const long gu = E * (s.inter / 128), dn = E * ((s.hidden + 255) / 256);
+  return (gu < dn ? gu : dn) >= 128 ? 4 * slots >= 13 * E : slots >= 16 * E;
+}
 
 // Outputs of the dispatch stage.  tiles: (expert, first position, rows,
 // first row within the expert); shared-expert tiles carry expert id E and a

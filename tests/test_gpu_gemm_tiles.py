@@ -88,3 +88,43 @@ def test_expert_rows_at_tile_edges(torch, oracle, H, I, Is, which, scales):
     check(every * 2 + 1, every, ("w_", "s_"), E - 1, I)
     if Is:
         check(2 * T + every, every, ("ws_", "ss_"), 0, Is)
+
+
+# (H, E, k, I, Is) and the token counts either side of the rule that sends the
+# experts to the GEMM: 3.25 tokens per expert, or 16 where a stage has fewer
+# than 128 items
+EDGES = [((1024, 64, 8, 256, 256), (25, 26, 64, 65)),
+         ((512, 8, 2, 256, 384), (63, 64, 65)),
+         ((640, 130, 3, 128, 0), (140, 141))]
+
+
+@pytest.mark.parametrize("dims,T", [(d, t) for d, ts in EDGES for t in ts])
+def test_forward_either_side_of_the_gemm_rule(torch, oracle, dims, T):
+    """The whole layer on both sides of the rule, in the fused (T <= 64) and
+    the staged dispatch, against the oracle, and its stages composed against
+    it (the stage entry takes the same rule)."""
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    print(f"[case] gemm rule {dims} T={T}", flush=True)
+    H, E, k, I, Is = dims
+    cfg = MoeConfig("rule", H, E, k, I, Is, (T,), seed=3)
+    ly = MoeLayer(cfg)
+    x = make_input(cfg, T)
+    ws = ly.workspace(T)
+    y = torch.full((T, H), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ly.forward(x, y, ws)
+    idx, w, sg, _ = ly.route(x, ws)
+    y2 = torch.empty_like(y)
+    ly.combine(ly.experts(x, idx, ws), w, sg, y2)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+
+    def bits(t):
+        return (t.view(torch.int16) if t.dtype in (torch.bfloat16, torch.float16) else t).cpu().numpy()
+
+    host = oracle.HostLayer(cfg.shape_tuple(), {
+        n: None if t is None else bits(t).view(np.uint16) if t.dtype in (torch.bfloat16, torch.float16)
+        else bits(t) for n, t in ly.t.items()}, ly.shape.scale_dtype)
+    ref = host.forward(bits(x).view(np.uint16), T).astype(np.float64)
+    got = y.double().cpu().numpy()
+    assert np.abs(got - ref).max() <= 2e-2 * np.abs(ref).max()  # the layer's bf16 tolerance
