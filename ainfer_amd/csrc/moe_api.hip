@@ -280,52 +280,30 @@ ExpertArgs expert_args(const ainfer_moe_shape *s, const ainfer_moe_weights *w, c
 // the routing kernel applies the RMSNorm itself
 int down_kbw(const ainfer_moe_shape &s) { return down_kbw_of(s); }
 
-// The layer in W4A8 (AINFER_PRECISION_W4A8): the routing and dispatch of
-// the W4A16 path, then x quantized, the grouped gate/up GEMVs with SiLU, act
+// The layer in W4A8 (AINFER_PRECISION_W4A8) at decode sizes: the W4A16 decode
+// routing kernel (canonical logits, top-k, weights, gate, the MFMA-order copy
+// of x with its W4A8 codes, the dispatch in tiles of DEC_MT tokens, and with
+// norm the block's RMSNorm), the grouped gate/up GEMVs with SiLU, act
 // quantized, the grouped down GEMVs and the fp32 combine (moe_w4a8.hip).
-// Decode sizes take the W4A16 decode routing kernel (canonical logits,
-// top-k, weights, gate, the MFMA-order copy of x with its W4A8 codes, the
-// dispatch in tiles of DEC_MT tokens, and with norm the block's RMSNorm);
-// larger T the staged router, 16-token tiles and x quantized on its own.
-int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void *x,
-                    const void *resid, void *y, int T, void *ws, hipStream_t st, ProfCall *pc,
-                    const NormIn *norm = nullptr) {
+int do_decode_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void *x,
+                   const void *resid, void *y, int T, void *ws, hipStream_t st, ProfCall *pc,
+                   const NormIn *norm) {
   const Layout L = layout_of(*s, T);
   const int E = s->n_experts, k = s->top_k, H = s->hidden, I = s->inter, Is = s->shared_inter;
   const int has_shared = Is > 0;
   DispatchOut d = dispatch_out(s, L, ws, T);
-  const bool decode = T <= DECODE_MAX_T && E <= 1024 && (!norm || T <= DECODE_NORM_MAX_T);
-  if (norm && !decode) return AINFER_ERR_ARG;  // the caller normalizes above that
-  d.mt = decode ? DEC_MT : W8_MT;
-  if (decode) {
-    DispatchOut dr = d;  // nothing here reads the per-expert counts or offsets
-    dr.counts = nullptr;
-    dr.offsets = nullptr;
-    int32_t *sync = at<int32_t>(ws, L.sync);
-    HIP_TRY(launch_route_decode(x, w->router_w, w->router_bias, w->shared_gate_w,
-                                at<float>(ws, L.logits), at<float>(ws, L.sg_logit),
-                                at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
-                                at<uint16_t>(ws, L.xperm), T, H, E, k, has_shared, &dr, sync,
-                                (uint32_t *)(sync + L.slots), norm, st, at<int8_t>(ws, L.w8_xq),
-                                at<float>(ws, L.w8_xs)));
-    pc->end(3);
-  } else if (T <= EXACT_ROUTER_MAX_T)
-    HIP_TRY(launch_router_exact(x, w->router_w, w->router_bias, w->shared_gate_w,
-                                at<float>(ws, L.logits), at<float>(ws, L.sg_logit),
-                                at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
-                                at<uint16_t>(ws, L.xperm), T, H, E, k, has_shared, nullptr, st));
-  else
-    HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
-                               at<float>(ws, L.logits), at<float>(ws, L.wnorm),
-                               at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
-                               at<uint16_t>(ws, L.xperm), nullptr, T, H, E, k, has_shared,
-                               nullptr, st));
-  if (!decode) {
-    pc->end(2);
-    HIP_TRY(launch_dispatch(at<int32_t>(ws, L.idx), T, k, E, W8_MT, has_shared,
-                            at<int32_t>(ws, L.chunk_counts), at<int32_t>(ws, L.rank), d, st));
-    pc->end(3);
-  }
+  d.mt = DEC_MT;
+  DispatchOut dr = d;  // nothing here reads the per-expert counts or offsets
+  dr.counts = nullptr;
+  dr.offsets = nullptr;
+  int32_t *sync = at<int32_t>(ws, L.sync);
+  HIP_TRY(launch_route_decode(x, w->router_w, w->router_bias, w->shared_gate_w,
+                              at<float>(ws, L.logits), at<float>(ws, L.sg_logit),
+                              at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
+                              at<uint16_t>(ws, L.xperm), T, H, E, k, has_shared, &dr, sync,
+                              (uint32_t *)(sync + L.slots), norm, st, at<int8_t>(ws, L.w8_xq),
+                              at<float>(ws, L.w8_xs)));
+  pc->end(3);
   W4A8Args a;
   memset(&a, 0, sizeof a);
   a.xq = at<int8_t>(ws, L.w8_xq);
@@ -347,9 +325,6 @@ int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, cons
   a.I = I;
   a.Is = Is;
   const int mtb = max_tiles_bound(*s, T, d.mt);
-  if (!decode)  // the decode routing kernel wrote the codes with its x copy
-    HIP_TRY(launch_act_quant_i8(x, AINFER_ACT_BF16, T, H, at<int8_t>(ws, L.w8_xq),
-                                at<float>(ws, L.w8_xs), st));
   a.w0 = w->w_gate;
   a.w1 = w->w_up;
   a.s0 = (const uint16_t *)w->s_gate;
@@ -371,6 +346,85 @@ int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, cons
   HIP_TRY(launch_w4a8_expert(1, s->scale_dtype, a, mtb, st));
   pc->end(5);
   HIP_TRY(launch_combine_f32(a.o, d.inv, at<float>(ws, L.w), at<float>(ws, L.sg), has_shared,
+                             resid, y, T, k, H, at<int32_t>(ws, L.sync) + SY_ERR, st));
+  pc->end(6);
+  return AINFER_OK;
+}
+
+// The same layer above the decode sizes: the staged router (k_select
+// quantizes x into W8 order), 64-token tiles, the gate/up GEMM (which
+// quantizes act), the down GEMM and the fp32 combine (moe_gemm_w4a8.hip).
+int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void *x,
+                    const void *resid, void *y, int T, void *ws, hipStream_t st, ProfCall *pc,
+                    const NormIn *norm = nullptr) {
+  if (T <= DECODE_MAX_T) return do_decode_w4a8(s, w, x, resid, y, T, ws, st, pc, norm);
+  if (norm) return AINFER_ERR_ARG;  // the caller normalizes at these sizes
+  const Layout L = layout_of(*s, T);
+  const int E = s->n_experts, k = s->top_k, H = s->hidden;
+  const int has_shared = s->shared_inter > 0;
+  DispatchOut d = dispatch_out(s, L, ws, T);
+  d.mt = gemm_mt(*s, T);
+  const bool fused = T <= FUSED_DISPATCH_MAX_T;
+  unsigned long long *cmask =
+      T >= GEMM_MIN_T ? at<unsigned long long>(ws, L.chunk_masks) : nullptr;
+  // the group sums take the places of the W4A16 GEMM's (the same counts of
+  // 4-byte values)
+  W8Rows xq, aq, aqs;
+  xq.q = at<int8_t>(ws, L.w8_xq);
+  xq.s = at<float>(ws, L.w8_xs);
+  xq.sum = at<int32_t>(ws, L.xsum);
+  aq.q = at<int8_t>(ws, L.w8_aq);
+  aq.s = at<float>(ws, L.w8_as);
+  aq.sum = at<int32_t>(ws, L.asum);
+  aqs.q = at<int8_t>(ws, L.w8_aqs);
+  aqs.s = at<float>(ws, L.w8_ass);
+  aqs.sum = at<int32_t>(ws, L.asum_s);
+  HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
+                             at<float>(ws, L.logits), at<float>(ws, L.wnorm),
+                             at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
+                             nullptr, nullptr, T, H, E, k, has_shared, fused ? &d : nullptr, st,
+                             cmask ? at<int32_t>(ws, L.chunk_counts) : nullptr, cmask, xq));
+  pc->end(2);
+  if (!fused)
+    HIP_TRY(launch_dispatch(at<int32_t>(ws, L.idx), T, k, E, d.mt, has_shared,
+                            at<int32_t>(ws, L.chunk_counts), at<int32_t>(ws, L.rank), d, st,
+                            cmask));
+  pc->end(3);
+  W8GemmArgs g;
+  memset(&g, 0, sizeof g);
+  g.x = xq;
+  g.act = aq;
+  g.act_s = aqs;
+  g.o = at<float>(ws, L.w8_o);
+  g.ptok = d.ptok;
+  g.tiles = d.tiles;
+  g.n_tiles = d.n_tiles;
+  g.T = T;
+  g.k = k;
+  g.E = E;
+  g.H = H;
+  g.I = s->inter;
+  g.Is = s->shared_inter;
+  g.w0 = w->w_gate;
+  g.w1 = w->w_up;
+  g.s0 = (const uint16_t *)w->s_gate;
+  g.s1 = (const uint16_t *)w->s_up;
+  g.ws0 = w->ws_gate;
+  g.ws1 = w->ws_up;
+  g.ss0 = (const uint16_t *)w->ss_gate;
+  g.ss1 = (const uint16_t *)w->ss_up;
+  const int gtiles = max_tiles_bound(*s, T, d.mt);
+  HIP_TRY(launch_w4a8_gemm(0, s->scale_dtype, g, gtiles, st));
+  pc->end(4);
+  g.w0 = w->w_down;
+  g.s0 = (const uint16_t *)w->s_down;
+  g.ws0 = w->ws_down;
+  g.ss0 = (const uint16_t *)w->ss_down;
+  g.w1 = g.ws1 = nullptr;
+  g.s1 = g.ss1 = nullptr;
+  HIP_TRY(launch_w4a8_gemm(1, s->scale_dtype, g, gtiles, st));
+  pc->end(5);
+  HIP_TRY(launch_combine_f32(g.o, d.inv, at<float>(ws, L.w), at<float>(ws, L.sg), has_shared,
                              resid, y, T, k, H, at<int32_t>(ws, L.sync) + SY_ERR, st));
   pc->end(6);
   return AINFER_OK;
@@ -398,7 +452,7 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
     g.xsum = at<float>(ws, L.xsum);
     g.asum = at<float>(ws, L.asum);
     g.asum_s = at<float>(ws, L.asum_s);
-    const int gtiles = max_tiles_bound(*s, T, GEMM_MT);
+    const int gtiles = max_tiles_bound(*s, T, d.mt);
     g.w0 = w->w_gate;
     g.w1 = w->w_up;
     g.s0 = (const uint16_t *)w->s_gate;
@@ -497,7 +551,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
   const int has_shared = s->shared_inter > 0;
   const bool fused = T <= FUSED_DISPATCH_MAX_T;
   const bool gemm = expert_gemm_at(*s, T);
-  const int mt = gemm ? GEMM_MT : DEC_MT;
+  const int mt = gemm ? gemm_mt(*s, T) : DEC_MT;
   DispatchOut d = dispatch_out(s, L, ws, T);
   d.mt = mt;
   DecodeGeom dg;
@@ -1027,7 +1081,7 @@ int ainfer_moe_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, c
   const int H = s->hidden, k = s->top_k, has_shared = s->shared_inter > 0;
   const bool gemm = expert_gemm_at(*s, T);
   DispatchOut d = dispatch_out(s, L, ws, T);
-  d.mt = gemm ? GEMM_MT : DEC_MT;
+  d.mt = gemm ? gemm_mt(*s, T) : DEC_MT;
   ProfCall pc(st);
   pc.start();
   HIP_TRY(launch_xperm(x, at<uint16_t>(ws, L.xperm), gemm ? at<float>(ws, L.xsum) : nullptr, T,

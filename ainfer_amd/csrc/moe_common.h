@@ -376,15 +376,18 @@ __device__ __forceinline__ uint32_t norm_pair(uint32_t xp, uint32_t wp, float in
 
 // q8 / sq8 (optional): the row's W4A8 codes and group scales as well, the
 // arithmetic of k_act_quant_i8 (ScalesMax + Quantize, kernels.cpp:551-579)
-// on the values written (the 4 lanes holding a 128-wide group share its max)
+// on the values written (the 4 lanes holding a 128-wide group share its max).
+// qsum8 (optional): the codes in W8 order (inside every 32-element block the
+// 16 even elements, then the 16 odd ones: the order the W4A8 GEMM unpacks
+// nibbles in) and -8 x the sum of each group's codes.  xperm may be null.
 __device__ __forceinline__ void write_xperm(const uint16_t *__restrict__ xrow,
                                             uint16_t *__restrict__ xperm,
                                             float *__restrict__ xsum, int t, int H, int lane,
                                             const NormIn *norm = nullptr, float inv = 1.0f,
                                             int8_t *__restrict__ q8 = nullptr,
-                                            float *__restrict__ sq8 = nullptr) {
+                                            float *__restrict__ sq8 = nullptr,
+                                            int32_t *__restrict__ qsum8 = nullptr) {
   {
-    uint16_t *xo = xperm + (size_t)t * H;
     for (int b = lane; b < (H >> 5); b += 64) {
       const u32x4 *src = (const u32x4 *)(xrow + b * 32);
       const u32x4 s0 = src[0], s1 = src[1], s2 = src[2], s3 = src[3];
@@ -400,21 +403,23 @@ __device__ __forceinline__ void write_xperm(const uint16_t *__restrict__ xrow,
 #pragma unroll
         for (int i = 0; i < 16; ++i) in[i] = norm_pair(in[i], wv[i >> 2][i & 3], inv, *norm);
       }
-      uint32_t out[16];
+      if (xperm) {
+        uint32_t out[16];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-          const int ka = 8 * e2 + j, kb = ka + 4;
-          const uint32_t lo = (in[ka >> 1] >> (16 * (ka & 1))) & 0xFFFFu;
-          const uint32_t hi = (in[kb >> 1] >> (16 * (kb & 1))) & 0xFFFFu;
-          out[4 * j + e2] = lo | (hi << 16);
-        }
-      u32x4 *dst = (u32x4 *)(xo + b * 32);
-      dst[0] = u32x4{out[0], out[1], out[2], out[3]};
-      dst[1] = u32x4{out[4], out[5], out[6], out[7]};
-      dst[2] = u32x4{out[8], out[9], out[10], out[11]};
-      dst[3] = u32x4{out[12], out[13], out[14], out[15]};
+          for (int e2 = 0; e2 < 4; ++e2) {
+            const int ka = 8 * e2 + j, kb = ka + 4;
+            const uint32_t lo = (in[ka >> 1] >> (16 * (ka & 1))) & 0xFFFFu;
+            const uint32_t hi = (in[kb >> 1] >> (16 * (kb & 1))) & 0xFFFFu;
+            out[4 * j + e2] = lo | (hi << 16);
+          }
+        u32x4 *dst = (u32x4 *)(xperm + (size_t)t * H + b * 32);
+        dst[0] = u32x4{out[0], out[1], out[2], out[3]};
+        dst[1] = u32x4{out[4], out[5], out[6], out[7]};
+        dst[2] = u32x4{out[8], out[9], out[10], out[11]};
+        dst[3] = u32x4{out[12], out[13], out[14], out[15]};
+      }
       if (xsum) {
         // sum of the 128-wide group: this block's 32 values, then the 4
         // consecutive lanes holding the group's blocks (fixed order)
@@ -442,6 +447,7 @@ __device__ __forceinline__ void write_xperm(const uint16_t *__restrict__ xrow,
         float sc = m / 127.0f;
         sc = sc == 0.0f ? 1.0f : sc;
         uint32_t pk[8];
+        int qs = 0;
 #pragma unroll
         for (int i2 = 0; i2 < 8; ++i2) pk[i2] = 0u;
 #pragma unroll
@@ -452,6 +458,20 @@ __device__ __forceinline__ void write_xperm(const uint16_t *__restrict__ xrow,
           int qi = (int)(r >= 0.0f ? r + 0.5f : r - 0.5f);
           qi = qi < -127 ? -127 : (qi > 127 ? 127 : qi);
           pk[i2 >> 2] |= (uint32_t)(uint8_t)qi << (8 * (i2 & 3));
+          qs += qi;
+        }
+        if (qsum8) {
+          uint32_t eo[8];  // even elements' bytes, then the odd ones'
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            eo[d] = __builtin_amdgcn_perm(pk[2 * d + 1], pk[2 * d], 0x06040200u);
+            eo[4 + d] = __builtin_amdgcn_perm(pk[2 * d + 1], pk[2 * d], 0x07050301u);
+          }
+#pragma unroll
+          for (int d = 0; d < 8; ++d) pk[d] = eo[d];
+          qs += __shfl_xor(qs, 1, 64);
+          qs += __shfl_xor(qs, 2, 64);
+          if ((b & 3) == 0) qsum8[(size_t)t * (H >> 7) + (b >> 2)] = -8 * qs;
         }
         u32x4 *qd = (u32x4 *)(q8 + (size_t)t * H + b * 32);
         qd[0] = u32x4{pk[0], pk[1], pk[2], pk[3]};

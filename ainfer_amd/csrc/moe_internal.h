@@ -52,8 +52,22 @@ hipError_t launch_router_gemm(const void *x, const void *rw, const float *bias, 
                               hipStream_t s);
 hipError_t launch_expert_gemm(int mode, int scale_dtype, GemmArgs a, int max_tiles,
                               hipStream_t s);
-// token-tile height of the prefill GEMM
+// token-tile height of the expert GEMMs (at most)
 constexpr int GEMM_MT = 64;
+// The height a call uses: the largest of 64, 32 and 16 that gives the gate/up
+// stage an item for every CU, and 16 only up to 64 tokens per expert.  A lower
+// tile re-reads weights through L2, but below one item per CU its shorter
+// items run side by side (E8 k2 I1024, T = 128: 58 -> 48 us, in W4A8 66 -> 48;
+// E66 k5 I128 T = 512: 109 -> 99 us, but 16 at T = 1024: 121 -> 128).
+inline int gemm_mt(const ainfer_moe_shape &s, int T) {
+  const long slots = (long)T * s.top_k, hit = slots < s.n_experts ? slots : s.n_experts;
+  int mt = GEMM_MT;
+  // tiles: the full ones and, on average, half a tile more per expert
+  while (mt > 16 && (slots / mt + hit / 2) * (s.inter / 128) < 256 &&
+         (mt > 32 || slots <= 64 * hit))
+    mt /= 2;
+  return mt;
+}
 #ifndef GEMM_WN
 #define GEMM_WN 4       // waves per GEMM block, 64 weight rows each
 #endif
@@ -61,21 +75,45 @@ constexpr int GEMM_MT = 64;
 // tiled GEMM (k_router_gemm), k_select runs one wave per token, and the
 // experts always run as the grouped GEMM
 constexpr int GEMM_MIN_T = 256;
-// Experts as the grouped GEMM (64-token tiles) or as streaming items of at
-// most DEC_MT tokens, for 16 < T.  The items re-read an expert's weights for
-// every 4 of its tokens; the GEMM reads them once but needs enough items to
-// fill the chip.  Measured crossover in tokens per expert (T k / E): 2.6 at
-// H2048 E512 k10 I512 (T=160: 225 us items, 210 GEMM; T=96: 175, 188), 1.9 at
-// H4096 I1024, 3 at E64 k8 and E32 k4, 3.2 at E128 k8, 3.5 at H3072 E324 k5
-// I256.  With fewer than 128 GEMM items in a stage a launch leaves half the
-// CUs idle and the crossover is 12 to 14 (E8 k2 I1024, E66 k5 I128).
+// Experts as the grouped GEMM or as streaming items of at most DEC_MT tokens,
+// for 16 < T.  The items re-read an expert's weights for every 4 of its
+// tokens; the GEMM reads them once but needs enough items to fill the chip.
+// Measured crossover in tokens per expert (T k / E): 2.6 at H2048 E512 k10
+// I512 (T=160: 225 us items, 210 GEMM; T=96: 175, 188), 1.9 at H4096 I1024, 2
+// to 3 at E64 k8 and E32 k4, 3.2 at E128 k8, 3.5 at H3072 E324 k5 I256; 5 at
+// E8 k2 I4096 and E66 k5 H3584 I128, one of whose stages has fewer than 128
+// items; 12 at E8 k2 I1024 (T=32: 38 us items, 41 GEMM; T=64: 47, 41), where
+// both have.
 inline bool expert_gemm_at(const ainfer_moe_shape &s, int T) {
   if (T >= GEMM_MIN_T) return true;
   if (T <= 16) return false;
   const long E = s.n_experts, slots = (long)T * s.top_k;
   const long gu = E * (s.inter / 128), dn = E * ((s.hidden + 255) / 256);
-  return (gu < dn ? gu : dn) >= 128 ? 4 * slots >= 13 * E : slots >= 16 * E;
+  const long quarters = (gu < dn ? gu : dn) >= 128 ? 13 : gu + dn >= 256 ? 20 : 48;
+  return 4 * slots >= quarters * E;
 }
+
+// Rows quantized for the W4A8 GEMM: codes in W8 order (write_xperm,
+// moe_common.h), their scales per 128-wide group, -8 x each group's code sum.
+struct W8Rows {
+  int8_t *q = nullptr;
+  float *s = nullptr;
+  int32_t *sum = nullptr;
+};
+// Arguments of the W4A8 GEMM (moe_gemm_w4a8.hip).
+struct W8GemmArgs {
+  const uint8_t *w0, *w1, *ws0, *ws1;  // MODE 0: gate, up; MODE 1: down (w0 / ws0)
+  const uint16_t *s0, *s1, *ss0, *ss1;
+  W8Rows x, act, act_s;  // [T][H]; [T k][I], [T][Is] (MODE 0 out, MODE 1 in)
+  float *o;              // MODE 1 out: [T k + T][H]
+  const int32_t *ptok;
+  const int4 *tiles;     // of at most GEMM_MT tokens
+  const int32_t *n_tiles;
+  int T, k, E, H, I, Is;
+  int n_nblk;            // set by the launcher
+};
+hipError_t launch_w4a8_gemm(int mode, int scale_dtype, W8GemmArgs a, int max_tiles,
+                            hipStream_t s);
 
 // Outputs of the dispatch stage.  tiles: (expert, first position, rows,
 // first row within the expert); shared-expert tiles carry expert id E and a
@@ -108,7 +146,8 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
                               float *approx, float *wnorm, int32_t *idx, float *w, float *sg,
                               void *xperm, float *xsum, int T, int H, int E, int k,
                               int has_shared, const DispatchOut *fused, hipStream_t s,
-                              int32_t *ccount = nullptr, unsigned long long *cmask = nullptr);
+                              int32_t *ccount = nullptr, unsigned long long *cmask = nullptr,
+                              W8Rows w8 = W8Rows());
 // Small T: canonical logits of all experts on VALU (k_router_logits), then the
 // same selection without the refine.  logits [T][E], sg_logit [T] out.
 hipError_t launch_router_exact(const void *x, const void *rw, const float *bias, const void *gw,
@@ -213,9 +252,8 @@ struct DecodeGeom {
   size_t lds;              // dynamic LDS bytes
 };
 // W4A8 GEMV numerics (moe_w4a8.hip)
-// The MoE layer in W4A8: the grouped expert GEMVs over dispatch tiles of at
-// most W8_MT tokens and the fp32 combine.
-constexpr int W8_MT = 16;
+// The MoE layer in W4A8 at decode sizes: the grouped expert GEMVs over
+// dispatch tiles of at most DEC_MT tokens and the fp32 combine.
 struct W4A8Args {
   const uint8_t *w0, *w1, *ws0, *ws1;     // MODE 0: gate, up; MODE 1: down (w0/ws0)
   const uint16_t *s0, *s1, *ss0, *ss1;

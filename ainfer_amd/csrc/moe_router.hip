@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
                                                 float *__restrict__ topk_w,
                                                 float *__restrict__ sgate,
                                                 uint16_t *__restrict__ xperm,
-                                                float *__restrict__ xsum, int T, int E,
+                                                float *__restrict__ xsum, W8Rows w8, int T, int E,
                                                 int k, int H, int has_shared, DispatchOut ds,
                                                 int fused, unsigned long long *cmask,
                                                 int32_t *ccount) {
@@ -241,7 +241,8 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
     // the MFMA-order copy of x (and its group sums) does not depend on the
     // routing: written first, its latency hides under the selection
     STRACE(0);
-    if (xperm && (!COOP || wave == 1)) write_xperm(x + (size_t)t * H, xperm, xsum, t, H, lane);
+    if ((xperm || w8.q) && (!COOP || wave == 1))
+      write_xperm(x + (size_t)t * H, xperm, xsum, t, H, lane, nullptr, 1.0f, w8.q, w8.s, w8.sum);
     STRACE(1);
     const float *ar = approx + (size_t)t * E;
     // ---- k-th largest approximate logit -------------------------------
@@ -521,12 +522,12 @@ template <int NV, bool EXACT, bool COOP>
 hipError_t launch_select_nv(int ch, unsigned grid, const float *approx, const float *sgl,
                             const float *wnorm,
                             const void *x, const void *rw, const float *bias, const void *gw,
-                            int32_t *idx, float *w, float *sg, void *xperm, float *xsum, int T,
+                            int32_t *idx, float *w, float *sg, void *xperm, float *xsum, W8Rows w8, int T,
                             int E, int k, int H, int has_shared, const DispatchOut &ds, int fused,
                             unsigned long long *cmask, int32_t *ccount, hipStream_t s) {
 #define SEL_ARGS                                                                            \
   approx, sgl, wnorm, (const uint16_t *)x, (const uint16_t *)rw, bias, (const uint16_t *)gw, idx, \
-      w, sg, (uint16_t *)xperm, xsum, T, E, k, H, has_shared, ds, fused, cmask, ccount
+      w, sg, (uint16_t *)xperm, xsum, w8, T, E, k, H, has_shared, ds, fused, cmask, ccount
   switch (ch) {
   case 1: k_select<NV, 1, EXACT, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
   case 2: k_select<NV, 2, EXACT, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
@@ -544,7 +545,7 @@ bool router_supported(int H, int E) { return H % 128 == 0 && H <= 4096 && E <= 1
 template <bool EXACT>
 hipError_t launch_select(const float *approx, const float *sgl, const float *wnorm,
                          const void *x, const void *rw, const float *bias, const void *gw,
-                         int32_t *idx, float *w, float *sg, void *xperm, float *xsum, int T,
+                         int32_t *idx, float *w, float *sg, void *xperm, float *xsum, W8Rows w8, int T,
                          int H, int E, int k, int has_shared, const DispatchOut *fused,
                          hipStream_t s, unsigned long long *cmask = nullptr,
                          int32_t *ccount = nullptr) {
@@ -560,10 +561,10 @@ hipError_t launch_select(const float *approx, const float *sgl, const float *wno
   const int fz = fused ? 1 : 0;
 #define SEL_CALL(NVV)                                                                          \
   (coop ? launch_select_nv<NVV, EXACT, !EXACT>(chp, g, approx, sgl, wnorm, x, rw, bias, gw, idx, \
-                                              w, sg, xperm, xsum, T, E, k, H, has_shared, ds, \
+                                              w, sg, xperm, xsum, w8, T, E, k, H, has_shared, ds, \
                                               fz, cmask, ccount, s)                           \
         : launch_select_nv<NVV, EXACT, false>(chp, g, approx, sgl, wnorm, x, rw, bias, gw, idx, \
-                                              w, sg, xperm, xsum, T, E, k, H, has_shared, ds, \
+                                              w, sg, xperm, xsum, w8, T, E, k, H, has_shared, ds, \
                                               fz, cmask, ccount, s))
   if (nv <= 1) return SEL_CALL(1);
   if (nv <= 2) return SEL_CALL(2);
@@ -577,7 +578,7 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
                               float *approx, float *wnorm, int32_t *idx, float *w, float *sg,
                               void *xperm, float *xsum, int T, int H, int E, int k,
                               int has_shared, const DispatchOut *fused, hipStream_t s,
-                              int32_t *ccount, unsigned long long *cmask) {
+                              int32_t *ccount, unsigned long long *cmask, W8Rows w8) {
   if (T == 0) return hipSuccess;
   // ---- approximate logits + row norms ------------------------------------
   if (T >= GEMM_MIN_T) {
@@ -588,7 +589,7 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
                                         (int)(zb / 4), s);
     if (err != hipSuccess) return err;
     return launch_select<false>(approx, nullptr, wnorm, x, rw, bias, gw, idx, w, sg, xperm,
-                                xsum, T, H, E, k, has_shared, fused, s, cmask, ccount);
+                                xsum, w8, T, H, E, k, has_shared, fused, s, cmask, ccount);
   }
   // one 16-token tile per workgroup: more workgroups share the token reads
   // (c3 T=64: 55 -> 44 us against 64-token tiles; the router rows are
@@ -608,7 +609,7 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
   if (err != hipSuccess) return err;
   // ---- refine + select ------------------------------------------------------
   return launch_select<false>(approx, nullptr, wnorm, x, rw, bias, gw, idx, w, sg, xperm, xsum,
-                              T, H, E, k, has_shared, fused, s);
+                              w8, T, H, E, k, has_shared, fused, s);
 }
 
 hipError_t launch_router_exact(const void *x, const void *rw, const float *bias, const void *gw,

@@ -1,7 +1,7 @@
 """The prefill expert GEMM at the edges of its tiles: experts of 1 to 300
-tokens (every 16-token subtile count, full and partial 64-token tiles), K of
-1, 7, 15, 18 and 32 quantization groups (one and two table windows, odd and
-4-divisible group counts), rows that do not fill a block.
+tokens (every 16-token subtile count; tiles of at most 16, 32 and 64 tokens,
+which the shapes below take), K of 1, 2, 5, 11, 15, 18 and 32 quantization
+groups (odd and even), rows that do not fill a block.
 
 Each expert row is compared with the float64 MLP of the dequantised weights.
 The bound per element is what the arithmetic states: fp32 sums of n exact
@@ -38,8 +38,8 @@ def routing(counts):
 
 @pytest.mark.parametrize("scales", ["fp16", "bf16"])
 @pytest.mark.parametrize("which", ["low", "high"])
-@pytest.mark.parametrize("H,I,Is", [(4096, 128, 128), (2304, 256, 128), (1920, 896, 0),
-                                    (128, 128, 1920)])
+@pytest.mark.parametrize("H,I,Is", [(4096, 128, 128), (2304, 256, 128), (1920, 1408, 0),
+                                    (128, 128, 1920), (640, 2304, 256), (4096, 2304, 256)])
 def test_expert_rows_at_tile_edges(torch, oracle, H, I, Is, which, scales):
     from ainfer_amd import _lib as L
     from ainfer_amd.moe import MoeLayer, make_input
@@ -91,10 +91,11 @@ def test_expert_rows_at_tile_edges(torch, oracle, H, I, Is, which, scales):
 
 
 # (H, E, k, I, Is) and the token counts either side of the rule that sends the
-# experts to the GEMM: 3.25 tokens per expert, or 16 where a stage has fewer
-# than 128 items
+# experts to the GEMM: 3.25 tokens per expert, 5 and 12 where the stages have
+# few items
 EDGES = [((1024, 64, 8, 256, 256), (25, 26, 64, 65)),
-         ((512, 8, 2, 256, 384), (63, 64, 65)),
+         ((512, 8, 2, 256, 384), (47, 48, 65)),
+         ((3584, 20, 4, 128, 0), (24, 25)),
          ((640, 130, 3, 128, 0), (140, 141))]
 
 
@@ -128,3 +129,34 @@ def test_forward_either_side_of_the_gemm_rule(torch, oracle, dims, T):
     ref = host.forward(bits(x).view(np.uint16), T).astype(np.float64)
     got = y.double().cpu().numpy()
     assert np.abs(got - ref).max() <= 2e-2 * np.abs(ref).max()  # the layer's bf16 tolerance
+
+
+@pytest.mark.parametrize("scales", ["fp16", "bf16"])
+@pytest.mark.parametrize("H,E,k,I,Is", [(4096, 6, 2, 128, 128), (2304, 24, 3, 256, 1280),
+                                        (1920, 3, 1, 896, 0), (128, 5, 5, 128, 1920),
+                                        (1024, 64, 8, 384, 256), (1920, 12, 2, 1408, 0),
+                                        (640, 12, 2, 2304, 256)])
+def test_w4a8_gemm_gives_the_decode_rows(torch, H, E, k, I, Is, scales):
+    """In W4A8 a token's output does not depend on how many tokens share the
+    call: every product and sum is defined by the format, so the GEMM's rows
+    (T > 16: tiles of 1 to 64 tokens, fused, staged and counted dispatch)
+    equal, bit for bit, the decode kernels' rows of the same tokens in calls
+    of 16."""
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    sd = L.SCALE_FP16 if scales == "fp16" else L.SCALE_BF16
+    cfg = MoeConfig("w8tiles", H, E, k, I, Is, (T,), seed=78)
+    ly = MoeLayer(cfg, scale_dtype=sd, precision=L.PRECISION_W4A8)
+    x = make_input(cfg, T) * 2
+    x[3] = 0  # a group of zeros has scale 1
+    ws = ly.workspace(T)
+    want = torch.empty_like(x)
+    for t in range(0, T, 16):
+        ly.forward(x[t:t + 16], want[t:t + 16], ws)
+    for n in (17, 33, 64, 65, 150, T):
+        print(f"[case] w4a8 gemm H={H} E={E} I={I} Is={Is} {scales} T={n}", flush=True)
+        y = torch.full((n, H), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ly.forward(x[:n], y, ws)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want[:n].view(torch.int16)), n
