@@ -571,18 +571,22 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
     pc->end(2);
     ExpertArgs gu = expert_args(s, w, L, ws, d, T, 0), dn = expert_args(s, w, L, ws, d, T, 1);
     if (T <= FUSED_EXPERTS_MAX_T) {
-      // latency-bound: gate/up, down and combine in one launch (T = 1: the
-      // gate/up items in a launch of their own first)
+      // latency-bound: gate/up, down and combine in one launch (T = 1: gate/up,
+      // then down with the combine)
       if (T == 1) {
         pc->kernel_events();
         HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, max_tiles_bound(*s, T, DEC_MT), 4,
                                      DEC_RG_GATE_UP, st));
         pc->end(4);
+        HIP_TRY(launch_down_combine_t1(s->scale_dtype, dn, at<float>(ws, L.w), at<float>(ws, L.sg),
+                                       d.inv, resid, y, sync + SY_ERR, st));
+        pc->end(5);
+        return AINFER_OK;
       }
       HIP_TRY(launch_experts_decode(s->scale_dtype, dg, gu, dn, at<float>(ws, L.w),
                                     at<float>(ws, L.sg), d.inv, resid, y, sync,
                                     max_tiles_bound(*s, T, DEC_MT),
-                                    max_tiles_bound(*s, DECODE_MAX_T, DEC_MT), T == 1, st));
+                                    max_tiles_bound(*s, DECODE_MAX_T, DEC_MT), st));
     } else {
       // bandwidth-bound: three launches whose items hold no waits
       const int mtb = max_tiles_bound(*s, T, DEC_MT);

@@ -1,5 +1,5 @@
-// moe_decode.hip - the decode routing kernel (T <= 16 tokens) and the fused
-// expert kernel (T <= 2).
+// moe_decode.hip - the decode routing kernel (T <= 16 tokens), the fused
+// expert kernel (T = 2) and the one-token down + combine kernel.
 //
 // Measured on MI355X: a dependent kernel launch costs about 2.5 us, a flag
 // handed from one workgroup to another through device memory about 0.8 us,
@@ -28,10 +28,11 @@
 //                   the tile's act rows, writes its o rows, and counts one
 //                   arrival per (token, row slab).  The (k+1)-th arrival of a
 //                   (token, slab) sums the token's k + 1 rows of that slab in
-//                   slot order (the combine).  At T = 1 the gate/up items
-//                   run first in a launch of their own (k_expert_lds) and
-//                   this kernel holds only the down items, which then wait
-//                   for nothing.
+//                   slot order (the combine).
+//
+// At T = 1 the gate/up items run in a launch of their own (k_expert_lds), then
+// k_down_combine_t1: each workgroup owns 8 output rows of every selected
+// expert, so the combine is an LDS exchange and no counter is needed.
 //
 // A wait only ever names work of lower workgroup index, and workgroups are
 // dispatched in index order, so every awaited workgroup is already running.
@@ -359,10 +360,7 @@ struct ExpertsDecodeArgs {
 
 // One item per workgroup.  A down item only ever waits for gate/up items of
 // lower index, which the dispatcher has started, so the waits end.
-// SPLIT: the gate/up items ran in an earlier launch (k_expert_lds): this
-// launch holds only the down items, which need no wait and read act with
-// plain (cacheable) loads.
-template <int SD, int KBW_GU, int RG_GU, int KBW_DN, int RG_DN, bool SPLIT>
+template <int SD, int KBW_GU, int RG_GU, int KBW_DN, int RG_DN>
 __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(ExpertsDecodeArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   // one counter per 256-byte line: same-line atomics and polls serialise
@@ -372,7 +370,7 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
   const int sg = a.gu.n_slabs, sd = a.dn.n_slabs;
   const int n_gu = a.max_tiles * sg;
   {
-    const int item = blockIdx.x + (SPLIT ? n_gu : 0);
+    const int item = blockIdx.x;
     // ---- item -> (kind, tile, slab): all gate/up items (tile-major,
     // slab-minor), then all down items ---------------------------------------
     const int is_gu = item < n_gu;
@@ -388,7 +386,7 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
     // one item per workgroup, and no barrier before its loads: each wave
     // issues its weight loads as soon as it is launched (the waves of a
     // workgroup start up to about 1.5 us apart at the launch's start)
-    if (!SPLIT && is_gu) {
+    if (is_gu) {
       // x (MFMA order) comes from the routing kernel: plain, cacheable loads
       expert_lds_item<SD, KBW_GU, RG_GU, DEC_MT, 0, true, false>(a.gu, tt, slab, lds);
       if (threadIdx.x >= 64) return;
@@ -403,8 +401,8 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
     // the down weights are requested before the wait for the tile's act rows
     const int32_t *gdone = &gu_done[tile * SY_STRIDE];
     int32_t *err = a.sync + SY_ERR;
-    expert_lds_item<SD, KBW_DN, RG_DN, DEC_MT, 1, true, !SPLIT>(a.dn, td, slab, lds, [=]() {
-      if (!SPLIT) block_wait_geq(gdone, sg, err, a.spin);
+    expert_lds_item<SD, KBW_DN, RG_DN, DEC_MT, 1, true, true>(a.dn, td, slab, lds, [=]() {
+      block_wait_geq(gdone, sg, err, a.spin);
       DTRACE_AT(1, item, 1);
     });
     if (threadIdx.x >= 64) return;
@@ -412,7 +410,7 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
     // ---- wave 0: publish o; count this tile's down items and each token's
     // arrivals on this row slab --------------------------------------------
     wait_stores();
-    if (!SPLIT && lane == 0 && atomicAdd(&dn_done[tile * SY_STRIDE], 1) == sd - 1) {
+    if (lane == 0 && atomicAdd(&dn_done[tile * SY_STRIDE], 1) == sd - 1) {
       gu_done[tile * SY_STRIDE] = 0;  // all of the tile's down items have passed their wait
       dn_done[tile * SY_STRIDE] = 0;
     }
@@ -469,6 +467,139 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
       }
     }
   }
+}
+
+// ---- T = 1: down and combine in one launch ---------------------------------
+// A workgroup owns DC_ROWS output rows of every selected expert: wave j takes
+// tile j (one expert; the shared one last), all waves' weight loads are in
+// flight together (c4: 512 workgroups x 11 waves x 4 KB, the whole 23 MB), the
+// tiles' rows meet in LDS and one lane per row sums them in slot order.  Items
+// of 32 rows of one expert that counted arrivals per row slab and combined on
+// the last took 11.8 us at H4096 I1024 k10 + shared (each waits for its sc1
+// stores, an atomic, and the last for a read of the others' rows).
+// The arithmetic is the decode item's at KBW = 2 (moe_expert_item.h), bit for
+// bit: per 32-wide chunk 8 MFMAs from -136 sum x and the group scale, the 8
+// chunks of two groups added as ((c, c+4), (c, c+2), (c, c+1)), then those
+// sums in k order.
+constexpr int DC_ROWS = 8;
+struct DownT1Args {
+  ExpertArgs dn;
+  const float *w, *sg;
+  const int32_t *inv;
+  const uint16_t *resid;
+  uint16_t *y;
+  const int32_t *err;
+  int n_tiles;  // k (+ 1)
+};
+constexpr int dc_scale_lds(int nh) { return nh > 4 ? 512 : 256; }
+
+// NH: runs of 4 k-groups of the longer down product
+template <int SD, int NH>
+__global__ __launch_bounds__(1024) void k_down_combine_t1(DownT1Args a) {
+  __shared__ float s_o[33][DC_ROWS];
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  constexpr int SCB = dc_scale_lds(NH), WB = NH * 1024 + SCB;  // LDS bytes per wave
+  const int tx = tid_opaque();
+  const int wave = __builtin_amdgcn_readfirstlane(tx >> 6), lane = tx & 63;
+  const int nw = blockDim.x >> 6, k = a.dn.k, H = a.dn.H;
+  const int row0 = blockIdx.x * DC_ROWS;
+  // what the combine needs, requested before the weights (wave 0)
+  float wj = 0.f, rv = 0.f, sgv = 0.f;
+  int pj = 0;
+  bool bad = false;
+  if (wave == 0) {
+    wj = a.w[min(lane, k - 1)];
+    pj = a.inv[min(lane, k - 1)];
+    sgv = a.sg[0];
+    if (a.resid) rv = bf16_to_f32(a.resid[row0 + (lane & (DC_ROWS - 1))]);
+    bad = *a.err != 0;
+  }
+  const int r4 = lane & 3, c = lane >> 2;
+  uint8_t *wl = lds + wave * WB;
+  const uint32_t wl32 = (uint32_t)(uintptr_t)wl;
+  for (int tile = wave; tile < a.n_tiles; tile += nw) {
+    const bool shared = tile == k;
+    int n_unused;
+    const int e = shared ? 0 : sload_tile(a.dn.tiles, a.dn.n_tiles, tile, n_unused).x;
+    const int K = shared ? a.dn.Is : a.dn.I, KB = K >> 7;
+    const uint8_t *w0 = shared ? a.dn.ws0 : a.dn.w0 + (size_t)e * H * (K / 2);
+    const uint16_t *s0 = shared ? a.dn.ss0 : a.dn.s0 + (size_t)e * H * KB;
+    const uint8_t *act = (const uint8_t *)(shared ? a.dn.a_shared : a.dn.a_routed + (size_t)tile * K);
+    // lane (r4, c): 32 nibbles of row r4 of a row quad at chunk 16 h + c
+    u32x4 B[NH][2];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      const int ch = min(16 * h + c, 4 * KB - 1);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        B[h][q] = ldg_stream(w0 + (size_t)(row0 + 4 * q + r4) * (K / 2) + ch * 16);
+    }
+    // scales: lane (h, row, pair) copies the dword of groups 4 h + 2 pair + {0, 1}
+#pragma unroll
+    for (int i = 0; i < SCB / 256; ++i) {
+      const int pr = min(8 * i + 2 * (lane >> 4) + (lane & 1), KB / 2 - 1);
+      dma4(s0 + (size_t)(row0 + ((lane >> 1) & 7)) * KB + 2 * pr, wl32 + NH * 1024 + i * 256);
+    }
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+      if (i * 4 < KB) dma16(act + min(i * 1024 + lane * 16, K * 2 - 16), wl32 + i * 1024);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t magic;
+    asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    const s16x4 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+    const uint32_t mask = 0x000F000Fu;
+    const uint16_t *sl = (const uint16_t *)(wl + NH * 1024);
+    float gs[2] = {0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      if (4 * h >= KB) break;
+      s16x4 A[8];
+#pragma unroll
+      for (int jh = 0; jh < 8; ++jh) A[jh] = *(const s16x4 *)(wl + (16 * h + c) * 64 + jh * 8);
+      f32x4 xs = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int jh = 0; jh < 8; ++jh) xs = mfma_bf16_4x4x4(A[jh], ones, xs);
+      const f32x4 c0 = xs * -136.0f;
+      const bool in = 16 * h + c < 4 * KB;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const u32x4 bw = B[h][q] ^ 0x88888888u;
+        f32x4 acc = c0;
+#pragma unroll
+        for (int jh = 0; jh < 8; ++jh) {
+          const int j = jh >> 1, hf = jh & 1;
+          const uint32_t d0 = ((bw[2 * hf] >> (4 * j)) & mask) | magic;
+          const uint32_t d1 = ((bw[2 * hf + 1] >> (4 * j)) & mask) | magic;
+          acc = mfma_bf16_4x4x4(A[jh], __builtin_bit_cast(s16x4, u32x2{d0, d1}), acc);
+        }
+        // dword (h, row, pair) at 16 h + 2 row + pair; the group's half of it
+        const float sc = scale_to_f32<SD>(sl[2 * (16 * h + 2 * (4 * q + r4) + (c >> 3)) + ((c >> 2) & 1)]);
+        float v = in ? acc[0] * sc : 0.f;
+        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (16 << 10) | 0x1F));
+        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (8 << 10) | 0x1F));
+        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (4 << 10) | 0x1F));
+        // lanes 0-31 hold groups 4 h, 4 h + 1; lanes 32-63 the next two
+        gs[q] += v;
+        gs[q] += __shfl_xor(v, 32, 64);
+      }
+    }
+    if (lane < 4) {
+      s_o[tile][r4] = bf16_to_f32(f32_to_bf16(gs[0]));
+      s_o[tile][4 + r4] = bf16_to_f32(f32_to_bf16(gs[1]));
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  // ---- the combine, slot order (k_combine's arithmetic) ----------------------
+  const int r = lane & (DC_ROWS - 1);
+  float acc = 0.f;
+  for (int j = 0; j < k; ++j) {
+    const int p = __builtin_amdgcn_readlane(pj, j);
+    acc = __builtin_fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wj), j)), s_o[p][r], acc);
+  }
+  if (a.n_tiles > k) acc = __builtin_fmaf(sgv, s_o[k][r], acc);
+  if (a.resid) acc += rv;
+  if (lane < DC_ROWS) a.y[row0 + lane] = bad ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
 }
 
 }  // namespace
@@ -563,8 +694,7 @@ hipError_t launch_route_decode(const void *x, const void *rw, const float *bias,
 hipError_t launch_experts_decode(int scale_dtype, const DecodeGeom &g, ExpertArgs gu,
                                  ExpertArgs dn, const float *w, const float *sg,
                                  const int32_t *inv, const void *resid, void *y,
-                                 int32_t *sync, int max_tiles, int cap, bool split,
-                                 hipStream_t s) {
+                                 int32_t *sync, int max_tiles, int cap, hipStream_t s) {
   if (max_tiles <= 0) return hipSuccess;
   if (max_tiles > cap) return hipErrorInvalidValue;
   ExpertsDecodeArgs a;
@@ -589,20 +719,46 @@ hipError_t launch_experts_decode(int scale_dtype, const DecodeGeom &g, ExpertArg
   const long grid = (long)max_tiles * (g.slabs_gu + g.slabs_dn);
   if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
   const int threads = g.nw * 64;
-  if (split) {
-    // the down items with the combine; the caller launched gate/up (the
-    // same items, k_expert_lds) just before
-    const long gd = (long)max_tiles * g.slabs_dn;
-    if (scale_dtype == AINFER_SCALE_FP16)
-      k_experts_decode<AINFER_SCALE_FP16, 4, DEC_RG_GU, 2, DEC_RG_DN, true><<<(unsigned)gd, threads, g.lds, s>>>(a);
-    else
-      k_experts_decode<AINFER_SCALE_BF16, 4, DEC_RG_GU, 2, DEC_RG_DN, true><<<(unsigned)gd, threads, g.lds, s>>>(a);
-    return hipGetLastError();
-  }
   if (scale_dtype == AINFER_SCALE_FP16)
-    k_experts_decode<AINFER_SCALE_FP16, 4, DEC_RG_GU, 2, DEC_RG_DN, false><<<(unsigned)grid, threads, g.lds, s>>>(a);
+    k_experts_decode<AINFER_SCALE_FP16, 4, DEC_RG_GU, 2, DEC_RG_DN><<<(unsigned)grid, threads, g.lds, s>>>(a);
   else
-    k_experts_decode<AINFER_SCALE_BF16, 4, DEC_RG_GU, 2, DEC_RG_DN, false><<<(unsigned)grid, threads, g.lds, s>>>(a);
+    k_experts_decode<AINFER_SCALE_BF16, 4, DEC_RG_GU, 2, DEC_RG_DN><<<(unsigned)grid, threads, g.lds, s>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t launch_down_combine_t1(int scale_dtype, const ExpertArgs &dn, const float *w,
+                                  const float *sg, const int32_t *inv, const void *resid, void *y,
+                                  const int32_t *err, hipStream_t s) {
+  const int Kmax = dn.I > dn.Is ? dn.I : dn.Is;
+  // (k-groups in pairs: the scale dwords; decode_geometry holds both to it)
+  if (dn.T != 1 || dn.k > 32 || dn.H % DC_ROWS || dn.I % 256 || dn.Is % 256 || Kmax > 4096)
+    return hipErrorInvalidValue;
+  DownT1Args a;
+  memset(&a, 0, sizeof a);
+  a.dn = dn;
+  a.w = w;
+  a.sg = sg;
+  a.inv = inv;
+  a.resid = (const uint16_t *)resid;
+  a.y = (uint16_t *)y;
+  a.err = err;
+  a.n_tiles = dn.k + (dn.Is > 0 ? 1 : 0);
+  const int nw = a.n_tiles < 16 ? a.n_tiles : 16;
+  auto go = [&](auto sd_c, auto nh_c) {
+    constexpr int SDc = decltype(sd_c)::value, NHc = decltype(nh_c)::value;
+    k_down_combine_t1<SDc, NHc>
+        <<<dn.H / DC_ROWS, nw * 64, (size_t)nw * (NHc * 1024 + dc_scale_lds(NHc)), s>>>(a);
+  };
+  auto go_nh = [&](auto sd_c) {
+    if (Kmax <= 512) go(sd_c, std::integral_constant<int, 1>());
+    else if (Kmax <= 1024) go(sd_c, std::integral_constant<int, 2>());
+    else if (Kmax <= 2048) go(sd_c, std::integral_constant<int, 4>());
+    else go(sd_c, std::integral_constant<int, 8>());
+  };
+  if (scale_dtype == AINFER_SCALE_FP16)
+    go_nh(std::integral_constant<int, AINFER_SCALE_FP16>());
+  else
+    go_nh(std::integral_constant<int, AINFER_SCALE_BF16>());
   return hipGetLastError();
 }
 

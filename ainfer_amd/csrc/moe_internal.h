@@ -295,17 +295,18 @@ hipError_t launch_route_decode(const void *x, const void *rw, const float *bias,
                                const DispatchOut *ds, int32_t *sync, uint32_t *slots,
                                const NormIn *norm, hipStream_t s, int8_t *w8q = nullptr,
                                float *w8sq = nullptr);
-// gate/up + SiLU, down and the combine (y = sum_j w_j o_j + g_s o_s (+ resid));
-// split: gate/up in a launch of its own first (measured faster at T = 1,
-// where the down items of a fused launch wait behind the gate/up items for
-// workgroup slots: c3 39.5 -> 33.0 us, c1 equal)
-// (split: only the down items and the combine; the caller has launched the
-// gate/up items, k_expert_lds, just before)
+// gate/up + SiLU, down and the combine (y = sum_j w_j o_j + g_s o_s (+ resid))
+// in one launch
 hipError_t launch_experts_decode(int scale_dtype, const DecodeGeom &g, ExpertArgs gu,
                                  ExpertArgs dn, const float *w, const float *sg,
                                  const int32_t *inv, const void *resid, void *y,
-                                 int32_t *sync, int max_tiles, int cap, bool split,
-                                 hipStream_t s);
+                                 int32_t *sync, int max_tiles, int cap, hipStream_t s);
+// T = 1: down and the combine; the gate/up items (launch_expert_stream) ran
+// before (a fused launch's down items would wait behind the gate/up items for
+// workgroup slots: c3 39.5 -> 33.0 us)
+hipError_t launch_down_combine_t1(int scale_dtype, const ExpertArgs &dn, const float *w,
+                                  const float *sg, const int32_t *inv, const void *resid, void *y,
+                                  const int32_t *err, hipStream_t s);
 hipError_t launch_zero_i32(int32_t *p, int n, hipStream_t s);
 
 // k-groups per wave of the 4-token down items: whole 256-byte row segments
