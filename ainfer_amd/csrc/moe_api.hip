@@ -570,36 +570,32 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
                                 (uint32_t *)(sync + L.slots), norm, st));
     pc->end(2);
     ExpertArgs gu = expert_args(s, w, L, ws, d, T, 0), dn = expert_args(s, w, L, ws, d, T, 1);
-    if (T <= FUSED_EXPERTS_MAX_T) {
-      // latency-bound: gate/up, down and combine in one launch (T = 1: gate/up,
-      // then down with the combine)
-      if (T == 1) {
-        pc->kernel_events();
-        HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, max_tiles_bound(*s, T, DEC_MT), 4,
-                                     DEC_RG_GATE_UP, st));
-        pc->end(4);
-        HIP_TRY(launch_down_combine_t1(s->scale_dtype, dn, at<float>(ws, L.w), at<float>(ws, L.sg),
-                                       d.inv, resid, y, sync + SY_ERR, st));
-        pc->end(5);
-        return AINFER_OK;
-      }
+    const int mtb = max_tiles_bound(*s, T, DEC_MT);
+    const int kbw_dn = T <= FUSED_EXPERTS_MAX_T ? 2 : down_kbw(*s);
+    if (T == FUSED_EXPERTS_MAX_T && !down_combine_at(*s, T)) {
+      // latency-bound: gate/up, down and combine in one launch
       HIP_TRY(launch_experts_decode(s->scale_dtype, dg, gu, dn, at<float>(ws, L.w),
-                                    at<float>(ws, L.sg), d.inv, resid, y, sync,
-                                    max_tiles_bound(*s, T, DEC_MT),
+                                    at<float>(ws, L.sg), d.inv, resid, y, sync, mtb,
                                     max_tiles_bound(*s, DECODE_MAX_T, DEC_MT), st));
-    } else {
-      // bandwidth-bound: three launches whose items hold no waits
-      const int mtb = max_tiles_bound(*s, T, DEC_MT);
-      pc->kernel_events();
-      HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, mtb, 4, DEC_RG_GATE_UP, st));
-      pc->end(4);
-      HIP_TRY(launch_expert_stream(1, s->scale_dtype, dn, mtb, down_kbw(*s), DEC_RG_DOWN, st));
       pc->end(5);
-      HIP_TRY(combine(d, L));
-      pc->end(6);
       return AINFER_OK;
     }
+    pc->kernel_events();
+    HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, mtb, 4, DEC_RG_GATE_UP, st));
+    pc->end(4);
+    if (down_combine_at(*s, T)) {
+      int kbw, wk, wr;
+      if (!expert_geometry(1, H, s->inter, s->shared_inter, kbw_dn, &kbw, &wk, &wr))
+        return AINFER_ERR_SHAPE;
+      HIP_TRY(launch_down_combine(s->scale_dtype, dn, kbw, at<float>(ws, L.w),
+                                  at<float>(ws, L.sg), d.inv, resid, y, sync + SY_ERR, st));
+      pc->end(5);
+      return AINFER_OK;
+    }
+    HIP_TRY(launch_expert_stream(1, s->scale_dtype, dn, mtb, kbw_dn, DEC_RG_DOWN, st));
     pc->end(5);
+    HIP_TRY(combine(d, L));
+    pc->end(6);
     return AINFER_OK;
   }
   if (T <= EXACT_ROUTER_MAX_T)

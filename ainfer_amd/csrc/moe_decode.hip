@@ -469,137 +469,198 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
   }
 }
 
-// ---- T = 1: down and combine in one launch ---------------------------------
-// A workgroup owns DC_ROWS output rows of every selected expert: wave j takes
-// tile j (one expert; the shared one last), all waves' weight loads are in
-// flight together (c4: 512 workgroups x 11 waves x 4 KB, the whole 23 MB), the
-// tiles' rows meet in LDS and one lane per row sums them in slot order.  Items
-// of 32 rows of one expert that counted arrivals per row slab and combined on
-// the last took 11.8 us at H4096 I1024 k10 + shared (each waits for its sc1
-// stores, an atomic, and the last for a read of the others' rows).
-// The arithmetic is the decode item's at KBW = 2 (moe_expert_item.h), bit for
-// bit: per 32-wide chunk 8 MFMAs from -136 sum x and the group scale, the 8
-// chunks of two groups added as ((c, c+4), (c, c+2), (c, c+1)), then those
-// sums in k order.
-constexpr int DC_ROWS = 8;
-struct DownT1Args {
+// ---- T <= DC_MAX_T: down and combine in one launch -------------------------
+// A workgroup owns ROWS = 4 Q output rows of every selected expert: its waves
+// take the dispatch tiles in turn (a tile: one expert, all its tokens; the
+// shared one last), each with all its weight loads in flight, the tiles' rows
+// meet in LDS and one lane per (token, row) sums them in slot order.  Items of
+// 32 rows of one expert that counted arrivals per row slab and combined on the
+// last took 11.8 us at T = 1, H4096 I1024 k10 + shared (each waits for its sc1
+// stores, an atomic, and the last for a read of the others' rows); this form
+// 8.5 us.
+// With few tiles and a long K (KS > 1, T = 1) KS waves share a tile's K.
+// The arithmetic is the decode item's (moe_expert_item.h), bit for bit: per
+// 32-wide chunk 8 MFMAs from -136 sum x and the group scale; then at KBW = 2
+// (T <= 2) the 8 chunks of two groups added as ((c, c+4), (c, c+2), (c, c+1)),
+// at KBW = 4 the 16 chunks of four groups with (c, c+8) first; then those sums
+// in k order.
+struct DownArgs {
   ExpertArgs dn;
   const float *w, *sg;
   const int32_t *inv;
   const uint16_t *resid;
   uint16_t *y;
   const int32_t *err;
-  int n_tiles;  // k (+ 1)
+  int has_shared, ks, max_tiles;
 };
-constexpr int dc_scale_lds(int nh) { return nh > 4 ? 512 : 256; }
+constexpr int DC_WMAX = 8;  // tiles at KS > 1
 
-// NH: runs of 4 k-groups of the longer down product
-template <int SD, int NH>
-__global__ __launch_bounds__(1024) void k_down_combine_t1(DownT1Args a) {
-  __shared__ float s_o[33][DC_ROWS];
+constexpr int dc_scale_dma(int rpu, int rows) { return (rpu * rows * 2 + 63) / 64; }
+// LDS bytes per wave: the tile's token rows of the wave's K, then its scales
+constexpr int dc_wave_lds(int rpu, int rows, int mt) {
+  return mt * rpu * 1024 + dc_scale_dma(rpu, rows) * 256;
+}
+
+// RPU: runs of 4 k-groups per wave (of the longer product, over KS); MT: most
+// tokens of a tile
+template <int SD, int RPU, int Q, int KBW, int MT>
+__global__ __launch_bounds__(1024) void k_down_combine(DownArgs a) {
+  constexpr int ROWS = 4 * Q;
+  __shared__ float s_o[33 * MT][ROWS];
+  __shared__ float s_wt[32 * MT];
+  __shared__ int s_inv[32 * MT];
+  __shared__ float s_part[MT == 1 ? DC_WMAX : 1][16][ROWS];  // KS > 1
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int SCB = dc_scale_lds(NH), WB = NH * 1024 + SCB;  // LDS bytes per wave
+  constexpr int SCD = RPU * ROWS * 2, SCI = dc_scale_dma(RPU, ROWS);  // scale dwords, DMA instructions
+  constexpr int SCO = MT * RPU * 1024;  // the scales' offset in the wave's LDS
+  static_assert(MT == 1 || ROWS * MT <= 64, "wave 0 combines");
   const int tx = tid_opaque();
   const int wave = __builtin_amdgcn_readfirstlane(tx >> 6), lane = tx & 63;
-  const int nw = blockDim.x >> 6, k = a.dn.k, H = a.dn.H;
-  const int row0 = blockIdx.x * DC_ROWS;
-  // what the combine needs, requested before the weights (wave 0)
-  float wj = 0.f, rv = 0.f, sgv = 0.f;
+  const int nw = blockDim.x >> 6, k = a.dn.k, H = a.dn.H, T = a.dn.T, KS = MT == 1 ? a.ks : 1;
+  const int row0 = blockIdx.x * ROWS;
+  // what the combine needs, requested before the weights
+  const int ct = lane / ROWS, cr = lane % ROWS;  // wave 0: token and row of this lane
+  float rv = 0.f, sgv = 0.f, wj = 0.f;
   int pj = 0;
   bool bad = false;
+  if (tx < T * k) {
+    wj = a.w[tx];
+    pj = a.inv[tx];
+  }
   if (wave == 0) {
-    wj = a.w[min(lane, k - 1)];
-    pj = a.inv[min(lane, k - 1)];
-    sgv = a.sg[0];
-    if (a.resid) rv = bf16_to_f32(a.resid[row0 + (lane & (DC_ROWS - 1))]);
+    const int t = min(ct, T - 1);
+    sgv = a.sg[t];
+    if (a.resid) rv = bf16_to_f32(a.resid[(size_t)t * H + row0 + cr]);
     bad = *a.err != 0;
   }
   const int r4 = lane & 3, c = lane >> 2;
-  uint8_t *wl = lds + wave * WB;
+  uint8_t *wl = lds + wave * dc_wave_lds(RPU, ROWS, MT);
   const uint32_t wl32 = (uint32_t)(uintptr_t)wl;
-  for (int tile = wave; tile < a.n_tiles; tile += nw) {
-    const bool shared = tile == k;
-    int n_unused;
-    const int e = shared ? 0 : sload_tile(a.dn.tiles, a.dn.n_tiles, tile, n_unused).x;
+  int n_tiles = a.max_tiles;
+  for (int u = wave; u < n_tiles * KS; u += nw) {
+    const int tile = u / KS, part = u % KS;
+    const int4 t4 = sload_tile(a.dn.tiles, a.dn.n_tiles, tile, n_tiles);
+    if (tile >= n_tiles) break;
+    const int pos0 = t4.y, mcnt = t4.z;
+    const bool shared = t4.x == a.dn.E;
     const int K = shared ? a.dn.Is : a.dn.I, KB = K >> 7;
-    const uint8_t *w0 = shared ? a.dn.ws0 : a.dn.w0 + (size_t)e * H * (K / 2);
-    const uint16_t *s0 = shared ? a.dn.ss0 : a.dn.s0 + (size_t)e * H * KB;
-    const uint8_t *act = (const uint8_t *)(shared ? a.dn.a_shared : a.dn.a_routed + (size_t)tile * K);
+    const size_t e = shared ? 0 : (size_t)t4.x;
+    const uint8_t *w0 = shared ? a.dn.ws0 : a.dn.w0 + e * H * (K / 2);
+    const uint16_t *s0 = shared ? a.dn.ss0 : a.dn.s0 + e * H * KB;
+    const int h0 = part * RPU;  // first run of 4 groups
     // lane (r4, c): 32 nibbles of row r4 of a row quad at chunk 16 h + c
-    u32x4 B[NH][2];
+    u32x4 B[RPU][Q];
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      const int ch = min(16 * h + c, 4 * KB - 1);
+    for (int h = 0; h < RPU; ++h) {
+      const int ch = min(16 * (h0 + h) + c, 4 * KB - 1);
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
+      for (int q = 0; q < Q; ++q)
         B[h][q] = ldg_stream(w0 + (size_t)(row0 + 4 * q + r4) * (K / 2) + ch * 16);
     }
-    // scales: lane (h, row, pair) copies the dword of groups 4 h + 2 pair + {0, 1}
+    // scales: dword (h, row, pair) holds groups 4 h + 2 pair + {0, 1} of a row
 #pragma unroll
-    for (int i = 0; i < SCB / 256; ++i) {
-      const int pr = min(8 * i + 2 * (lane >> 4) + (lane & 1), KB / 2 - 1);
-      dma4(s0 + (size_t)(row0 + ((lane >> 1) & 7)) * KB + 2 * pr, wl32 + NH * 1024 + i * 256);
+    for (int i = 0; i < SCI; ++i) {
+      const int d = min(64 * i + lane, SCD - 1);
+      const int pr = min(2 * (h0 + d / (2 * ROWS)) + (d & 1), KB / 2 - 1);
+      dma4(s0 + (size_t)(row0 + ((d >> 1) % ROWS)) * KB + 2 * pr, wl32 + SCO + i * 256);
     }
+    // token rows in MFMA order: run h of row t at (t RPU + h) KB
+    const uint8_t *act = (const uint8_t *)((shared ? a.dn.a_shared : a.dn.a_routed) + (size_t)pos0 * K);
 #pragma unroll
-    for (int i = 0; i < NH; ++i)
-      if (i * 4 < KB) dma16(act + min(i * 1024 + lane * 16, K * 2 - 16), wl32 + i * 1024);
+    for (int t = 0; t < MT; ++t) {
+      if (t >= mcnt) break;
+#pragma unroll
+      for (int h = 0; h < RPU; ++h)
+        dma16(act + (size_t)t * K * 2 + min((h0 + h) * 1024 + lane * 16, K * 2 - 16),
+              wl32 + (t * RPU + h) * 1024);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     uint32_t magic;
-    asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
+    asm volatile("v_mov_b32 %0, 0x43084308" : "=v"(magic));
     const s16x4 ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
     const uint32_t mask = 0x000F000Fu;
-    const uint16_t *sl = (const uint16_t *)(wl + NH * 1024);
-    float gs[2] = {0.f, 0.f};
+    const uint16_t *sl = (const uint16_t *)(wl + SCO);
+    float gs[Q][MT];
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-      if (4 * h >= KB) break;
-      s16x4 A[8];
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
-      for (int jh = 0; jh < 8; ++jh) A[jh] = *(const s16x4 *)(wl + (16 * h + c) * 64 + jh * 8);
+      for (int t = 0; t < MT; ++t) gs[q][t] = 0.f;
+#pragma unroll
+    for (int h = 0; h < RPU; ++h) {
+      if (4 * (h0 + h) >= KB) break;
+      const uint8_t *xa = wl + ((MT == 1 ? 0 : min(r4, mcnt - 1)) * RPU + h) * 1024 + c * 64;
+      s16x4 av[8];
+#pragma unroll
+      for (int jh = 0; jh < 8; ++jh) av[jh] = *(const s16x4 *)(xa + jh * 8);
       f32x4 xs = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int jh = 0; jh < 8; ++jh) xs = mfma_bf16_4x4x4(A[jh], ones, xs);
+      for (int jh = 0; jh < 8; ++jh) xs = mfma_bf16_4x4x4(av[jh], ones, xs);
       const f32x4 c0 = xs * -136.0f;
-      const bool in = 16 * h + c < 4 * KB;
+      const bool in = 16 * (h0 + h) + c < 4 * KB;
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const u32x4 bw = B[h][q] ^ 0x88888888u;
+      for (int q = 0; q < Q; ++q) {
         f32x4 acc = c0;
 #pragma unroll
         for (int jh = 0; jh < 8; ++jh) {
           const int j = jh >> 1, hf = jh & 1;
-          const uint32_t d0 = ((bw[2 * hf] >> (4 * j)) & mask) | magic;
-          const uint32_t d1 = ((bw[2 * hf + 1] >> (4 * j)) & mask) | magic;
-          acc = mfma_bf16_4x4x4(A[jh], __builtin_bit_cast(s16x4, u32x2{d0, d1}), acc);
+          const uint32_t d0 = ((B[h][q][2 * hf] >> (4 * j)) & mask) ^ magic;
+          const uint32_t d1 = ((B[h][q][2 * hf + 1] >> (4 * j)) & mask) ^ magic;
+          acc = mfma_bf16_4x4x4(av[jh], __builtin_bit_cast(s16x4, u32x2{d0, d1}), acc);
         }
-        // dword (h, row, pair) at 16 h + 2 row + pair; the group's half of it
-        const float sc = scale_to_f32<SD>(sl[2 * (16 * h + 2 * (4 * q + r4) + (c >> 3)) + ((c >> 2) & 1)]);
-        float v = in ? acc[0] * sc : 0.f;
-        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (16 << 10) | 0x1F));
-        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (8 << 10) | 0x1F));
-        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (4 << 10) | 0x1F));
-        // lanes 0-31 hold groups 4 h, 4 h + 1; lanes 32-63 the next two
-        gs[q] += v;
-        gs[q] += __shfl_xor(v, 32, 64);
+        const float sc = scale_to_f32<SD>(sl[2 * (2 * ROWS * h + 2 * (4 * q + r4) + (c >> 3)) + ((c >> 2) & 1)]);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          if (t >= mcnt) break;
+          float v = in ? acc[t] * sc : 0.f;
+          if (KBW == 4) v += __shfl_xor(v, 32, 64);
+          v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (16 << 10) | 0x1F));
+          v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (8 << 10) | 0x1F));
+          v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (4 << 10) | 0x1F));
+          if (KBW == 4) {
+            gs[q][t] += v;
+          } else if (MT == 1 && KS > 1) {
+            // lanes 0-31 hold groups 4 h, 4 h + 1; lanes 32-63 the next two
+            if ((c & 7) == 0) s_part[tile][2 * (h0 + h) + (c >> 3)][4 * q + r4] = v;
+          } else {
+            gs[q][t] += v;
+            gs[q][t] += __shfl_xor(v, 32, 64);
+          }
+        }
       }
     }
-    if (lane < 4) {
-      s_o[tile][r4] = bf16_to_f32(f32_to_bf16(gs[0]));
-      s_o[tile][4 + r4] = bf16_to_f32(f32_to_bf16(gs[1]));
+    if (lane < 4 && KS == 1) {
+      const int o0 = (shared ? T * k : 0) + pos0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          if (t < mcnt) s_o[o0 + t][4 * q + r4] = bf16_to_f32(f32_to_bf16(gs[q][t]));
     }
+    // this tile's LDS reads are done before the next tile's copies land there
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  if (tx < T * k) {
+    s_wt[tx] = wj;
+    s_inv[tx] = pj;
   }
   __syncthreads();
-  if (wave != 0) return;
-  // ---- the combine, slot order (k_combine's arithmetic) ----------------------
-  const int r = lane & (DC_ROWS - 1);
-  float acc = 0.f;
-  for (int j = 0; j < k; ++j) {
-    const int p = __builtin_amdgcn_readlane(pj, j);
-    acc = __builtin_fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wj), j)), s_o[p][r], acc);
+  if (MT == 1 && KS > 1) {  // T = 1: tile j's row is o row j (k: the shared one)
+    const int nt = k + a.has_shared;
+    for (int i = tx; i < nt * ROWS; i += blockDim.x) {
+      const int tile = i / ROWS, r = i % ROWS, n = (tile == k ? a.dn.Is : a.dn.I) >> 8;
+      float g = 0.f;
+      for (int j = 0; j < n; ++j) g += s_part[tile][j][r];
+      s_o[tile][r] = bf16_to_f32(f32_to_bf16(g));
+    }
+    __syncthreads();
   }
-  if (a.n_tiles > k) acc = __builtin_fmaf(sgv, s_o[k][r], acc);
+  if (wave != 0 || ct >= T) return;
+  // ---- the combine, slot order (k_combine's arithmetic) ----------------------
+  float acc = 0.f;
+  for (int j = 0; j < k; ++j) acc = __builtin_fmaf(s_wt[ct * k + j], s_o[s_inv[ct * k + j]][cr], acc);
+  if (a.has_shared) acc = __builtin_fmaf(sgv, s_o[T * k + ct][cr], acc);
   if (a.resid) acc += rv;
-  if (lane < DC_ROWS) a.y[row0 + lane] = bad ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
+  a.y[(size_t)ct * H + row0 + cr] = bad ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
 }
 
 }  // namespace
@@ -726,14 +787,16 @@ hipError_t launch_experts_decode(int scale_dtype, const DecodeGeom &g, ExpertArg
   return hipGetLastError();
 }
 
-hipError_t launch_down_combine_t1(int scale_dtype, const ExpertArgs &dn, const float *w,
-                                  const float *sg, const int32_t *inv, const void *resid, void *y,
-                                  const int32_t *err, hipStream_t s) {
-  const int Kmax = dn.I > dn.Is ? dn.I : dn.Is;
-  // (k-groups in pairs: the scale dwords; decode_geometry holds both to it)
-  if (dn.T != 1 || dn.k > 32 || dn.H % DC_ROWS || dn.I % 256 || dn.Is % 256 || Kmax > 4096)
+hipError_t launch_down_combine(int scale_dtype, const ExpertArgs &dn, int kbw, const float *w,
+                               const float *sg, const int32_t *inv, const void *resid, void *y,
+                               const int32_t *err, hipStream_t s) {
+  const int Kmax = dn.I > dn.Is ? dn.I : dn.Is, has_shared = dn.Is > 0 ? 1 : 0;
+  // (k-groups in whole waves of the item's split; decode_geometry holds both to it)
+  if (dn.T < 1 || dn.T > DC_MAX_T || dn.k > 32 || dn.H % 128 ||
+      (kbw != 2 && (kbw != 4 || dn.T == 1)) ||
+      dn.I % (128 * kbw) || dn.Is % (128 * kbw) || Kmax > 4096)
     return hipErrorInvalidValue;
-  DownT1Args a;
+  DownArgs a;
   memset(&a, 0, sizeof a);
   a.dn = dn;
   a.w = w;
@@ -742,23 +805,53 @@ hipError_t launch_down_combine_t1(int scale_dtype, const ExpertArgs &dn, const f
   a.resid = (const uint16_t *)resid;
   a.y = (uint16_t *)y;
   a.err = err;
-  a.n_tiles = dn.k + (dn.Is > 0 ? 1 : 0);
-  const int nw = a.n_tiles < 16 ? a.n_tiles : 16;
-  auto go = [&](auto sd_c, auto nh_c) {
-    constexpr int SDc = decltype(sd_c)::value, NHc = decltype(nh_c)::value;
-    k_down_combine_t1<SDc, NHc>
-        <<<dn.H / DC_ROWS, nw * 64, (size_t)nw * (NHc * 1024 + dc_scale_lds(NHc)), s>>>(a);
+  a.has_shared = has_shared;
+  const int tiles = a.max_tiles = dn.T * dn.k + has_shared;  // at most
+  int rpu = 1;
+  while (512 * rpu < Kmax) rpu *= 2;
+  // few tiles: KS waves share a tile's K
+  a.ks = 1;
+  while (dn.T == 1 && kbw == 2 && rpu > 1 && tiles <= DC_WMAX && tiles * a.ks * 2 <= 16) {
+    a.ks *= 2;
+    rpu /= 2;
+  }
+  if (dn.T > 1 && rpu > 2) return hipErrorInvalidValue;  // down_combine_at
+  const int nw = tiles * a.ks < 16 ? tiles * a.ks : 16;
+  using std::integral_constant;
+  auto go = [&](auto sd_c, auto rpu_c, auto q_c, auto kbw_c, auto mt_c) {
+    constexpr int SDc = decltype(sd_c)::value, R = decltype(rpu_c)::value,
+                  Qc = decltype(q_c)::value, KW = decltype(kbw_c)::value,
+                  M = decltype(mt_c)::value;
+    k_down_combine<SDc, R, Qc, KW, M>
+        <<<dn.H / (4 * Qc), nw * 64, (size_t)nw * dc_wave_lds(R, 4 * Qc, M), s>>>(a);
   };
-  auto go_nh = [&](auto sd_c) {
-    if (Kmax <= 512) go(sd_c, std::integral_constant<int, 1>());
-    else if (Kmax <= 1024) go(sd_c, std::integral_constant<int, 2>());
-    else if (Kmax <= 2048) go(sd_c, std::integral_constant<int, 4>());
-    else go(sd_c, std::integral_constant<int, 8>());
+  // T > 1: 16 rows per workgroup where that still gives every CU one
+  const bool wide = dn.H >= 16 * 256;
+  auto go_t = [&](auto sd_c, auto rpu_c, auto kbw_c) {
+    if (wide)
+      go(sd_c, rpu_c, integral_constant<int, 4>(), kbw_c, integral_constant<int, 4>());
+    else
+      go(sd_c, rpu_c, integral_constant<int, 2>(), kbw_c, integral_constant<int, 4>());
+  };
+  auto go_r = [&](auto sd_c, auto kbw_c) {
+    if (rpu == 1) go_t(sd_c, integral_constant<int, 1>(), kbw_c);
+    else go_t(sd_c, integral_constant<int, 2>(), kbw_c);
+  };
+  auto go_k = [&](auto sd_c) {
+    using two = integral_constant<int, 2>;
+    using one = integral_constant<int, 1>;
+    if (dn.T > 1) {
+      if (kbw == 2) go_r(sd_c, two());
+      else go_r(sd_c, integral_constant<int, 4>());
+    } else if (rpu == 1) go(sd_c, one(), two(), two(), one());
+    else if (rpu == 2) go(sd_c, two(), two(), two(), one());
+    else if (rpu == 4) go(sd_c, integral_constant<int, 4>(), two(), two(), one());
+    else go(sd_c, integral_constant<int, 8>(), two(), two(), one());
   };
   if (scale_dtype == AINFER_SCALE_FP16)
-    go_nh(std::integral_constant<int, AINFER_SCALE_FP16>());
+    go_k(integral_constant<int, AINFER_SCALE_FP16>());
   else
-    go_nh(std::integral_constant<int, AINFER_SCALE_BF16>());
+    go_k(integral_constant<int, AINFER_SCALE_BF16>());
   return hipGetLastError();
 }
 

@@ -301,12 +301,17 @@ hipError_t launch_experts_decode(int scale_dtype, const DecodeGeom &g, ExpertArg
                                  ExpertArgs dn, const float *w, const float *sg,
                                  const int32_t *inv, const void *resid, void *y,
                                  int32_t *sync, int max_tiles, int cap, hipStream_t s);
-// T = 1: down and the combine; the gate/up items (launch_expert_stream) ran
-// before (a fused launch's down items would wait behind the gate/up items for
-// workgroup slots: c3 39.5 -> 33.0 us)
-hipError_t launch_down_combine_t1(int scale_dtype, const ExpertArgs &dn, const float *w,
-                                  const float *sg, const int32_t *inv, const void *resid, void *y,
-                                  const int32_t *err, hipStream_t s);
+// T <= DC_MAX_T: down and the combine; the gate/up items (launch_expert_stream)
+// ran before.  kbw: the k-groups whose sums a wave of the down items adds (the
+// order of the additions, as launch_expert_stream's at the same T).
+constexpr int DC_MAX_T = 4;
+// beyond one token a wave's LDS holds the token rows of up to 1024 columns
+inline bool down_combine_at(const ainfer_moe_shape &s, int T) {
+  return T == 1 || (T <= DC_MAX_T && s.inter <= 1024 && s.shared_inter <= 1024);
+}
+hipError_t launch_down_combine(int scale_dtype, const ExpertArgs &dn, int kbw, const float *w,
+                               const float *sg, const int32_t *inv, const void *resid, void *y,
+                               const int32_t *err, hipStream_t s);
 hipError_t launch_zero_i32(int32_t *p, int n, hipStream_t s);
 
 // k-groups per wave of the 4-token down items: whole 256-byte row segments
