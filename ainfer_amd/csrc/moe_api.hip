@@ -232,7 +232,7 @@ DispatchOut dispatch_out(const ainfer_moe_shape *s, const Layout &L, void *ws, i
   d.tiles = at<int4>(ws, L.tiles);
   d.n_tiles = at<int32_t>(ws, L.n_tiles);
   d.ticket = at<int32_t>(ws, L.ticket);
-  d.mt = SMALL_MT;
+  d.mt = DEC_MT;
   return d;
 }
 
@@ -555,8 +555,8 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
   DispatchOut d = dispatch_out(s, L, ws, T);
   d.mt = mt;
   DecodeGeom dg;
-  if (T <= DECODE_MAX_T && decode_geometry(*s, &dg)) {
-    // decode: two launches (moe_decode.hip)
+  if (T <= DECODE_MAX_T) {
+    // decode: the routing kernel, then two or three expert launches
     int32_t *sync = at<int32_t>(ws, L.sync);
     // the expert kernels read the tiles and positions only: no per-expert
     // counts or offsets on this path
@@ -572,7 +572,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
     ExpertArgs gu = expert_args(s, w, L, ws, d, T, 0), dn = expert_args(s, w, L, ws, d, T, 1);
     const int mtb = max_tiles_bound(*s, T, DEC_MT);
     const int kbw_dn = T <= FUSED_EXPERTS_MAX_T ? 2 : down_kbw(*s);
-    if (T == FUSED_EXPERTS_MAX_T && !down_combine_at(*s, T)) {
+    if (T == FUSED_EXPERTS_MAX_T && !down_combine_at(*s, T) && decode_geometry(*s, &dg)) {
       // latency-bound: gate/up, down and combine in one launch
       HIP_TRY(launch_experts_decode(s->scale_dtype, dg, gu, dn, at<float>(ws, L.w),
                                     at<float>(ws, L.sg), d.inv, resid, y, sync, mtb,
@@ -598,18 +598,11 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
     pc->end(6);
     return AINFER_OK;
   }
-  if (T <= EXACT_ROUTER_MAX_T)
-    HIP_TRY(launch_router_exact(x, w->router_w, w->router_bias, w->shared_gate_w,
-                                at<float>(ws, L.logits), at<float>(ws, L.sg_logit),
-                                at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
-                                at<uint16_t>(ws, L.xperm), T, H, E, k, has_shared,
-                                fused ? &d : nullptr, st));
   // prefill (T >= GEMM_MIN_T, unfused dispatch): the selection builds the
   // dispatch's per-chunk token masks itself, so the dispatch needs no counting launch
   unsigned long long *cmask =
       T >= GEMM_MIN_T ? at<unsigned long long>(ws, L.chunk_masks) : nullptr;
-  if (T > EXACT_ROUTER_MAX_T)
-    HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
+  HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
                                at<float>(ws, L.logits), at<float>(ws, L.wnorm),
                                at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
                                at<uint16_t>(ws, L.xperm), gemm ? at<float>(ws, L.xsum) : nullptr,
@@ -648,9 +641,7 @@ int do_block(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void 
   void *h = at<void>(ws, L.h);
   ProfCall pc(st);
   pc.start();
-  DecodeGeom dg;
-  if (T <= DECODE_NORM_MAX_T && s->n_experts <= 1024 &&
-      (s->precision == AINFER_PRECISION_W4A8 || decode_geometry(*s, &dg))) {
+  if (T <= DECODE_NORM_MAX_T) {
     // decode at up to 4 tokens: the routing kernel normalizes x itself (one
     // launch fewer per block: c4 T=1 about 2470 -> 2235 us per 60-block
     // step); the values are those k_rmsnorm writes
@@ -704,8 +695,7 @@ int do_route(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void 
              int32_t *topk_idx, float *topk_w, float *shared_gate, float *logits, void *ws,
              hipStream_t st) {
   const Layout L = layout_of(*s, T);
-  DecodeGeom dg;
-  if (T <= DECODE_MAX_T && decode_geometry(*s, &dg)) {
+  if (T <= DECODE_MAX_T) {
     // the decode routing kernel, without its dispatch
     HIP_TRY(launch_route_decode(x, w->router_w, w->router_bias, w->shared_gate_w,
                                 logits ? logits : at<float>(ws, L.logits),
@@ -713,14 +703,6 @@ int do_route(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void 
                                 T, s->hidden, s->n_experts, s->top_k, s->shared_inter > 0,
                                 nullptr, at<int32_t>(ws, L.sync),
                                 at<uint32_t>(ws, L.sync) + L.slots, nullptr, st));
-    return AINFER_OK;
-  }
-  if (T <= EXACT_ROUTER_MAX_T) {
-    HIP_TRY(launch_router_exact(x, w->router_w, w->router_bias, w->shared_gate_w,
-                                logits ? logits : at<float>(ws, L.logits),
-                                at<float>(ws, L.sg_logit), topk_idx, topk_w, shared_gate, nullptr,
-                                T, s->hidden, s->n_experts, s->top_k, s->shared_inter > 0,
-                                nullptr, st));
     return AINFER_OK;
   }
   HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
@@ -965,9 +947,7 @@ int check_stack_args(const ainfer_moe_shape *s, const void *table, int32_t n_lay
 int do_stack(const ainfer_moe_shape *s, const std::vector<StackLayer> &ly, int n_layers,
              int norm_mode, float eps, const void *resid_in, void *resid_out, int T, void *ws,
              hipStream_t st) {
-  DecodeGeom dg;
-  const bool folded = T <= DECODE_NORM_MAX_T && s->n_experts <= 1024 &&
-                      (s->precision == AINFER_PRECISION_W4A8 || decode_geometry(*s, &dg));
+  const bool folded = T <= DECODE_NORM_MAX_T;
   if (folded || s->precision == AINFER_PRECISION_W4A8) {
     for (int l = 0; l < n_layers; ++l) {
       int rc = do_block(s, &ly[l].w, ly[l].norm_w, norm_mode, eps, l ? resid_out : resid_in,
@@ -1126,7 +1106,7 @@ int ainfer_moe_dispatch(const ainfer_moe_shape *s, const int32_t *topk_idx, int3
   d.offsets = offsets;
   d.perm = perm;
   d.inv = inv_perm;
-  HIP_TRY(launch_dispatch(topk_idx, T, s->top_k, s->n_experts, SMALL_MT, s->shared_inter > 0,
+  HIP_TRY(launch_dispatch(topk_idx, T, s->top_k, s->n_experts, DEC_MT, s->shared_inter > 0,
                           at<int32_t>(ws, L.chunk_counts), at<int32_t>(ws, L.rank), d,
                           (hipStream_t)stream));
   return AINFER_OK;

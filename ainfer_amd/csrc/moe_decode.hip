@@ -184,7 +184,9 @@ __global__ __launch_bounds__(W * 64) void k_route_decode(RouteDecodeArgs a) {
         for (int j = 0; j < RD_TT; ++j) acc[i][j] = 0.0f;
       // NB chunks' loads in flight at once; the sums still run over
       // chunks l, l + 64, ... in order
-      for (int cb = lane; cb < nch; cb += 64 * NB) {
+      // (every lane takes part, H < 512 included: the RMSNorm's wave reductions
+      // read all 64)
+      for (int cb = lane; cb - lane < nch; cb += 64 * NB) {
         u32x4 wv[NB][RD_R], xv[NB][RD_TT], nv[NB];
         // x and the norm weight first: loads complete in issue order, so the
         // RMSNorm (which needs only them) runs while the router row, a cold
@@ -482,8 +484,8 @@ __global__ __launch_bounds__(1024, DEC_WAVES_PER_SIMD) void k_experts_decode(Exp
 // The arithmetic is the decode item's (moe_expert_item.h), bit for bit: per
 // 32-wide chunk 8 MFMAs from -136 sum x and the group scale; then at KBW = 2
 // (T <= 2) the 8 chunks of two groups added as ((c, c+4), (c, c+2), (c, c+1)),
-// at KBW = 4 the 16 chunks of four groups with (c, c+8) first; then those sums
-// in k order.
+// at KBW = 4 the 16 chunks of four groups with (c, c+8) first, at KBW = 1 (an odd
+// number of groups) the 4 of one; then those sums in k order.
 struct DownArgs {
   ExpertArgs dn;
   const float *w, *sg;
@@ -495,10 +497,12 @@ struct DownArgs {
 };
 constexpr int DC_WMAX = 8;  // tiles at KS > 1
 
-constexpr int dc_scale_dma(int rpu, int rows) { return (rpu * rows * 2 + 63) / 64; }
+// scale dwords of a run's row: one per pair of groups, or (KBW = 1, where a
+// row's pairs may straddle dwords) the dword holding each group's scale
+constexpr int dc_scale_dma(int rpu, int rows, int kbw) { return (rpu * rows * (kbw == 1 ? 4 : 2) + 63) / 64; }
 // LDS bytes per wave: the tile's token rows of the wave's K, then its scales
-constexpr int dc_wave_lds(int rpu, int rows, int mt) {
-  return mt * rpu * 1024 + dc_scale_dma(rpu, rows) * 256;
+constexpr int dc_wave_lds(int rpu, int rows, int mt, int kbw) {
+  return mt * rpu * 1024 + dc_scale_dma(rpu, rows, kbw) * 256;
 }
 
 // RPU: runs of 4 k-groups per wave (of the longer product, over KS); MT: most
@@ -509,14 +513,15 @@ __global__ __launch_bounds__(1024) void k_down_combine(DownArgs a) {
   __shared__ float s_o[33 * MT][ROWS];
   __shared__ float s_wt[32 * MT];
   __shared__ int s_inv[32 * MT];
-  __shared__ float s_part[MT == 1 ? DC_WMAX : 1][16][ROWS];  // KS > 1
+  __shared__ float s_part[MT == 1 && KBW == 2 ? DC_WMAX : 1][16][ROWS];  // KS > 1
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  constexpr int SCD = RPU * ROWS * 2, SCI = dc_scale_dma(RPU, ROWS);  // scale dwords, DMA instructions
+  constexpr int DPR = KBW == 1 ? 4 : 2;  // scale dwords per run and row
+  constexpr int SCD = RPU * ROWS * DPR, SCI = dc_scale_dma(RPU, ROWS, KBW);
   constexpr int SCO = MT * RPU * 1024;  // the scales' offset in the wave's LDS
   static_assert(MT == 1 || ROWS * MT <= 64, "wave 0 combines");
   const int tx = tid_opaque();
   const int wave = __builtin_amdgcn_readfirstlane(tx >> 6), lane = tx & 63;
-  const int nw = blockDim.x >> 6, k = a.dn.k, H = a.dn.H, T = a.dn.T, KS = MT == 1 ? a.ks : 1;
+  const int nw = blockDim.x >> 6, k = a.dn.k, H = a.dn.H, T = a.dn.T, KS = MT == 1 && KBW == 2 ? a.ks : 1;
   const int row0 = blockIdx.x * ROWS;
   // what the combine needs, requested before the weights
   const int ct = lane / ROWS, cr = lane % ROWS;  // wave 0: token and row of this lane
@@ -534,7 +539,7 @@ __global__ __launch_bounds__(1024) void k_down_combine(DownArgs a) {
     bad = *a.err != 0;
   }
   const int r4 = lane & 3, c = lane >> 2;
-  uint8_t *wl = lds + wave * dc_wave_lds(RPU, ROWS, MT);
+  uint8_t *wl = lds + wave * dc_wave_lds(RPU, ROWS, MT, KBW);
   const uint32_t wl32 = (uint32_t)(uintptr_t)wl;
   int n_tiles = a.max_tiles;
   for (int u = wave; u < n_tiles * KS; u += nw) {
@@ -557,12 +562,14 @@ __global__ __launch_bounds__(1024) void k_down_combine(DownArgs a) {
       for (int q = 0; q < Q; ++q)
         B[h][q] = ldg_stream(w0 + (size_t)(row0 + 4 * q + r4) * (K / 2) + ch * 16);
     }
-    // scales: dword (h, row, pair) holds groups 4 h + 2 pair + {0, 1} of a row
+    // scales: dword (h, row, i) of DPR per row (KBW = 1: the aligned dword of
+    // group 4 h + i; H rows are an even number, so it never ends past them)
 #pragma unroll
     for (int i = 0; i < SCI; ++i) {
       const int d = min(64 * i + lane, SCD - 1);
-      const int pr = min(2 * (h0 + d / (2 * ROWS)) + (d & 1), KB / 2 - 1);
-      dma4(s0 + (size_t)(row0 + ((d >> 1) % ROWS)) * KB + 2 * pr, wl32 + SCO + i * 256);
+      const int gi = DPR * (h0 + d / (DPR * ROWS)) + d % DPR, row = row0 + (d / DPR) % ROWS;
+      const size_t at = (size_t)row * KB + (KBW == 1 ? min(gi, KB - 1) : 2 * min(gi, KB / 2 - 1));
+      dma4(s0 + (at & ~(size_t)1), wl32 + SCO + i * 256);
     }
     // token rows in MFMA order: run h of row t at (t RPU + h) KB
     const uint8_t *act = (const uint8_t *)((shared ? a.dn.a_shared : a.dn.a_routed) + (size_t)pos0 * K);
@@ -607,18 +614,25 @@ __global__ __launch_bounds__(1024) void k_down_combine(DownArgs a) {
           const uint32_t d1 = ((B[h][q][2 * hf + 1] >> (4 * j)) & mask) ^ magic;
           acc = mfma_bf16_4x4x4(av[jh], __builtin_bit_cast(s16x4, u32x2{d0, d1}), acc);
         }
-        const float sc = scale_to_f32<SD>(sl[2 * (2 * ROWS * h + 2 * (4 * q + r4) + (c >> 3)) + ((c >> 2) & 1)]);
+        const int sr = ROWS * h + 4 * q + r4, gr = c >> 2;
+        const float sc = scale_to_f32<SD>(
+            KBW == 1 ? sl[2 * (4 * sr + gr) + (((row0 + 4 * q + r4) * KB + 4 * (h0 + h) + gr) & 1)]
+                     : sl[2 * (2 * sr + (gr >> 1)) + (gr & 1)]);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
           if (t >= mcnt) break;
           float v = in ? acc[t] * sc : 0.f;
           if (KBW == 4) v += __shfl_xor(v, 32, 64);
-          v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (16 << 10) | 0x1F));
+          if (KBW > 1) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (16 << 10) | 0x1F));
           v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (8 << 10) | 0x1F));
           v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (4 << 10) | 0x1F));
           if (KBW == 4) {
             gs[q][t] += v;
-          } else if (MT == 1 && KS > 1) {
+          } else if (KBW == 1) {
+            // group 4 h + i's sum in the lanes of chunk 4 i
+#pragma unroll
+            for (int i = 0; i < 4; ++i) gs[q][t] += __shfl(v, 16 * i + r4, 64);
+          } else if (MT == 1 && KBW == 2 && KS > 1) {
             // lanes 0-31 hold groups 4 h, 4 h + 1; lanes 32-63 the next two
             if ((c & 7) == 0) s_part[tile][2 * (h0 + h) + (c >> 3)][4 * q + r4] = v;
           } else {
@@ -644,7 +658,7 @@ __global__ __launch_bounds__(1024) void k_down_combine(DownArgs a) {
     s_inv[tx] = pj;
   }
   __syncthreads();
-  if (MT == 1 && KS > 1) {  // T = 1: tile j's row is o row j (k: the shared one)
+  if (MT == 1 && KBW == 2 && KS > 1) {  // T = 1: tile j's row is o row j (k: the shared one)
     const int nt = k + a.has_shared;
     for (int i = tx; i < nt * ROWS; i += blockDim.x) {
       const int tile = i / ROWS, r = i % ROWS, n = (tile == k ? a.dn.Is : a.dn.I) >> 8;
@@ -791,9 +805,9 @@ hipError_t launch_down_combine(int scale_dtype, const ExpertArgs &dn, int kbw, c
                                const float *sg, const int32_t *inv, const void *resid, void *y,
                                const int32_t *err, hipStream_t s) {
   const int Kmax = dn.I > dn.Is ? dn.I : dn.Is, has_shared = dn.Is > 0 ? 1 : 0;
-  // (k-groups in whole waves of the item's split; decode_geometry holds both to it)
+  // (k-groups in whole waves of the item's split)
   if (dn.T < 1 || dn.T > DC_MAX_T || dn.k > 32 || dn.H % 128 ||
-      (kbw != 2 && (kbw != 4 || dn.T == 1)) ||
+      (kbw != 1 && kbw != 2 && (kbw != 4 || dn.T == 1)) ||
       dn.I % (128 * kbw) || dn.Is % (128 * kbw) || Kmax > 4096)
     return hipErrorInvalidValue;
   DownArgs a;
@@ -823,7 +837,7 @@ hipError_t launch_down_combine(int scale_dtype, const ExpertArgs &dn, int kbw, c
                   Qc = decltype(q_c)::value, KW = decltype(kbw_c)::value,
                   M = decltype(mt_c)::value;
     k_down_combine<SDc, R, Qc, KW, M>
-        <<<dn.H / (4 * Qc), nw * 64, (size_t)nw * dc_wave_lds(R, 4 * Qc, M), s>>>(a);
+        <<<dn.H / (4 * Qc), nw * 64, (size_t)nw * dc_wave_lds(R, 4 * Qc, M, KW), s>>>(a);
   };
   // T > 1: 16 rows per workgroup where that still gives every CU one
   const bool wide = dn.H >= 16 * 256;
@@ -837,16 +851,23 @@ hipError_t launch_down_combine(int scale_dtype, const ExpertArgs &dn, int kbw, c
     if (rpu == 1) go_t(sd_c, integral_constant<int, 1>(), kbw_c);
     else go_t(sd_c, integral_constant<int, 2>(), kbw_c);
   };
+  auto go_1 = [&](auto sd_c, auto kbw_c) {
+    using two = integral_constant<int, 2>;
+    using one = integral_constant<int, 1>;
+    if (rpu == 1) go(sd_c, one(), two(), kbw_c, one());
+    else if (rpu == 2) go(sd_c, two(), two(), kbw_c, one());
+    else if (rpu == 4) go(sd_c, integral_constant<int, 4>(), two(), kbw_c, one());
+    else go(sd_c, integral_constant<int, 8>(), two(), kbw_c, one());
+  };
   auto go_k = [&](auto sd_c) {
     using two = integral_constant<int, 2>;
     using one = integral_constant<int, 1>;
     if (dn.T > 1) {
-      if (kbw == 2) go_r(sd_c, two());
+      if (kbw == 1) go_r(sd_c, one());
+      else if (kbw == 2) go_r(sd_c, two());
       else go_r(sd_c, integral_constant<int, 4>());
-    } else if (rpu == 1) go(sd_c, one(), two(), two(), one());
-    else if (rpu == 2) go(sd_c, two(), two(), two(), one());
-    else if (rpu == 4) go(sd_c, integral_constant<int, 4>(), two(), two(), one());
-    else go(sd_c, integral_constant<int, 8>(), two(), two(), one());
+    } else if (kbw == 1) go_1(sd_c, one());
+    else go_1(sd_c, two());
   };
   if (scale_dtype == AINFER_SCALE_FP16)
     go_k(integral_constant<int, AINFER_SCALE_FP16>());

@@ -116,7 +116,6 @@ __device__ __forceinline__ void expert_lds_item(const ExpertArgs &a, int4 t, int
   const int wave = __builtin_amdgcn_readfirstlane(tx >> 6);
   const int lane = tx & 63;
   const int kw = wave % a.WK, wr = wave / a.WK;
-  const int m = lane & 15, q = lane >> 4;
   const int n0 = (slab * a.WR + wr) * RG * 16;
   const bool act = n0 < N && kw * KBW < KB;
   const int kb0 = act ? kw * KBW : 0;

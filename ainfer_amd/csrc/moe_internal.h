@@ -148,14 +148,6 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
                               int has_shared, const DispatchOut *fused, hipStream_t s,
                               int32_t *ccount = nullptr, unsigned long long *cmask = nullptr,
                               W8Rows w8 = W8Rows());
-// Small T: canonical logits of all experts on VALU (k_router_logits), then the
-// same selection without the refine.  logits [T][E], sg_logit [T] out.
-hipError_t launch_router_exact(const void *x, const void *rw, const float *bias, const void *gw,
-                               float *logits, float *sg_logit, int32_t *idx, float *w, float *sg,
-                               void *xperm, int T, int H, int E, int k, int has_shared,
-                               const DispatchOut *fused, hipStream_t s);
-// below this many tokens the router computes every logit in the canonical order
-constexpr int EXACT_ROUTER_MAX_T = 16;
 // cmask non-null: the per-(64-token chunk, expert) token masks (and, in
 // chunk_counts, the counts) the router's k_select already built
 // (T >= GEMM_MIN_T), so no counting launch
@@ -212,8 +204,6 @@ void set_expert_launch_events(hipEvent_t start, hipEvent_t stop);
 hipError_t launch_expert_stream(int mode, int scale_dtype, ExpertArgs a, int max_tiles,
                                 int pref_kbw, int rg, hipStream_t s);
 
-// most tokens the small selection (k_select_small) takes
-constexpr int SMALL_MT = 16;
 // LDS bytes per wave of a decode expert item (moe_expert_item.h): its A
 // rows (MT x KBW * 256 B), its scales (KBW >= 2: one dword DMA per 256 B),
 // and its K-split partials where they do not fit the A rows.
@@ -224,13 +214,15 @@ __host__ __device__ constexpr int item_lds_per_wave(int mt, int kbw, int rg, int
   return mt * kbw * 256 + item_scale_lds(kbw, rg, mode) +
          (mt * kbw * 256 >= (mode == 0 ? 2 : 1) * rg * 1024 ? 0 : (mode == 0 ? 2 : 1) * rg * 1024);
 }
-constexpr int DEC_MT = 4;  // tile rows of the decode dispatch (T <= EXACT_ROUTER_MAX_T)
+constexpr int DEC_MT = 4;  // token rows of the streaming items' tiles
 // largest T routed by the fused top-k + dispatch launch
 constexpr int FUSED_DISPATCH_MAX_T = 64;
 
 
 // ---- decode layer in two launches (moe_decode.hip), T <= DECODE_MAX_T ----
-constexpr int DECODE_MAX_T = EXACT_ROUTER_MAX_T;
+// (every logit in the canonical order; above, approximate logits and the
+// canonical ones of the candidates)
+constexpr int DECODE_MAX_T = 16;
 // ainfer_moe_block_forward folds the RMSNorm into the decode routing kernel
 // up to this many tokens (its one-token-per-wave form)
 constexpr int DECODE_NORM_MAX_T = 4;

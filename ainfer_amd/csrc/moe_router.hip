@@ -201,17 +201,14 @@ constexpr int SEL_WAVES = 4;
 #define SEL_NB 4  // candidate rows whose loads are issued together
 #endif
 
-// EXACT: `approx` already holds the canonical logits (k_router_logits) and
-// `sgl` the canonical shared-gate logits; the refine is skipped.
 // COOP (T < GEMM_MIN_T, where one wave per token leaves most of the chip
 // idle and a token's latency is the kernel's): one token per workgroup.
 // Wave 0 takes the approximate top-k and the candidate list, wave 1 writes
 // the MFMA-order copy of x, wave 2 the shared-gate dot, and the candidates'
 // canonical dots are shared by all waves (c3 T=64: the dots were 13 of 25 us
 // per token).
-template <int NV, int CH, bool EXACT, bool COOP = false>
+template <int NV, int CH, bool COOP>
 __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx,
-                                                const float *__restrict__ sgl,
                                                 const float *__restrict__ wnorm,
                                                 const uint16_t *__restrict__ x,
                                                 const uint16_t *__restrict__ rw,
@@ -225,9 +222,9 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
                                                 int k, int H, int has_shared, DispatchOut ds,
                                                 int fused, unsigned long long *cmask,
                                                 int32_t *ccount) {
-  // candidate lists (fast path only)
-  __shared__ int cl[SEL_WAVES][EXACT ? 1 : 1024];
-  __shared__ float cv[SEL_WAVES][EXACT ? 1 : 1024];
+  // candidate lists
+  __shared__ int cl[SEL_WAVES][1024];
+  __shared__ float cv[SEL_WAVES][1024];
   __shared__ uint64_t s_cand[SEL_WAVES][64];
   __shared__ uint64_t s_sel[SEL_WAVES][16];
   __shared__ int s_nc;
@@ -236,7 +233,6 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
   const int t = COOP ? (int)blockIdx.x : (int)blockIdx.x * SEL_WAVES + wave;
   const int sw = COOP ? 0 : wave;  // this wave's LDS lists
   const bool lead = !COOP || wave == 0;
-  static_assert(!(COOP && EXACT), "the cooperative form refines approximate logits");
   if (t < T) {
     // the MFMA-order copy of x (and its group sums) does not depend on the
     // routing: written first, its latency hides under the selection
@@ -254,7 +250,7 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
       const int e = lane + 64 * i;
       const float v = ar[min(e, E - 1)];  // unconditional: loads issue together
       key[i] = e < E ? ordered_key(v) : 0u;
-      if (!EXACT) wn = fmaxf(wn, e < E ? wnorm[min(e, E - 1)] : 0.0f);
+      wn = fmaxf(wn, e < E ? wnorm[min(e, E - 1)] : 0.0f);
     }
     int seli = 0;
     uint32_t selk = 0u;
@@ -263,11 +259,7 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
     const uint32_t kth = (uint32_t)__shfl((int)selk, k - 1, 64);
     float selv = 0.0f, sgv = 0.0f;
     const uint16_t *xrow = x + (size_t)t * H;
-    if (EXACT) {
-      // canonical logits already: the picks above are the top-k
-      if (lane < k) selv = ar[seli];
-      if (gw) sgv = sgl[t];
-    } else {
+    {
       // ---- x row in registers (canonical chunk layout) and its norm ------
       const int nch = H >> 3;
       u32x4 xc[CH];
@@ -416,123 +408,20 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
   dispatch_small_block(topk_idx, T, k, E, has_shared, ds);
 }
 
-// Decode routing for T <= 16 in one block, one wave per token: the exact
-// top-k of the canonical logits, softmax weights, the shared-expert gate and
-// the MFMA-order copy of x; then wave 0 builds the dispatch from the picks
-// kept in LDS (tiles of at most DEC_MT tokens).
-__device__ __forceinline__ void dispatch_wave(const int *__restrict__ s_idx, int T, int k, int E,
-                                              int has_shared, const DispatchOut &ds,
-                                              uint32_t *msk, int *off, int lane) {
-  for (int e = lane; e < E; e += 64) msk[e] = 0u;
-  __builtin_amdgcn_wave_barrier();
-  for (int i = lane; i < T * k; i += 64) atomicOr(&msk[s_idx[i]], 1u << (i / k));
-  __builtin_amdgcn_wave_barrier();
-  // lane owns experts [e0, e1): counts, then one tile per expert with tokens
-  const int npl = (E + 63) / 64, e0 = lane * npl, e1 = min(e0 + npl, E);
-  int c_loc = 0, t_loc = 0;
-  for (int e = e0; e < e1; ++e) {
-    const int c = __popc(msk[e]);
-    c_loc += c;
-    t_loc += (c + DEC_MT - 1) / DEC_MT;
-  }
-  int c_inc = c_loc, t_inc = t_loc;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int a = __shfl_up(c_inc, d, 64), b = __shfl_up(t_inc, d, 64);
-    if (lane >= d) {
-      c_inc += a;
-      t_inc += b;
-    }
-  }
-  int o = c_inc - c_loc, tb = t_inc - t_loc;
-  for (int e = e0; e < e1; ++e) {
-    const uint32_t m = msk[e];
-    const int c = __popc(m);
-    ds.counts[e] = c;
-    ds.offsets[e] = o;
-    off[e] = o;
-    for (int m0 = 0; m0 < c; m0 += DEC_MT) ds.tiles[tb++] = make_int4(e, o + m0, min(DEC_MT, c - m0), 0);
-    o += c;
-  }
-  const int total = __shfl(c_inc, 63, 64), routed = __shfl(t_inc, 63, 64);
-  const int nsh = has_shared ? (T + DEC_MT - 1) / DEC_MT : 0;
-  if (lane < nsh) ds.tiles[routed + lane] = make_int4(E, lane * DEC_MT, min(DEC_MT, T - lane * DEC_MT), 0);
-  if (lane == 0) {
-    ds.offsets[E] = total;
-    *ds.n_tiles = routed + nsh;
-  }
-  __builtin_amdgcn_wave_barrier();
-  // placement: rank of token t among the tokens of expert e
-  for (int i = lane; i < T * k; i += 64) {
-    const int t = i / k, e = s_idx[i];
-    const int pos = off[e] + __popc(msk[e] & ((1u << t) - 1u));
-    ds.perm[pos] = i;
-    ds.inv[i] = pos;
-    ds.ptok[pos] = t;
-  }
-}
-
-template <int NV>
-__global__ __launch_bounds__(1024) void k_select_small(const float *__restrict__ logits,
-                                                       const float *__restrict__ sgl,
-                                                       const uint16_t *__restrict__ x,
-                                                       int32_t *__restrict__ topk_idx,
-                                                       float *__restrict__ topk_w,
-                                                       float *__restrict__ sgate,
-                                                       uint16_t *__restrict__ xperm, int T, int E,
-                                                       int k, int H, int has_shared, int has_gate,
-                                                       DispatchOut ds, int fused) {
-  __shared__ int s_idx[SMALL_MT * 32];
-  __shared__ uint32_t s_msk[1024];
-  __shared__ int s_off[1024];
-  __shared__ uint64_t s_cand[SMALL_MT][64];
-  __shared__ uint64_t s_sel[SMALL_MT][16];
-  const int t = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (t < T) {
-    const float *ar = logits + (size_t)t * E;
-    uint32_t key[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int e = lane + 64 * i;
-      const float v = ar[min(e, E - 1)];  // unconditional: loads issue together
-      key[i] = e < E ? ordered_key(v) : 0u;
-    }
-    int seli;
-    uint32_t selk;
-    wave_topk_fast<NV>(key, E, k, lane, seli, selk, s_cand[t], s_sel[t]);
-    const float selv = lane < k ? ar[seli] : 0.0f;
-    const float vmax = __shfl(selv, 0, 64);
-    const float p = lane < k ? expf(selv - vmax) : 0.0f;
-    float sum = 0.0f;
-    for (int j = 0; j < k; ++j) sum += __shfl(p, j, 64);
-    if (lane < k) {
-      topk_idx[(size_t)t * k + lane] = seli;
-      topk_w[(size_t)t * k + lane] = p / sum;
-      s_idx[t * k + lane] = seli;
-    }
-    if (lane == 0) sgate[t] = has_gate ? 1.0f / (1.0f + expf(-sgl[t])) : 1.0f;
-    if (xperm) write_xperm(x + (size_t)t * H, xperm, nullptr, t, H, lane);
-  }
-  if (!fused) return;
-  __syncthreads();
-  if (t == 0) dispatch_wave(s_idx, T, k, E, has_shared, ds, s_msk, s_off, lane);
-}
-
-template <int NV, bool EXACT, bool COOP>
-hipError_t launch_select_nv(int ch, unsigned grid, const float *approx, const float *sgl,
-                            const float *wnorm,
+template <int NV, bool COOP>
+hipError_t launch_select_nv(int ch, unsigned grid, const float *approx, const float *wnorm,
                             const void *x, const void *rw, const float *bias, const void *gw,
                             int32_t *idx, float *w, float *sg, void *xperm, float *xsum, W8Rows w8, int T,
                             int E, int k, int H, int has_shared, const DispatchOut &ds, int fused,
                             unsigned long long *cmask, int32_t *ccount, hipStream_t s) {
 #define SEL_ARGS                                                                            \
-  approx, sgl, wnorm, (const uint16_t *)x, (const uint16_t *)rw, bias, (const uint16_t *)gw, idx, \
+  approx, wnorm, (const uint16_t *)x, (const uint16_t *)rw, bias, (const uint16_t *)gw, idx, \
       w, sg, (uint16_t *)xperm, xsum, w8, T, E, k, H, has_shared, ds, fused, cmask, ccount
   switch (ch) {
-  case 1: k_select<NV, 1, EXACT, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
-  case 2: k_select<NV, 2, EXACT, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
-  case 4: k_select<NV, 4, EXACT, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
-  default: k_select<NV, 8, EXACT, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
+  case 1: k_select<NV, 1, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
+  case 2: k_select<NV, 2, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
+  case 4: k_select<NV, 4, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
+  default: k_select<NV, 8, COOP><<<grid, 256, 0, s>>>(SEL_ARGS); break;
   }
 #undef SEL_ARGS
   return hipGetLastError();
@@ -542,8 +431,7 @@ hipError_t launch_select_nv(int ch, unsigned grid, const float *approx, const fl
 
 bool router_supported(int H, int E) { return H % 128 == 0 && H <= 4096 && E <= 1024; }
 
-template <bool EXACT>
-hipError_t launch_select(const float *approx, const float *sgl, const float *wnorm,
+hipError_t launch_select(const float *approx, const float *wnorm,
                          const void *x, const void *rw, const float *bias, const void *gw,
                          int32_t *idx, float *w, float *sg, void *xperm, float *xsum, W8Rows w8, int T,
                          int H, int E, int k, int has_shared, const DispatchOut *fused,
@@ -556,14 +444,14 @@ hipError_t launch_select(const float *approx, const float *sgl, const float *wno
   memset(&ds, 0, sizeof ds);
   if (fused) ds = *fused;
   // one token per workgroup below the GEMM path (k_select, COOP)
-  const bool coop = !EXACT && T < GEMM_MIN_T;
+  const bool coop = T < GEMM_MIN_T;
   const unsigned g = coop ? (unsigned)T : (T + SEL_WAVES - 1) / SEL_WAVES;
   const int fz = fused ? 1 : 0;
 #define SEL_CALL(NVV)                                                                          \
-  (coop ? launch_select_nv<NVV, EXACT, !EXACT>(chp, g, approx, sgl, wnorm, x, rw, bias, gw, idx, \
+  (coop ? launch_select_nv<NVV, true>(chp, g, approx, wnorm, x, rw, bias, gw, idx, \
                                               w, sg, xperm, xsum, w8, T, E, k, H, has_shared, ds, \
                                               fz, cmask, ccount, s)                           \
-        : launch_select_nv<NVV, EXACT, false>(chp, g, approx, sgl, wnorm, x, rw, bias, gw, idx, \
+        : launch_select_nv<NVV, false>(chp, g, approx, wnorm, x, rw, bias, gw, idx, \
                                               w, sg, xperm, xsum, w8, T, E, k, H, has_shared, ds, \
                                               fz, cmask, ccount, s))
   if (nv <= 1) return SEL_CALL(1);
@@ -588,7 +476,7 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
     hipError_t err = launch_router_gemm(x, rw, bias, approx, wnorm, T, H, E, (uint32_t *)ccount,
                                         (int)(zb / 4), s);
     if (err != hipSuccess) return err;
-    return launch_select<false>(approx, nullptr, wnorm, x, rw, bias, gw, idx, w, sg, xperm,
+    return launch_select(approx, wnorm, x, rw, bias, gw, idx, w, sg, xperm,
                                 xsum, w8, T, H, E, k, has_shared, fused, s, cmask, ccount);
   }
   // one 16-token tile per workgroup: more workgroups share the token reads
@@ -608,32 +496,6 @@ hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, 
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   // ---- refine + select ------------------------------------------------------
-  return launch_select<false>(approx, nullptr, wnorm, x, rw, bias, gw, idx, w, sg, xperm, xsum,
+  return launch_select(approx, wnorm, x, rw, bias, gw, idx, w, sg, xperm, xsum,
                               w8, T, H, E, k, has_shared, fused, s);
-}
-
-hipError_t launch_router_exact(const void *x, const void *rw, const float *bias, const void *gw,
-                               float *logits, float *sg_logit, int32_t *idx, float *w, float *sg,
-                               void *xperm, int T, int H, int E, int k, int has_shared,
-                               const DispatchOut *fused, hipStream_t s) {
-  if (T == 0) return hipSuccess;
-  hipError_t err = launch_router(x, rw, bias, gw, logits, sg_logit,
-                                 fused ? fused->ticket : nullptr, T, H, E, s);
-  if (err != hipSuccess) return err;
-  if (T > SMALL_MT) return hipErrorInvalidValue;
-  DispatchOut ds;
-  memset(&ds, 0, sizeof ds);
-  if (fused) ds = *fused;
-  const int nv = (E + 63) / 64;
-#define SMALL_CALL(NVV)                                                                      \
-  k_select_small<NVV><<<1, 64 * T, 0, s>>>(logits, sg_logit, (const uint16_t *)x, idx, w, sg,  \
-                                          (uint16_t *)xperm, T, E, k, H, has_shared,          \
-                                          gw ? 1 : 0, ds, fused ? 1 : 0)
-  if (nv <= 1) SMALL_CALL(1);
-  else if (nv <= 2) SMALL_CALL(2);
-  else if (nv <= 4) SMALL_CALL(4);
-  else if (nv <= 8) SMALL_CALL(8);
-  else SMALL_CALL(16);
-#undef SMALL_CALL
-  return hipGetLastError();
 }

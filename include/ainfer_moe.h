@@ -425,10 +425,11 @@ int ainfer_moe_fill(int32_t kind, uint64_t seed, float std_, size_t n,
  * tools/decode/decode_l0.cpp:705,714-725,870-884, with device events) -----
  * While enabled, forward/block_forward record a HIP event on the caller's
  * stream before and after every kernel.  For T <= 16 stage 2 is the routing
- * kernel (logits, top-k, weights, dispatch) and stages 1 and 3 read 0; at
- * T = 1 stage 5 is the down + combine kernel (stage 4 the gate/up kernel) and
- * at T = 2 the fused expert kernel (gate/up, down and combine), with stage 6
- * (and at T = 2 stage 4) reading 0.  ainfer_moe_profile_read()
+ * kernel (logits, top-k, weights, dispatch) and stages 1 and 3 read 0; up to
+ * 4 tokens (intermediate sizes up to 1024; at T = 1 any) stage 5 is the down +
+ * combine kernel and stage 6 reads 0, and at T = 2 beyond that size stage 5 may
+ * be the fused expert kernel (gate/up, down and combine) with stages 4 and 6
+ * reading 0.  ainfer_moe_profile_read()
  * waits for them and returns, per stage, the mean device time in
  * microseconds over the calls since enable, and the call count.  Stages:
  * 0 rmsnorm, 1 router, 2 top-k (+ dispatch when T <= 64), 3 dispatch,

@@ -1,0 +1,86 @@
+"""The down + combine kernel of 1 to 4 tokens and the routing kernel in front of
+it at every kind of shape: odd and even numbers of k-groups, experts narrower
+and wider than the shared one, more tiles than waves, one expert with a long K
+(its K shared by several waves), 8 and 16 rows per workgroup.
+
+Outputs are compared with the oracle at the layer's tolerance, and bit for bit
+with the stage entries, whose rows come from the item kernels: the order of
+the additions is the same wherever the items' split of K is."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import check_close, host_copy, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+SHAPES = [(1024, 12, 5, 128, 128), (512, 9, 4, 384, 0), (640, 16, 3, 896, 1792),
+          (1024, 8, 2, 768, 256), (2048, 6, 2, 1152, 0), (256, 40, 32, 256, 256),
+          (384, 8, 1, 2048, 0), (512, 8, 2, 4096, 4096), (4096, 16, 6, 1024, 512),
+          (4096, 12, 3, 640, 384), (128, 1, 1, 128, 128)]
+
+
+@pytest.mark.parametrize("scales", ["fp16", "bf16"])
+@pytest.mark.parametrize("H,E,k,I,Is", SHAPES)
+def test_few_tokens_any_shape(torch, oracle, H, E, k, I, Is, scales):
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    cfg = MoeConfig("dc", H, E, k, I, Is, (4,), seed=11)
+    ly = MoeLayer(cfg, scale_dtype=L.SCALE_FP16 if scales == "fp16" else L.SCALE_BF16)
+    hl = host_copy(oracle, ly)
+    g = torch.Generator().manual_seed(4)
+    nw = (torch.randn(H, generator=g) * 0.3 + 1.0).to(torch.bfloat16).cuda()
+    for T in (1, 2, 3, 4, 5):
+        what = f"H={H} E={E} k={k} I={I} Is={Is} {scales} T={T}"
+        print(f"[case] {what}", flush=True)
+        x = make_input(cfg, T, tag=T)
+        ws = ly.workspace(T)
+        y = torch.full((T, H), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ly.forward(x, y, ws)
+        idx, w, sg, lg = ly.route(x, ws, want_logits=True)
+        y2 = torch.empty_like(y)
+        ly.combine(ly.experts(x, idx, ws), w, sg, y2)
+        b = torch.empty_like(y)
+        ly.block_forward(x, b, ws, norm_w=nw)
+        torch.cuda.synchronize()
+        r_idx, _, _, r_lg = hl.route(to_np(x), T)
+        assert np.array_equal(to_np(lg).view(np.uint32), r_lg.view(np.uint32)), what
+        assert np.array_equal(to_np(idx), r_idx), what
+        check_close(to_np(y), hl.forward(to_np(x), T), what)
+        check_close(to_np(b), oracle.bf16_to_f32(hl.block_forward(to_np(x), T, norm_w=to_np(nw))),
+                    "block " + what)
+        if T >= 3 or max(I, Is) < 1024:
+            assert torch.equal(y.view(torch.int16), y2.view(torch.int16)), what
+        assert ly.workspace_check(ws) == 0
+
+
+@pytest.mark.parametrize("H", [128, 256, 384])
+def test_w4a8_block_of_a_narrow_row(torch, oracle, H):
+    """The folded RMSNorm of rows with fewer 16-byte chunks than a wave has
+    lanes (H < 512), in W4A8."""
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    cfg = MoeConfig("narrow", H, 16, 4, 256, 128, (4,), seed=12)
+    ly = MoeLayer(cfg, precision=L.PRECISION_W4A8)
+    hl = host_copy(oracle, ly)
+    g = torch.Generator().manual_seed(5)
+    nw = (torch.randn(H, generator=g) * 0.3 + 1.0).to(torch.bfloat16).cuda()
+    for T in (1, 4):
+        print(f"[case] w4a8 narrow block H={H} T={T}", flush=True)
+        x = make_input(cfg, T, tag=T)
+        out = torch.empty_like(x)
+        ly.block_forward(x, out, ly.workspace(T), norm_w=nw)
+        torch.cuda.synchronize()
+        h = oracle.rmsnorm_bf16(to_np(x), to_np(nw), L.NORM_PLAIN)
+        want = oracle.bf16_to_f32(to_np(x)) + hl.forward_w4a8(np.ascontiguousarray(h), T)
+        check_close(to_np(out), want, f"w4a8 narrow block H={H} T={T}")
