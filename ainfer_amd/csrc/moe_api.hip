@@ -343,6 +343,12 @@ int do_decode_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const
   a.ss0 = (const uint16_t *)w->ss_down;
   a.w1 = a.ws1 = nullptr;
   a.s1 = a.ss1 = nullptr;
+  if (T == 1 && I <= W8DC_MAX_K && Is <= W8DC_MAX_K) {
+    HIP_TRY(launch_w4a8_down_combine_t1(s->scale_dtype, a, at<float>(ws, L.w),
+                                        at<float>(ws, L.sg), d.inv, resid, y, sync + SY_ERR, st));
+    pc->end(5);
+    return AINFER_OK;
+  }
   HIP_TRY(launch_w4a8_expert(1, s->scale_dtype, a, mtb, st));
   pc->end(5);
   HIP_TRY(launch_combine_f32(a.o, d.inv, at<float>(ws, L.w), at<float>(ws, L.sg), has_shared,

@@ -266,6 +266,12 @@ struct W4A8Args {
 };
 hipError_t launch_w4a8_expert(int mode, int scale_dtype, const W4A8Args &a, int max_tiles,
                               hipStream_t s);
+// T = 1, intermediate sizes up to W8DC_MAX_K: down (a's MODE 1 pointers, act in
+// fp32) and the combine
+constexpr int W8DC_MAX_K = 2048;
+hipError_t launch_w4a8_down_combine_t1(int scale_dtype, const W4A8Args &a, const float *w,
+                                       const float *sg, const int32_t *inv, const void *resid,
+                                       void *y, const int32_t *err, hipStream_t s);
 hipError_t launch_combine_f32(const float *o, const int32_t *inv, const float *w,
                               const float *sg, int has_shared, const void *resid, void *y, int T,
                               int k, int H, const int32_t *err, hipStream_t s);

@@ -537,7 +537,210 @@ __global__ __launch_bounds__(256) void k_combine_f32(const float *__restrict__ o
   y[(size_t)t * H + h] = (err && *err) ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
 }
 
+// ---- T = 1: down and combine in one launch ----------------------------------
+// As k_down_combine (moe_decode.hip): a workgroup owns 8 output rows of every
+// selected expert, a wave per tile, all weight loads in flight together; the
+// rows meet in LDS and are summed in slot order (k_combine_f32's arithmetic).
+// Each wave quantizes its tile's act row while its weights fly (16 elements per
+// lane, k_act_quant_i8's arithmetic), so neither the quantization nor the
+// combine is a launch.  A row's K / 32 chunks of 16 bytes sit in CP lanes, 64 /
+// CP rows per load instruction; the terms are formed and added as gemv1_rows
+// does.  Against the down GEMVs and k_combine_f32 (H4096 I1024 k10 + shared):
+// 12.8 + 5.0 us and a launch gap.
+constexpr int W8DC_ROWS = 8;
+struct W8DownT1Args {
+  const uint8_t *w, *ws;      // down, the shared expert's
+  const uint16_t *s, *ss;
+  const float *act, *act_s;   // [k][I], [Is]
+  const int4 *tiles;
+  const float *wt, *sg;
+  const int32_t *inv;
+  const uint16_t *resid;
+  uint16_t *y;
+  const int32_t *err;
+  int k, H, I, Is, n_tiles;
+};
+
+template <int SD, int CP>
+__global__ __launch_bounds__(1024) void k_w4a8_down_combine_t1(W8DownT1Args a) {
+  constexpr int RPI = 64 / CP, NR = W8DC_ROWS / RPI;  // rows per load, loads per tile
+  constexpr int KM = CP * 32, GM = KM / 128, NPC = (KM + 1023) / 1024;
+  __shared__ float s_o[33][W8DC_ROWS];
+  __shared__ __attribute__((aligned(16))) uint8_t s_q[16][KM];  // codes, W8 order
+  __shared__ float s_sq[16][GM], s_term[16][W8DC_ROWS][GM];
+  const int tx = tid_opaque();
+  const int wave = __builtin_amdgcn_readfirstlane(tx >> 6), lane = tx & 63;
+  const int nw = blockDim.x >> 6, k = a.k, H = a.H;
+  const int row0 = blockIdx.x * W8DC_ROWS;
+  float wj = 0.f, rv = 0.f, sgv = 0.f;
+  int pj = 0;
+  bool bad = false;
+  if (wave == 0) {
+    wj = a.wt[min(lane, k - 1)];
+    pj = a.inv[min(lane, k - 1)];
+    sgv = a.sg[0];
+    if (a.resid) rv = bf16_to_f32(a.resid[row0 + (lane & (W8DC_ROWS - 1))]);
+    bad = *a.err != 0;
+  }
+  const int sub = lane / CP, c = lane % CP;
+  for (int tile = wave; tile < a.n_tiles; tile += nw) {
+    const bool shared = tile == k;
+    const size_t e = shared ? 0 : (size_t)a.tiles[tile].x;
+    const int K = shared ? a.Is : a.I, G = K >> 7, C = K >> 5;
+    const uint8_t *w0 = (shared ? a.ws : a.w) + e * H * (K / 2);
+    const uint16_t *s0 = (shared ? a.ss : a.s) + e * H * G;
+    // act first: its quantization must not wait for the weights
+    const float *act = shared ? a.act_s : a.act + (size_t)tile * K;
+    float4 av[NPC][4];
+#pragma unroll
+    for (int p = 0; p < NPC; ++p)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        av[p][i] = *(const float4 *)(act + min(1024 * p + 16 * lane + 4 * i, K - 4));
+    uint16_t sc[NR];
+    u32x4 wv[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const size_t row = (size_t)(row0 + r * RPI + sub);
+      sc[r] = s0[row * G + min(c >> 2, G - 1)];
+      wv[r] = __builtin_nontemporal_load((const u32x4 *)(w0 + row * (K / 2) + min(c, C - 1) * 16));
+    }
+#pragma unroll
+    for (int p = 0; p < NPC; ++p) {
+      const int e0 = 1024 * p + 16 * lane;
+      float m = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float f[4] = {av[p][i].x, av[p][i].y, av[p][i].z, av[p][i].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float ab = fabsf(f[j]);
+          m = ab > m ? ab : m;
+        }
+      }
+      // the group's 8 lanes
+#pragma unroll
+      for (int o = 4; o >= 1; o >>= 1)
+        m = __uint_as_float(max(__float_as_uint(m), (uint32_t)__shfl_xor((int)__float_as_uint(m), o, 64)));
+      float q1 = m / 127.0f;
+      q1 = q1 == 0.0f ? 1.0f : q1;
+      uint32_t pk[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float f[4] = {av[p][i].x, av[p][i].y, av[p][i].z, av[p][i].w};
+        pk[i] = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float r = f[j] / q1;
+          int qi = (int)(r >= 0.0f ? r + 0.5f : r - 0.5f);
+          qi = qi < -127 ? -127 : (qi > 127 ? 127 : qi);
+          pk[i] |= (uint32_t)(uint8_t)(int8_t)qi << (8 * j);
+        }
+      }
+      if (e0 < K) {
+        // half a 32-element block: its 8 even elements, its 8 odd ones
+        uint8_t *qd = s_q[wave] + (e0 >> 5) * 32 + ((lane & 1) ? 8 : 0);
+        *(uint2 *)qd = make_uint2(__builtin_amdgcn_perm(pk[1], pk[0], 0x06040200u),
+                                  __builtin_amdgcn_perm(pk[3], pk[2], 0x06040200u));
+        *(uint2 *)(qd + 16) = make_uint2(__builtin_amdgcn_perm(pk[1], pk[0], 0x07050301u),
+                                         __builtin_amdgcn_perm(pk[3], pk[2], 0x07050301u));
+        if ((lane & 7) == 0) s_sq[wave][e0 >> 7] = q1;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int cc = min(c, C - 1);
+    const i32x4 xe = *(const i32x4 *)(s_q[wave] + cc * 32), xo = *(const i32x4 *)(s_q[wave] + cc * 32 + 16);
+    const float sqg = s_sq[wave][cc >> 2];
+    int sx = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sx = __builtin_amdgcn_sdot4(xe[j], 0x01010101, sx, false);
+      sx = __builtin_amdgcn_sdot4(xo[j], 0x01010101, sx, false);
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      int d = -8 * sx;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t u = wv[r][j] ^ 0x88888888u;  // nibble q -> q + 8
+        d = __builtin_amdgcn_sdot4((int)(u & 0x0F0F0F0Fu), xe[j], d, false);
+        d = __builtin_amdgcn_sdot4((int)((u >> 4) & 0x0F0F0F0Fu), xo[j], d, false);
+      }
+      d += __builtin_amdgcn_mov_dpp(d, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
+      d += __builtin_amdgcn_mov_dpp(d, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
+      if ((c & 3) == 0 && c < C) {
+#pragma clang fp contract(off)
+        s_term[wave][r * RPI + sub][c >> 2] = (float)d * scale_to_f32<SD>(sc[r]) * sqg;  // unfused
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < W8DC_ROWS) {
+#pragma clang fp contract(off)
+      float acc = 0.0f;
+      for (int g = 0; g < G; ++g) acc = acc + s_term[wave][lane][g];  // group order
+      s_o[tile][lane] = acc;
+    }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  const int r = lane & (W8DC_ROWS - 1);
+  float acc = 0.f;
+  for (int j = 0; j < k; ++j) {
+    const int p = __builtin_amdgcn_readlane(pj, j);
+    acc = __builtin_fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wj), j)), s_o[p][r], acc);
+  }
+  if (a.n_tiles > k) acc = __builtin_fmaf(sgv, s_o[k][r], acc);
+  if (a.resid) acc += rv;
+  if (lane < W8DC_ROWS) a.y[row0 + lane] = bad ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
+}
+
 }  // namespace
+
+hipError_t launch_w4a8_down_combine_t1(int scale_dtype, const W4A8Args &d, const float *w,
+                                       const float *sg, const int32_t *inv, const void *resid,
+                                       void *y, const int32_t *err, hipStream_t s) {
+  const int Kmax = d.I > d.Is ? d.I : d.Is;
+  if (d.T != 1 || d.k > 32 || d.H % W8DC_ROWS || Kmax > W8DC_MAX_K) return hipErrorInvalidValue;
+  W8DownT1Args a;
+  a.w = d.w0;
+  a.ws = d.ws0;
+  a.s = d.s0;
+  a.ss = d.ss0;
+  a.act = d.act;
+  a.act_s = d.act_s;
+  a.tiles = d.tiles;
+  a.wt = w;
+  a.sg = sg;
+  a.inv = inv;
+  a.resid = (const uint16_t *)resid;
+  a.y = (uint16_t *)y;
+  a.err = err;
+  a.k = d.k;
+  a.H = d.H;
+  a.I = d.I;
+  a.Is = d.Is;
+  a.n_tiles = d.k + (d.Is > 0 ? 1 : 0);
+  const int nw = a.n_tiles < 16 ? a.n_tiles : 16;
+  auto go = [&](auto sd_c) {
+    constexpr int SDc = decltype(sd_c)::value;
+    const dim3 g(d.H / W8DC_ROWS), b(nw * 64);
+    if (Kmax <= 512)
+      k_w4a8_down_combine_t1<SDc, 16><<<g, b, 0, s>>>(a);
+    else if (Kmax <= 1024)
+      k_w4a8_down_combine_t1<SDc, 32><<<g, b, 0, s>>>(a);
+    else
+      k_w4a8_down_combine_t1<SDc, 64><<<g, b, 0, s>>>(a);
+  };
+  if (scale_dtype == AINFER_SCALE_FP16)
+    go(std::integral_constant<int, AINFER_SCALE_FP16>());
+  else
+    go(std::integral_constant<int, AINFER_SCALE_BF16>());
+  return hipGetLastError();
+}
 
 hipError_t launch_act_quant_i8(const void *x, int x_dtype, int T, int K, int8_t *q, float *sq,
                                hipStream_t s) {

@@ -84,3 +84,29 @@ def test_w4a8_block_of_a_narrow_row(torch, oracle, H):
         h = oracle.rmsnorm_bf16(to_np(x), to_np(nw), L.NORM_PLAIN)
         want = oracle.bf16_to_f32(to_np(x)) + hl.forward_w4a8(np.ascontiguousarray(h), T)
         check_close(to_np(out), want, f"w4a8 narrow block H={H} T={T}")
+
+
+@pytest.mark.parametrize("H,E,k,I,Is", [(512, 8, 3, 128, 384), (1024, 40, 20, 512, 0),
+                                        (4096, 12, 10, 1024, 256), (640, 9, 4, 896, 1792),
+                                        (256, 5, 2, 2048, 128), (384, 4, 2, 2304, 256)])
+def test_w4a8_one_token_equals_its_row_of_two(torch, H, E, k, I, Is):
+    """In W4A8 a token's output is defined bit by bit: the T = 1 kernels
+    (down with the quantization and the combine in it up to I = 2048) give the
+    token's row of a T = 2 call, with and without the residual."""
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    cfg = MoeConfig("w8dc", H, E, k, I, Is, (2,), seed=13)
+    for sd in (L.SCALE_FP16, L.SCALE_BF16):
+        print(f"[case] w4a8 T=1 H={H} E={E} k={k} I={I} Is={Is} scales={sd}", flush=True)
+        ly = MoeLayer(cfg, scale_dtype=sd, precision=L.PRECISION_W4A8)
+        x = make_input(cfg, 2, tag=3)
+        ws = ly.workspace(2)
+        two, one = torch.empty_like(x), torch.empty_like(x)
+        for fn in (ly.forward, ly.block_forward):
+            fn(x, two, ws)
+            for t in range(2):
+                fn(x[t:t + 1], one[t:t + 1], ws)
+            torch.cuda.synchronize()
+            assert torch.isfinite(two.float()).all()
+            assert torch.equal(one.view(torch.int16), two.view(torch.int16)), fn.__name__
