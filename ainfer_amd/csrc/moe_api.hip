@@ -280,158 +280,133 @@ ExpertArgs expert_args(const ainfer_moe_shape *s, const ainfer_moe_weights *w, c
 // the routing kernel applies the RMSNorm itself
 int down_kbw(const ainfer_moe_shape &s) { return down_kbw_of(s); }
 
-// The layer in W4A8 (AINFER_PRECISION_W4A8) at decode sizes: the W4A16 decode
-// routing kernel (canonical logits, top-k, weights, gate, the MFMA-order copy
-// of x with its W4A8 codes, the dispatch in tiles of DEC_MT tokens, and with
-// norm the block's RMSNorm), the grouped gate/up GEMVs with SiLU, act
-// quantized, the grouped down GEMVs and the fp32 combine (moe_w4a8.hip).
-int do_decode_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void *x,
-                   const void *resid, void *y, int T, void *ws, hipStream_t st, ProfCall *pc,
-                   const NormIn *norm) {
-  const Layout L = layout_of(*s, T);
-  const int E = s->n_experts, k = s->top_k, H = s->hidden, I = s->inter, Is = s->shared_inter;
-  const int has_shared = Is > 0;
-  DispatchOut d = dispatch_out(s, L, ws, T);
-  d.mt = DEC_MT;
-  DispatchOut dr = d;  // nothing here reads the per-expert counts or offsets
-  dr.counts = nullptr;
-  dr.offsets = nullptr;
-  int32_t *sync = at<int32_t>(ws, L.sync);
-  HIP_TRY(launch_route_decode(x, w->router_w, w->router_bias, w->shared_gate_w,
-                              at<float>(ws, L.logits), at<float>(ws, L.sg_logit),
-                              at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
-                              at<uint16_t>(ws, L.xperm), T, H, E, k, has_shared, &dr, sync,
-                              (uint32_t *)(sync + L.slots), norm, st, at<int8_t>(ws, L.w8_xq),
-                              at<float>(ws, L.w8_xs)));
-  pc->end(3);
-  W4A8Args a;
-  memset(&a, 0, sizeof a);
-  a.xq = at<int8_t>(ws, L.w8_xq);
-  a.xs = at<float>(ws, L.w8_xs);
-  a.act = at<float>(ws, L.w8_act);
-  a.act_s = at<float>(ws, L.w8_acts);
-  a.aq = at<int8_t>(ws, L.w8_aq);
-  a.as = at<float>(ws, L.w8_as);
-  a.aq_s = at<int8_t>(ws, L.w8_aqs);
-  a.as_s = at<float>(ws, L.w8_ass);
-  a.o = at<float>(ws, L.w8_o);
-  a.ptok = d.ptok;
-  a.tiles = d.tiles;
-  a.n_tiles = d.n_tiles;
-  a.T = T;
-  a.k = k;
-  a.E = E;
-  a.H = H;
-  a.I = I;
-  a.Is = Is;
-  const int mtb = max_tiles_bound(*s, T, d.mt);
-  a.w0 = w->w_gate;
-  a.w1 = w->w_up;
-  a.s0 = (const uint16_t *)w->s_gate;
-  a.s1 = (const uint16_t *)w->s_up;
-  a.ws0 = w->ws_gate;
-  a.ws1 = w->ws_up;
-  a.ss0 = (const uint16_t *)w->ss_gate;
-  a.ss1 = (const uint16_t *)w->ss_up;
-  HIP_TRY(launch_w4a8_expert(0, s->scale_dtype, a, mtb, st));
-  pc->end(4);
-  // the down launch quantizes act itself (at T = 1 inside its blocks)
-  a.quant_in = 1;
-  a.w0 = w->w_down;
-  a.s0 = (const uint16_t *)w->s_down;
-  a.ws0 = w->ws_down;
-  a.ss0 = (const uint16_t *)w->ss_down;
-  a.w1 = a.ws1 = nullptr;
-  a.s1 = a.ss1 = nullptr;
-  if (T == 1 && I <= W8DC_MAX_K && Is <= W8DC_MAX_K) {
-    HIP_TRY(launch_w4a8_down_combine_t1(s->scale_dtype, a, at<float>(ws, L.w),
-                                        at<float>(ws, L.sg), d.inv, resid, y, sync + SY_ERR, st));
-    pc->end(5);
-    return AINFER_OK;
-  }
-  HIP_TRY(launch_w4a8_expert(1, s->scale_dtype, a, mtb, st));
-  pc->end(5);
-  HIP_TRY(launch_combine_f32(a.o, d.inv, at<float>(ws, L.w), at<float>(ws, L.sg), has_shared,
-                             resid, y, T, k, H, at<int32_t>(ws, L.sync) + SY_ERR, st));
-  pc->end(6);
-  return AINFER_OK;
-}
-
-// The same layer above the decode sizes: the staged router (k_select
-// quantizes x into W8 order), 64-token tiles, the gate/up GEMM (which
-// quantizes act), the down GEMM and the fp32 combine (moe_gemm_w4a8.hip).
+// The layer in W4A8 (AINFER_PRECISION_W4A8): routing as in W4A16, with x
+// quantized beside it, then the expert GEMVs of the reference's numerics.
+//  T <= 16  the decode routing kernel (with norm the block's RMSNorm), tiles of
+//           DEC_MT tokens
+//  above    the staged router (k_select quantizes x), tiles of gemm_mt tokens
+// Gate/up: the one-token GEMVs at T = 1 (moe_w4a8.hip), the int8 GEMM where
+// w4a8_gemm_at (moe_gemm_w4a8.hip; it quantizes act), else the 16-row GEMV
+// blocks.  Down: with the combine in one launch up to DC_MAX_T tokens (sizes to
+// W8DC_MAX_K), else as gate/up with the fp32 combine.
 int do_forward_w4a8(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const void *x,
                     const void *resid, void *y, int T, void *ws, hipStream_t st, ProfCall *pc,
                     const NormIn *norm = nullptr) {
-  if (T <= DECODE_MAX_T) return do_decode_w4a8(s, w, x, resid, y, T, ws, st, pc, norm);
-  if (norm) return AINFER_ERR_ARG;  // the caller normalizes at these sizes
   const Layout L = layout_of(*s, T);
-  const int E = s->n_experts, k = s->top_k, H = s->hidden;
-  const int has_shared = s->shared_inter > 0;
+  const int E = s->n_experts, k = s->top_k, H = s->hidden, I = s->inter, Is = s->shared_inter;
+  const int has_shared = Is > 0;
+  const bool decode = T <= DECODE_MAX_T, gemm = w4a8_gemm_at(*s, T);
+  if (norm && !decode) return AINFER_ERR_ARG;  // the caller normalizes above that
   DispatchOut d = dispatch_out(s, L, ws, T);
-  d.mt = gemm_mt(*s, T);
-  const bool fused = T <= FUSED_DISPATCH_MAX_T;
-  unsigned long long *cmask =
-      T >= GEMM_MIN_T ? at<unsigned long long>(ws, L.chunk_masks) : nullptr;
+  d.mt = decode ? DEC_MT : gemm_mt(*s, T);
   // the group sums take the places of the W4A16 GEMM's (the same counts of
   // 4-byte values)
   W8Rows xq, aq, aqs;
   xq.q = at<int8_t>(ws, L.w8_xq);
   xq.s = at<float>(ws, L.w8_xs);
-  xq.sum = at<int32_t>(ws, L.xsum);
+  xq.sum = gemm ? at<int32_t>(ws, L.xsum) : nullptr;
   aq.q = at<int8_t>(ws, L.w8_aq);
   aq.s = at<float>(ws, L.w8_as);
   aq.sum = at<int32_t>(ws, L.asum);
   aqs.q = at<int8_t>(ws, L.w8_aqs);
   aqs.s = at<float>(ws, L.w8_ass);
   aqs.sum = at<int32_t>(ws, L.asum_s);
-  HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
-                             at<float>(ws, L.logits), at<float>(ws, L.wnorm),
-                             at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
-                             nullptr, nullptr, T, H, E, k, has_shared, fused ? &d : nullptr, st,
-                             cmask ? at<int32_t>(ws, L.chunk_counts) : nullptr, cmask, xq));
-  pc->end(2);
-  if (!fused)
-    HIP_TRY(launch_dispatch(at<int32_t>(ws, L.idx), T, k, E, d.mt, has_shared,
-                            at<int32_t>(ws, L.chunk_counts), at<int32_t>(ws, L.rank), d, st,
-                            cmask));
+  int32_t *sync = at<int32_t>(ws, L.sync);
+  if (decode) {
+    DispatchOut dr = d;  // nothing here reads the per-expert counts or offsets
+    dr.counts = nullptr;
+    dr.offsets = nullptr;
+    HIP_TRY(launch_route_decode(x, w->router_w, w->router_bias, w->shared_gate_w,
+                                at<float>(ws, L.logits), at<float>(ws, L.sg_logit),
+                                at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
+                                nullptr, T, H, E, k, has_shared, &dr, sync,
+                                (uint32_t *)(sync + L.slots), norm, st, xq));
+  } else {
+    const bool fused = T <= FUSED_DISPATCH_MAX_T;
+    unsigned long long *cmask =
+        T >= GEMM_MIN_T ? at<unsigned long long>(ws, L.chunk_masks) : nullptr;
+    HIP_TRY(launch_router_fast(x, w->router_w, w->router_bias, w->shared_gate_w,
+                               at<float>(ws, L.logits), at<float>(ws, L.wnorm),
+                               at<int32_t>(ws, L.idx), at<float>(ws, L.w), at<float>(ws, L.sg),
+                               nullptr, nullptr, T, H, E, k, has_shared, fused ? &d : nullptr, st,
+                               cmask ? at<int32_t>(ws, L.chunk_counts) : nullptr, cmask, xq));
+    pc->end(2);
+    if (!fused)
+      HIP_TRY(launch_dispatch(at<int32_t>(ws, L.idx), T, k, E, d.mt, has_shared,
+                              at<int32_t>(ws, L.chunk_counts), at<int32_t>(ws, L.rank), d, st,
+                              cmask));
+  }
   pc->end(3);
-  W8GemmArgs g;
+  const int mtb = max_tiles_bound(*s, T, d.mt);
+  float *o = at<float>(ws, L.w8_o);
+  W8GemmArgs g;  // the GEMM's, and the one-token kernels'
   memset(&g, 0, sizeof g);
+  W4A8Args a;
+  memset(&a, 0, sizeof a);
   g.x = xq;
   g.act = aq;
   g.act_s = aqs;
-  g.o = at<float>(ws, L.w8_o);
-  g.ptok = d.ptok;
-  g.tiles = d.tiles;
-  g.n_tiles = d.n_tiles;
-  g.T = T;
-  g.k = k;
-  g.E = E;
-  g.H = H;
-  g.I = s->inter;
-  g.Is = s->shared_inter;
-  g.w0 = w->w_gate;
-  g.w1 = w->w_up;
-  g.s0 = (const uint16_t *)w->s_gate;
-  g.s1 = (const uint16_t *)w->s_up;
-  g.ws0 = w->ws_gate;
-  g.ws1 = w->ws_up;
-  g.ss0 = (const uint16_t *)w->ss_gate;
-  g.ss1 = (const uint16_t *)w->ss_up;
-  const int gtiles = max_tiles_bound(*s, T, d.mt);
-  HIP_TRY(launch_w4a8_gemm(0, s->scale_dtype, g, gtiles, st));
+  a.xq = xq.q;
+  a.xs = xq.s;
+  a.act = at<float>(ws, L.w8_act);
+  a.act_s = at<float>(ws, L.w8_acts);
+  a.aq = aq.q;
+  a.as = aq.s;
+  a.aq_s = aqs.q;
+  a.as_s = aqs.s;
+  auto set = [&](auto &q, const void *w0, const void *s0, const void *w1, const void *s1,
+                 const void *ws0, const void *ss0, const void *ws1, const void *ss1) {
+    q.o = o;
+    q.ptok = d.ptok;
+    q.tiles = d.tiles;
+    q.n_tiles = d.n_tiles;
+    q.T = T;
+    q.k = k;
+    q.E = E;
+    q.H = H;
+    q.I = I;
+    q.Is = Is;
+    q.w0 = (const uint8_t *)w0;
+    q.s0 = (const uint16_t *)s0;
+    q.w1 = (const uint8_t *)w1;
+    q.s1 = (const uint16_t *)s1;
+    q.ws0 = (const uint8_t *)ws0;
+    q.ss0 = (const uint16_t *)ss0;
+    q.ws1 = (const uint8_t *)ws1;
+    q.ss1 = (const uint16_t *)ss1;
+  };
+  auto gate_up = [&](auto &q) {
+    set(q, w->w_gate, w->s_gate, w->w_up, w->s_up, w->ws_gate, w->ss_gate, w->ws_up, w->ss_up);
+  };
+  auto down = [&](auto &q) {
+    set(q, w->w_down, w->s_down, nullptr, nullptr, w->ws_down, w->ss_down, nullptr, nullptr);
+  };
+  if (gemm) {
+    gate_up(g);
+    HIP_TRY(launch_w4a8_gemm(0, s->scale_dtype, g, mtb, st));
+  } else {
+    gate_up(a);
+    HIP_TRY(T == 1 ? launch_w4a8_expert_t1(0, s->scale_dtype, a, mtb, st)
+                   : launch_w4a8_expert(0, s->scale_dtype, a, mtb, st));
+  }
   pc->end(4);
-  g.w0 = w->w_down;
-  g.s0 = (const uint16_t *)w->s_down;
-  g.ws0 = w->ws_down;
-  g.ss0 = (const uint16_t *)w->ss_down;
-  g.w1 = g.ws1 = nullptr;
-  g.s1 = g.ss1 = nullptr;
-  HIP_TRY(launch_w4a8_gemm(1, s->scale_dtype, g, gtiles, st));
+  down(a);
+  if (T <= DC_MAX_T && (T == 1 || gemm) && I <= W8DC_MAX_K && Is <= W8DC_MAX_K) {
+    HIP_TRY(launch_w4a8_down_combine(s->scale_dtype, a, aq, aqs, at<float>(ws, L.w),
+                                     at<float>(ws, L.sg), d.inv, resid, y, sync + SY_ERR, st));
+    pc->end(5);
+    return AINFER_OK;
+  }
+  if (gemm) {
+    down(g);
+    HIP_TRY(launch_w4a8_gemm(1, s->scale_dtype, g, mtb, st));
+  } else {
+    HIP_TRY(T == 1 ? launch_w4a8_expert_t1(1, s->scale_dtype, a, mtb, st)
+                   : launch_w4a8_expert(1, s->scale_dtype, a, mtb, st));
+  }
   pc->end(5);
-  HIP_TRY(launch_combine_f32(g.o, d.inv, at<float>(ws, L.w), at<float>(ws, L.sg), has_shared,
-                             resid, y, T, k, H, at<int32_t>(ws, L.sync) + SY_ERR, st));
+  HIP_TRY(launch_combine_f32(o, d.inv, at<float>(ws, L.w), at<float>(ws, L.sg), has_shared, resid,
+                             y, T, k, H, sync + SY_ERR, st));
   pc->end(6);
   return AINFER_OK;
 }

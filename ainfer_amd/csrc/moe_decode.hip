@@ -131,8 +131,7 @@ struct RouteDecodeArgs {
   int32_t *idx;
   float *w, *sg;
   uint16_t *xperm;
-  int8_t *w8q;      // optional: W4A8 codes and group scales of the (normalized) x
-  float *w8sq;
+  W8Rows w8;        // optional: W4A8 rows of the (normalized) x (sum null: natural order)
   DispatchOut ds;
   int32_t *sync;
   uint32_t *slots;  // [DECODE_MAX_T][E + 1] ~bits of the logits (sync region)
@@ -279,10 +278,10 @@ __global__ __launch_bounds__(W * 64) void k_route_decode(RouteDecodeArgs a) {
     // ---- workgroup NR + 1: the MFMA-order copy of x, one wave per token.
     // It does not depend on the routing; a workgroup of its own keeps it off
     // the selection's path (the selection polls as soon as it starts).
-    if (t < T && a.xperm) {
+    if (t < T && (a.xperm || a.w8.q)) {
       const float inv = NORM ? row_rms_inv(a.x + (size_t)t * H, H, a.norm.eps, lane) : 1.0f;
       write_xperm(a.x + (size_t)t * H, a.xperm, nullptr, t, H, lane, NORM ? &a.norm : nullptr, inv,
-                  a.w8q, a.w8sq);
+                  a.w8.q, a.w8.s, a.w8.sum);
     }
     return;
   }
@@ -709,7 +708,7 @@ hipError_t launch_route_decode(const void *x, const void *rw, const float *bias,
                                float *logits, float *sgl, int32_t *idx, float *w, float *sg,
                                void *xperm, int T, int H, int E, int k, int has_shared,
                                const DispatchOut *ds, int32_t *sync, uint32_t *slots,
-                               const NormIn *norm, hipStream_t s, int8_t *w8q, float *w8sq) {
+                               const NormIn *norm, hipStream_t s, W8Rows w8) {
   if (T <= 0) return hipSuccess;
   if (T > DECODE_MAX_T || T > RD_WAVES || E > 1024) return hipErrorInvalidValue;
   RouteDecodeArgs a;
@@ -724,9 +723,7 @@ hipError_t launch_route_decode(const void *x, const void *rw, const float *bias,
   a.w = w;
   a.sg = sg;
   a.xperm = (uint16_t *)xperm;
-  a.w8q = w8q;
-  a.w8sq = w8sq;
-  if (w8q && !xperm) return hipErrorInvalidValue;  // the codes come with the MFMA-order copy
+  a.w8 = w8;
   if (ds) a.ds = *ds;
   a.sync = sync;
   a.slots = slots;

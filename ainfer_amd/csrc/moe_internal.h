@@ -112,6 +112,15 @@ struct W8GemmArgs {
   int T, k, E, H, I, Is;
   int n_nblk;            // set by the launcher
 };
+// The W4A8 GEMM from 2 tokens on, except at decode sizes where its items are few
+// and long: a down product of more than 2048 columns (H2048 E8 k2 I4096, T = 2:
+// 34 us by 16-row GEMV blocks, 45), or fewer than 24 gate/up items (H3584 E66 k5
+// I128, T = 2: 32 and 33; T = 6: 41 and 37).  Else T = 2 to 16 gain 10 to 35%
+// (H2048 E512 k10 I512: T = 4 42 -> 32 us, T = 16 94 -> 79).
+inline bool w4a8_gemm_at(const ainfer_moe_shape &s, int T) {
+  if (T > 16 || T < 2) return T > 1;
+  return s.inter <= 2048 && s.shared_inter <= 2048 && (long)T * s.top_k * (s.inter / 128) >= 24;
+}
 hipError_t launch_w4a8_gemm(int mode, int scale_dtype, W8GemmArgs a, int max_tiles,
                             hipStream_t s);
 
@@ -244,43 +253,44 @@ struct DecodeGeom {
   size_t lds;              // dynamic LDS bytes
 };
 // W4A8 GEMV numerics (moe_w4a8.hip)
-// The MoE layer in W4A8 at decode sizes: the grouped expert GEMVs over
-// dispatch tiles of at most DEC_MT tokens and the fp32 combine.
+// The MoE layer in W4A8 at decode sizes: the expert GEMVs and the fp32 combine.
 struct W4A8Args {
   const uint8_t *w0, *w1, *ws0, *ws1;     // MODE 0: gate, up; MODE 1: down (w0/ws0)
   const uint16_t *s0, *s1, *ss0, *ss1;
   const int8_t *xq;                      // [T][H] x quantized
   const float *xs;                       // [T][H/128]
   float *act, *act_s;                    // MODE 0 out: [T*k][I], [T][Is]
-  const int8_t *aq, *aq_s;               // MODE 1 in: act quantized
-  const float *as, *as_s;                // their group scales
+  int8_t *aq, *aq_s;                     // MODE 1: act quantized (T > 1; written by the launch)
+  float *as, *as_s;                      // their group scales
   float *o;                              // MODE 1 out: [T*k + T][H]
   const int32_t *ptok;
   const int4 *tiles;
   const int32_t *n_tiles;
   int T, k, E, H, I, Is;
-  // MODE 1: act / act_s are the fp32 inputs; the launch quantizes them into
-  // aq / as (one token per tile: inside the GEMV kernel, each block into its
-  // LDS; else a quantization launch first)
-  int quant_in;
 };
+// T > 1, tiles of at most 16 tokens: mode 0 gate/up + SiLU (act in fp32), mode 1
+// act's quantization, then down
 hipError_t launch_w4a8_expert(int mode, int scale_dtype, const W4A8Args &a, int max_tiles,
                               hipStream_t s);
-// T = 1, intermediate sizes up to W8DC_MAX_K: down (a's MODE 1 pointers, act in
-// fp32) and the combine
+hipError_t launch_act_quant_f32_pair(const float *x, int T, int K, int8_t *q, float *sq,
+                                     const float *x2, int T2, int K2, int8_t *q2, float *sq2,
+                                     hipStream_t s);
+// T = 1: mode 0 gate/up + SiLU (act in fp32), mode 1 down (quantizes act in its
+// blocks)
+hipError_t launch_w4a8_expert_t1(int mode, int scale_dtype, const W4A8Args &a, int max_tiles,
+                                 hipStream_t s);
+// T <= DC_MAX_T, intermediate sizes up to W8DC_MAX_K: down (a's MODE 1 pointers)
+// and the combine.  T = 1: act in a in fp32; else quantized in q, q_s.
 constexpr int W8DC_MAX_K = 2048;
-hipError_t launch_w4a8_down_combine_t1(int scale_dtype, const W4A8Args &a, const float *w,
-                                       const float *sg, const int32_t *inv, const void *resid,
-                                       void *y, const int32_t *err, hipStream_t s);
+hipError_t launch_w4a8_down_combine(int scale_dtype, const W4A8Args &a, const W8Rows &q,
+                                    const W8Rows &q_s, const float *w, const float *sg,
+                                    const int32_t *inv, const void *resid, void *y,
+                                    const int32_t *err, hipStream_t s);
 hipError_t launch_combine_f32(const float *o, const int32_t *inv, const float *w,
                               const float *sg, int has_shared, const void *resid, void *y, int T,
                               int k, int H, const int32_t *err, hipStream_t s);
 hipError_t launch_act_quant_i8(const void *x, int x_dtype, int T, int K, int8_t *q, float *sq,
                                hipStream_t s);
-// two fp32 quantizations in one launch (x2 may be null)
-hipError_t launch_act_quant_f32_pair(const float *x, int T, int K, int8_t *q, float *sq,
-                                     const float *x2, int T2, int K2, int8_t *q2, float *sq2,
-                                     hipStream_t s);
 hipError_t launch_int4_gemv_i8(const uint8_t *P, const void *S, int scale_dtype, const int8_t *xq,
                                const float *sq, int M, int K, int T, float *y, hipStream_t s);
 // 0 when the shape has no decode geometry (the staged path is used then)
@@ -291,8 +301,7 @@ hipError_t launch_route_decode(const void *x, const void *rw, const float *bias,
                                float *logits, float *sgl, int32_t *idx, float *w, float *sg,
                                void *xperm, int T, int H, int E, int k, int has_shared,
                                const DispatchOut *ds, int32_t *sync, uint32_t *slots,
-                               const NormIn *norm, hipStream_t s, int8_t *w8q = nullptr,
-                               float *w8sq = nullptr);
+                               const NormIn *norm, hipStream_t s, W8Rows w8 = W8Rows());
 // gate/up + SiLU, down and the combine (y = sum_j w_j o_j + g_s o_s (+ resid))
 // in one launch
 hipError_t launch_experts_decode(int scale_dtype, const DecodeGeom &g, ExpertArgs gu,

@@ -409,8 +409,9 @@ __device__ __forceinline__ void quant_row_lds(const QRow &r, int K, int8_t *q, f
 //   MODE 0: act[pos][n] = silu(gate . x) * (up . x), fp32 (SiluMul,
 //           tools/cmdlist/kernels.cpp:29-37);
 //   MODE 1: o[pos][h] = down . act.
-template <int SD, int MODE, int NC, bool QIN = false>
+template <int SD, int MODE, int NC>
 __global__ __launch_bounds__(GV1_WAVES * 64) void k_w4a8_expert_t1(W4A8Args a) {
+  constexpr bool QIN = MODE == 1;
   constexpr int NMAT = MODE == 0 ? 2 : 1;
   __shared__ float term[GV1_WAVES][NMAT * GV1_RW * NC * 16];
   // QIN: the block's own int8 copy of its fp32 activation row
@@ -444,18 +445,11 @@ __global__ __launch_bounds__(GV1_WAVES * 64) void k_w4a8_expert_t1(W4A8Args a) {
   } else {
     const uint8_t *const Pm[1] = {shared ? a.ws0 : a.w0 + (size_t)e * N * rowb};
     const uint16_t *const Sm[1] = {shared ? a.ss0 : a.s0 + (size_t)e * N * G};
-    float v;
-    if constexpr (QIN) {
-      const QRow xr = quant_row_load((shared ? a.act_s : a.act) + (size_t)pos0 * K, K);
-      v = gemv1_rows<SD, NC, 1>(Pm, Sm, m0, N, K, q_l, sq_l, term[wave], lane, [&]() {
-        quant_row_lds(xr, K, q_l, sq_l);
-        __syncthreads();
-      });
-    } else {
-      const int8_t *aq = (shared ? a.aq_s : a.aq) + (size_t)pos0 * K;
-      const float *as = (shared ? a.as_s : a.as) + (size_t)pos0 * G;
-      v = gemv1_rows<SD, NC, 1>(Pm, Sm, m0, N, K, aq, as, term[wave], lane);
-    }
+    const QRow xr = quant_row_load((shared ? a.act_s : a.act) + (size_t)pos0 * K, K);
+    const float v = gemv1_rows<SD, NC, 1>(Pm, Sm, m0, N, K, q_l, sq_l, term[wave], lane, [&]() {
+      quant_row_lds(xr, K, q_l, sq_l);
+      __syncthreads();
+    });
     if (lane < GV1_RW && m0 + lane < N)
       a.o[(size_t)((shared ? a.T * a.k : 0) + pos0) * N + m0 + lane] = v;
   }
@@ -537,66 +531,101 @@ __global__ __launch_bounds__(256) void k_combine_f32(const float *__restrict__ o
   y[(size_t)t * H + h] = (err && *err) ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
 }
 
-// ---- T = 1: down and combine in one launch ----------------------------------
+// ---- T <= 4: down and combine in one launch ---------------------------------
 // As k_down_combine (moe_decode.hip): a workgroup owns 8 output rows of every
 // selected expert, a wave per tile, all weight loads in flight together; the
 // rows meet in LDS and are summed in slot order (k_combine_f32's arithmetic).
-// Each wave quantizes its tile's act row while its weights fly (16 elements per
-// lane, k_act_quant_i8's arithmetic), so neither the quantization nor the
-// combine is a launch.  A row's K / 32 chunks of 16 bytes sit in CP lanes, 64 /
-// CP rows per load instruction; the terms are formed and added as gemv1_rows
-// does.  Against the down GEMVs and k_combine_f32 (H4096 I1024 k10 + shared):
-// 12.8 + 5.0 us and a launch gap.
+// A row's K / 32 chunks of 16 bytes sit in CP lanes, 64 / CP rows per load
+// instruction; the terms are formed and added as gemv1_rows does.
+// MT = 1 (T = 1): act comes in fp32 and each wave quantizes its tile's row while
+// its weights fly (16 elements per lane, k_act_quant_i8's arithmetic), so
+// neither the quantization nor the combine is a launch: 9.9 us against 12.8
+// (down GEMVs) + 5.0 (combine) and a launch gap at H4096 I1024 k10 + shared.
+// MT = 4 (T = 2 to 4): act comes quantized in W8 order from the GEMM's gate/up
+// epilogue (quantizing T rows per tile in every workgroup would cost more than
+// it hides).
 constexpr int W8DC_ROWS = 8;
-struct W8DownT1Args {
+struct W8DownArgs {
   const uint8_t *w, *ws;      // down, the shared expert's
   const uint16_t *s, *ss;
-  const float *act, *act_s;   // [k][I], [Is]
+  const float *act, *act_s;   // MT = 1: [k][I], [Is]
+  W8Rows q, q_s;              // MT = 4: [T k][I], [T][Is]
   const int4 *tiles;
+  const int32_t *n_tiles;
   const float *wt, *sg;
   const int32_t *inv;
   const uint16_t *resid;
   uint16_t *y;
   const int32_t *err;
-  int k, H, I, Is, n_tiles;
+  int T, k, E, H, I, Is, max_tiles;
 };
 
-template <int SD, int CP>
-__global__ __launch_bounds__(1024) void k_w4a8_down_combine_t1(W8DownT1Args a) {
+template <int SD, int CP, int MT>
+__global__ __launch_bounds__(1024) void k_w4a8_down_combine(W8DownArgs a) {
   constexpr int RPI = 64 / CP, NR = W8DC_ROWS / RPI;  // rows per load, loads per tile
   constexpr int KM = CP * 32, GM = KM / 128, NPC = (KM + 1023) / 1024;
-  __shared__ float s_o[33][W8DC_ROWS];
-  __shared__ __attribute__((aligned(16))) uint8_t s_q[16][KM];  // codes, W8 order
-  __shared__ float s_sq[16][GM], s_term[16][W8DC_ROWS][GM];
+  __shared__ float s_o[33 * MT][W8DC_ROWS];
+  __shared__ __attribute__((aligned(16))) uint8_t s_q[MT == 1 ? 16 : 1][KM];  // codes, W8 order
+  __shared__ float s_sq[MT == 1 ? 16 : 1][GM], s_term[16][MT][W8DC_ROWS][GM];
+  __shared__ float s_wt[MT > 1 ? 32 * MT : 1];
+  __shared__ int s_inv[MT > 1 ? 32 * MT : 1];
   const int tx = tid_opaque();
   const int wave = __builtin_amdgcn_readfirstlane(tx >> 6), lane = tx & 63;
-  const int nw = blockDim.x >> 6, k = a.k, H = a.H;
+  const int nw = blockDim.x >> 6, k = a.k, H = a.H, T = MT == 1 ? 1 : a.T;
   const int row0 = blockIdx.x * W8DC_ROWS;
+  // what the combine needs, requested before the weights
+  const int ct = lane / W8DC_ROWS, cr = lane % W8DC_ROWS;  // wave 0: token and row of this lane
   float wj = 0.f, rv = 0.f, sgv = 0.f;
   int pj = 0;
   bool bad = false;
+  if (MT > 1 && tx < T * k) {
+    wj = a.wt[tx];
+    pj = a.inv[tx];
+  }
   if (wave == 0) {
-    wj = a.wt[min(lane, k - 1)];
-    pj = a.inv[min(lane, k - 1)];
-    sgv = a.sg[0];
-    if (a.resid) rv = bf16_to_f32(a.resid[row0 + (lane & (W8DC_ROWS - 1))]);
+    if constexpr (MT == 1) {
+      wj = a.wt[min(lane, k - 1)];
+      pj = a.inv[min(lane, k - 1)];
+    }
+    const int t = min(ct, T - 1);
+    sgv = a.sg[t];
+    if (a.resid) rv = bf16_to_f32(a.resid[(size_t)t * H + row0 + cr]);
     bad = *a.err != 0;
   }
   const int sub = lane / CP, c = lane % CP;
-  for (int tile = wave; tile < a.n_tiles; tile += nw) {
-    const bool shared = tile == k;
-    const size_t e = shared ? 0 : (size_t)a.tiles[tile].x;
+  const int n_tiles = MT == 1 ? a.max_tiles : min(a.max_tiles, *a.n_tiles);
+  for (int tile = wave; tile < n_tiles; tile += nw) {
+    // (MT = 1: tile j < k is one token of one expert at position j)
+    const int4 t4 = MT > 1 ? a.tiles[tile]
+                           : make_int4(tile == k ? a.E : a.tiles[tile].x, tile == k ? 0 : tile, 1, 0);
+    const bool shared = t4.x == a.E;
+    const size_t e = shared ? 0 : (size_t)t4.x;
+    const int pos0 = t4.y, mcnt = t4.z;
     const int K = shared ? a.Is : a.I, G = K >> 7, C = K >> 5;
     const uint8_t *w0 = (shared ? a.ws : a.w) + e * H * (K / 2);
     const uint16_t *s0 = (shared ? a.ss : a.s) + e * H * G;
+    const int cc = min(c, C - 1);
+    i32x4 xe[MT], xo[MT];
+    float sqg[MT];
     // act first: its quantization must not wait for the weights
-    const float *act = shared ? a.act_s : a.act + (size_t)tile * K;
-    float4 av[NPC][4];
+    float4 av[MT == 1 ? NPC : 1][4];
+    if constexpr (MT == 1) {
+      const float *act = shared ? a.act_s : a.act + (size_t)pos0 * K;
 #pragma unroll
-    for (int p = 0; p < NPC; ++p)
+      for (int p = 0; p < NPC; ++p)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        av[p][i] = *(const float4 *)(act + min(1024 * p + 16 * lane + 4 * i, K - 4));
+        for (int i = 0; i < 4; ++i)
+          av[p][i] = *(const float4 *)(act + min(1024 * p + 16 * lane + 4 * i, K - 4));
+    } else {
+      const W8Rows &src = shared ? a.q_s : a.q;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const size_t row = (size_t)(pos0 + min(t, mcnt - 1));
+        xe[t] = *(const i32x4 *)(src.q + row * K + cc * 32);
+        xo[t] = *(const i32x4 *)(src.q + row * K + cc * 32 + 16);
+        sqg[t] = src.s[row * G + (cc >> 2)];
+      }
+    }
     uint16_t sc[NR];
     u32x4 wv[NR];
 #pragma unroll
@@ -605,135 +634,158 @@ __global__ __launch_bounds__(1024) void k_w4a8_down_combine_t1(W8DownT1Args a) {
       sc[r] = s0[row * G + min(c >> 2, G - 1)];
       wv[r] = __builtin_nontemporal_load((const u32x4 *)(w0 + row * (K / 2) + min(c, C - 1) * 16));
     }
+    if constexpr (MT == 1) {
 #pragma unroll
-    for (int p = 0; p < NPC; ++p) {
-      const int e0 = 1024 * p + 16 * lane;
-      float m = 0.0f;
+      for (int p = 0; p < NPC; ++p) {
+        const int e0 = 1024 * p + 16 * lane;
+        float m = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float f[4] = {av[p][i].x, av[p][i].y, av[p][i].z, av[p][i].w};
+        for (int i = 0; i < 4; ++i) {
+          const float f[4] = {av[p][i].x, av[p][i].y, av[p][i].z, av[p][i].w};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float ab = fabsf(f[j]);
-          m = ab > m ? ab : m;
+          for (int j = 0; j < 4; ++j) {
+            const float ab = fabsf(f[j]);
+            m = ab > m ? ab : m;
+          }
+        }
+        // the group's 8 lanes
+#pragma unroll
+        for (int o = 4; o >= 1; o >>= 1)
+          m = __uint_as_float(max(__float_as_uint(m), (uint32_t)__shfl_xor((int)__float_as_uint(m), o, 64)));
+        float q1 = m / 127.0f;
+        q1 = q1 == 0.0f ? 1.0f : q1;
+        uint32_t pk[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float f[4] = {av[p][i].x, av[p][i].y, av[p][i].z, av[p][i].w};
+          pk[i] = 0;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float r = f[j] / q1;
+            int qi = (int)(r >= 0.0f ? r + 0.5f : r - 0.5f);
+            qi = qi < -127 ? -127 : (qi > 127 ? 127 : qi);
+            pk[i] |= (uint32_t)(uint8_t)(int8_t)qi << (8 * j);
+          }
+        }
+        if (e0 < K) {
+          // half a 32-element block: its 8 even elements, its 8 odd ones
+          uint8_t *qd = s_q[wave] + (e0 >> 5) * 32 + ((lane & 1) ? 8 : 0);
+          *(uint2 *)qd = make_uint2(__builtin_amdgcn_perm(pk[1], pk[0], 0x06040200u),
+                                    __builtin_amdgcn_perm(pk[3], pk[2], 0x06040200u));
+          *(uint2 *)(qd + 16) = make_uint2(__builtin_amdgcn_perm(pk[1], pk[0], 0x07050301u),
+                                           __builtin_amdgcn_perm(pk[3], pk[2], 0x07050301u));
+          if ((lane & 7) == 0) s_sq[wave][e0 >> 7] = q1;
         }
       }
-      // the group's 8 lanes
-#pragma unroll
-      for (int o = 4; o >= 1; o >>= 1)
-        m = __uint_as_float(max(__float_as_uint(m), (uint32_t)__shfl_xor((int)__float_as_uint(m), o, 64)));
-      float q1 = m / 127.0f;
-      q1 = q1 == 0.0f ? 1.0f : q1;
-      uint32_t pk[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float f[4] = {av[p][i].x, av[p][i].y, av[p][i].z, av[p][i].w};
-        pk[i] = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float r = f[j] / q1;
-          int qi = (int)(r >= 0.0f ? r + 0.5f : r - 0.5f);
-          qi = qi < -127 ? -127 : (qi > 127 ? 127 : qi);
-          pk[i] |= (uint32_t)(uint8_t)(int8_t)qi << (8 * j);
-        }
-      }
-      if (e0 < K) {
-        // half a 32-element block: its 8 even elements, its 8 odd ones
-        uint8_t *qd = s_q[wave] + (e0 >> 5) * 32 + ((lane & 1) ? 8 : 0);
-        *(uint2 *)qd = make_uint2(__builtin_amdgcn_perm(pk[1], pk[0], 0x06040200u),
-                                  __builtin_amdgcn_perm(pk[3], pk[2], 0x06040200u));
-        *(uint2 *)(qd + 16) = make_uint2(__builtin_amdgcn_perm(pk[1], pk[0], 0x07050301u),
-                                         __builtin_amdgcn_perm(pk[3], pk[2], 0x07050301u));
-        if ((lane & 7) == 0) s_sq[wave][e0 >> 7] = q1;
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const int cc = min(c, C - 1);
-    const i32x4 xe = *(const i32x4 *)(s_q[wave] + cc * 32), xo = *(const i32x4 *)(s_q[wave] + cc * 32 + 16);
-    const float sqg = s_sq[wave][cc >> 2];
-    int sx = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      sx = __builtin_amdgcn_sdot4(xe[j], 0x01010101, sx, false);
-      sx = __builtin_amdgcn_sdot4(xo[j], 0x01010101, sx, false);
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      xe[0] = *(const i32x4 *)(s_q[wave] + cc * 32);
+      xo[0] = *(const i32x4 *)(s_q[wave] + cc * 32 + 16);
+      sqg[0] = s_sq[wave][cc >> 2];
     }
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      int d = -8 * sx;
+    for (int t = 0; t < MT; ++t) {
+      if (t >= mcnt) break;
+      int sx = 0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint32_t u = wv[r][j] ^ 0x88888888u;  // nibble q -> q + 8
-        d = __builtin_amdgcn_sdot4((int)(u & 0x0F0F0F0Fu), xe[j], d, false);
-        d = __builtin_amdgcn_sdot4((int)((u >> 4) & 0x0F0F0F0Fu), xo[j], d, false);
+        sx = __builtin_amdgcn_sdot4(xe[t][j], 0x01010101, sx, false);
+        sx = __builtin_amdgcn_sdot4(xo[t][j], 0x01010101, sx, false);
       }
-      d += __builtin_amdgcn_mov_dpp(d, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
-      d += __builtin_amdgcn_mov_dpp(d, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
-      if ((c & 3) == 0 && c < C) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        int d = -8 * sx;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t u = wv[r][j] ^ 0x88888888u;  // nibble q -> q + 8
+          d = __builtin_amdgcn_sdot4((int)(u & 0x0F0F0F0Fu), xe[t][j], d, false);
+          d = __builtin_amdgcn_sdot4((int)((u >> 4) & 0x0F0F0F0Fu), xo[t][j], d, false);
+        }
+        d += __builtin_amdgcn_mov_dpp(d, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
+        d += __builtin_amdgcn_mov_dpp(d, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
+        if ((c & 3) == 0 && c < C) {
 #pragma clang fp contract(off)
-        s_term[wave][r * RPI + sub][c >> 2] = (float)d * scale_to_f32<SD>(sc[r]) * sqg;  // unfused
+          s_term[wave][t][r * RPI + sub][c >> 2] = (float)d * scale_to_f32<SD>(sc[r]) * sqg[t];  // unfused
+        }
       }
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    if (lane < W8DC_ROWS) {
+    if (lane < W8DC_ROWS * mcnt) {
 #pragma clang fp contract(off)
       float acc = 0.0f;
-      for (int g = 0; g < G; ++g) acc = acc + s_term[wave][lane][g];  // group order
-      s_o[tile][lane] = acc;
+      for (int g = 0; g < G; ++g) acc = acc + s_term[wave][MT == 1 ? 0 : ct][cr][g];  // group order
+      s_o[(shared ? T * k : 0) + pos0 + ct][cr] = acc;
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  if (MT > 1 && tx < T * k) {
+    s_wt[tx] = wj;
+    s_inv[tx] = pj;
   }
   __syncthreads();
   if (wave != 0) return;
-  const int r = lane & (W8DC_ROWS - 1);
   float acc = 0.f;
-  for (int j = 0; j < k; ++j) {
-    const int p = __builtin_amdgcn_readlane(pj, j);
-    acc = __builtin_fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wj), j)), s_o[p][r], acc);
+  if constexpr (MT == 1) {
+    for (int j = 0; j < k; ++j)  // lane j holds slot j's weight and position
+      acc = __builtin_fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wj), j)),
+                           s_o[__builtin_amdgcn_readlane(pj, j)][cr], acc);
   }
-  if (a.n_tiles > k) acc = __builtin_fmaf(sgv, s_o[k][r], acc);
+  if (ct >= T) return;
+  if constexpr (MT > 1)
+    for (int j = 0; j < k; ++j) acc = __builtin_fmaf(s_wt[ct * k + j], s_o[s_inv[ct * k + j]][cr], acc);
+  if (a.Is > 0) acc = __builtin_fmaf(sgv, s_o[T * k + ct][cr], acc);
   if (a.resid) acc += rv;
-  if (lane < W8DC_ROWS) a.y[row0 + lane] = bad ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
+  a.y[(size_t)ct * H + row0 + cr] = bad ? (uint16_t)0x7FC0u : f32_to_bf16(acc);
 }
 
 }  // namespace
 
-hipError_t launch_w4a8_down_combine_t1(int scale_dtype, const W4A8Args &d, const float *w,
-                                       const float *sg, const int32_t *inv, const void *resid,
-                                       void *y, const int32_t *err, hipStream_t s) {
+hipError_t launch_w4a8_down_combine(int scale_dtype, const W4A8Args &d, const W8Rows &q,
+                                    const W8Rows &q_s, const float *w, const float *sg,
+                                    const int32_t *inv, const void *resid, void *y,
+                                    const int32_t *err, hipStream_t s) {
   const int Kmax = d.I > d.Is ? d.I : d.Is;
-  if (d.T != 1 || d.k > 32 || d.H % W8DC_ROWS || Kmax > W8DC_MAX_K) return hipErrorInvalidValue;
-  W8DownT1Args a;
+  if (d.T < 1 || d.T > DC_MAX_T || d.k > 32 || d.H % W8DC_ROWS || Kmax > W8DC_MAX_K)
+    return hipErrorInvalidValue;
+  W8DownArgs a;
   a.w = d.w0;
   a.ws = d.ws0;
   a.s = d.s0;
   a.ss = d.ss0;
   a.act = d.act;
   a.act_s = d.act_s;
+  a.q = q;
+  a.q_s = q_s;
   a.tiles = d.tiles;
+  a.n_tiles = d.n_tiles;
   a.wt = w;
   a.sg = sg;
   a.inv = inv;
   a.resid = (const uint16_t *)resid;
   a.y = (uint16_t *)y;
   a.err = err;
+  a.T = d.T;
   a.k = d.k;
+  a.E = d.E;
   a.H = d.H;
   a.I = d.I;
   a.Is = d.Is;
-  a.n_tiles = d.k + (d.Is > 0 ? 1 : 0);
-  const int nw = a.n_tiles < 16 ? a.n_tiles : 16;
-  auto go = [&](auto sd_c) {
-    constexpr int SDc = decltype(sd_c)::value;
+  a.max_tiles = d.T * d.k + (d.Is > 0 ? 1 : 0);
+  const int nw = a.max_tiles < 16 ? a.max_tiles : 16;
+  auto go_cp = [&](auto sd_c, auto cp_c) {
+    constexpr int SDc = decltype(sd_c)::value, CPc = decltype(cp_c)::value;
     const dim3 g(d.H / W8DC_ROWS), b(nw * 64);
-    if (Kmax <= 512)
-      k_w4a8_down_combine_t1<SDc, 16><<<g, b, 0, s>>>(a);
-    else if (Kmax <= 1024)
-      k_w4a8_down_combine_t1<SDc, 32><<<g, b, 0, s>>>(a);
+    if (d.T == 1)
+      k_w4a8_down_combine<SDc, CPc, 1><<<g, b, 0, s>>>(a);
     else
-      k_w4a8_down_combine_t1<SDc, 64><<<g, b, 0, s>>>(a);
+      k_w4a8_down_combine<SDc, CPc, DC_MAX_T><<<g, b, 0, s>>>(a);
+  };
+  auto go = [&](auto sd_c) {
+    if (Kmax <= 512) go_cp(sd_c, std::integral_constant<int, 16>());
+    else if (Kmax <= 1024) go_cp(sd_c, std::integral_constant<int, 32>());
+    else go_cp(sd_c, std::integral_constant<int, 64>());
   };
   if (scale_dtype == AINFER_SCALE_FP16)
     go(std::integral_constant<int, AINFER_SCALE_FP16>());
@@ -768,46 +820,11 @@ hipError_t launch_w4a8_expert(int mode, int scale_dtype, const W4A8Args &a, int 
   if (max_tiles <= 0) return hipSuccess;
   const int N = mode == 0 ? (a.I > a.Is ? a.I : a.Is) : a.H;
   const int K = mode == 0 ? a.H : (a.I > a.Is ? a.I : a.Is);
-  const int Kmin = mode == 0 ? a.H : (a.Is > 0 && a.Is < a.I ? a.Is : a.I);
-  if (a.T == 1 && K <= 8192 && Kmin % 128 == 0) {
-    // one token per tile: the wide one-token rows (gemv1_rows)
-    const int nc = (K / 32 + 63) / 64;
-    const dim3 g1((N + GV1_WAVES * GV1_RW - 1) / (GV1_WAVES * GV1_RW), max_tiles);
-    // the in-kernel quantization needs whole blocks of rows and K <= 4096
-    const bool qin = mode == 1 && a.quant_in && a.H % (GV1_WAVES * GV1_RW) == 0 && K <= 4096;
-    if (mode == 1 && a.quant_in && !qin) {
-      hipError_t e = launch_act_quant_f32_pair(a.act, a.T * a.k, a.I, const_cast<int8_t *>(a.aq),
-                                               const_cast<float *>(a.as), a.Is > 0 ? a.act_s : nullptr,
-                                               a.T, a.Is, const_cast<int8_t *>(a.aq_s),
-                                               const_cast<float *>(a.as_s), s);
-      if (e != hipSuccess) return e;
-    }
-    auto go1 = [&](auto sd_c, auto nc_c) {
-      constexpr int SDc = decltype(sd_c)::value, NCc = decltype(nc_c)::value;
-      if (mode == 0)
-        k_w4a8_expert_t1<SDc, 0, NCc><<<g1, GV1_WAVES * 64, 0, s>>>(a);
-      else if (qin)
-        k_w4a8_expert_t1<SDc, 1, NCc, true><<<g1, GV1_WAVES * 64, 0, s>>>(a);
-      else
-        k_w4a8_expert_t1<SDc, 1, NCc><<<g1, GV1_WAVES * 64, 0, s>>>(a);
-    };
-    auto go_nc = [&](auto sd_c) {
-      if (nc == 1) go1(sd_c, std::integral_constant<int, 1>());
-      else if (nc == 2) go1(sd_c, std::integral_constant<int, 2>());
-      else if (nc == 3) go1(sd_c, std::integral_constant<int, 3>());
-      else go1(sd_c, std::integral_constant<int, 4>());
-    };
-    if (scale_dtype == AINFER_SCALE_FP16)
-      go_nc(std::integral_constant<int, AINFER_SCALE_FP16>());
-    else
-      go_nc(std::integral_constant<int, AINFER_SCALE_BF16>());
-    return hipGetLastError();
-  }
-  if (mode == 1 && a.quant_in) {
-    hipError_t e = launch_act_quant_f32_pair(a.act, a.T * a.k, a.I, const_cast<int8_t *>(a.aq),
-                                             const_cast<float *>(a.as), a.Is > 0 ? a.act_s : nullptr,
-                                             a.T, a.Is, const_cast<int8_t *>(a.aq_s),
-                                             const_cast<float *>(a.as_s), s);
+  if (mode == 1) {
+    hipError_t e = launch_act_quant_f32_pair(a.act, a.T * a.k, a.I, a.aq,
+                                             a.as, a.Is > 0 ? a.act_s : nullptr,
+                                             a.T, a.Is, a.aq_s,
+                                             a.as_s, s);
     if (e != hipSuccess) return e;
   }
   const dim3 grid((N + 15) / 16, max_tiles);
@@ -823,6 +840,33 @@ hipError_t launch_w4a8_expert(int mode, int scale_dtype, const W4A8Args &a, int 
     go(std::integral_constant<int, AINFER_SCALE_FP16>());
   else
     go(std::integral_constant<int, AINFER_SCALE_BF16>());
+  return hipGetLastError();
+}
+
+hipError_t launch_w4a8_expert_t1(int mode, int scale_dtype, const W4A8Args &a, int max_tiles,
+                                 hipStream_t s) {
+  if (max_tiles <= 0) return hipSuccess;
+  const int N = mode == 0 ? (a.I > a.Is ? a.I : a.Is) : a.H;
+  const int K = mode == 0 ? a.H : (a.I > a.Is ? a.I : a.Is);
+  // (MODE 1 quantizes in the kernel: whole blocks of rows and K <= 4096)
+  if (a.T != 1 || K > 4096 || a.H % (GV1_WAVES * GV1_RW)) return hipErrorInvalidValue;
+  const int nc = (K / 32 + 63) / 64;
+  const dim3 g1((N + GV1_WAVES * GV1_RW - 1) / (GV1_WAVES * GV1_RW), max_tiles);
+  auto go1 = [&](auto sd_c, auto nc_c) {
+    constexpr int SDc = decltype(sd_c)::value, NCc = decltype(nc_c)::value;
+    if (mode == 0)
+      k_w4a8_expert_t1<SDc, 0, NCc><<<g1, GV1_WAVES * 64, 0, s>>>(a);
+    else
+      k_w4a8_expert_t1<SDc, 1, NCc><<<g1, GV1_WAVES * 64, 0, s>>>(a);
+  };
+  auto go_nc = [&](auto sd_c) {
+    if (nc == 1) go1(sd_c, std::integral_constant<int, 1>());
+    else go1(sd_c, std::integral_constant<int, 2>());
+  };
+  if (scale_dtype == AINFER_SCALE_FP16)
+    go_nc(std::integral_constant<int, AINFER_SCALE_FP16>());
+  else
+    go_nc(std::integral_constant<int, AINFER_SCALE_BF16>());
   return hipGetLastError();
 }
 

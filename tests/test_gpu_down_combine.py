@@ -89,24 +89,28 @@ def test_w4a8_block_of_a_narrow_row(torch, oracle, H):
 @pytest.mark.parametrize("H,E,k,I,Is", [(512, 8, 3, 128, 384), (1024, 40, 20, 512, 0),
                                         (4096, 12, 10, 1024, 256), (640, 9, 4, 896, 1792),
                                         (256, 5, 2, 2048, 128), (384, 4, 2, 2304, 256)])
-def test_w4a8_one_token_equals_its_row_of_two(torch, H, E, k, I, Is):
-    """In W4A8 a token's output is defined bit by bit: the T = 1 kernels
-    (down with the quantization and the combine in it up to I = 2048) give the
-    token's row of a T = 2 call, with and without the residual."""
+def test_w4a8_rows_do_not_depend_on_the_call(torch, oracle, H, E, k, I, Is):
+    """In W4A8 a token's output is defined bit by bit, so a token's row is the
+    same in calls of 1, 2, 3, 4, 5 and 16 tokens, which take different kernels
+    (the one-token GEMVs; the GEMM, or 16-row blocks where its items would be
+    few or long; down with the combine in it up to 4 tokens), with and without
+    the residual.  Against the oracle at the layer's tolerance."""
     from ainfer_amd import _lib as L
     from ainfer_amd.moe import MoeLayer, make_input
     from ainfer_amd.synthetic import MoeConfig
-    cfg = MoeConfig("w8dc", H, E, k, I, Is, (2,), seed=13)
+    cfg = MoeConfig("w8dc", H, E, k, I, Is, (16,), seed=13)
     for sd in (L.SCALE_FP16, L.SCALE_BF16):
-        print(f"[case] w4a8 T=1 H={H} E={E} k={k} I={I} Is={Is} scales={sd}", flush=True)
+        print(f"[case] w4a8 H={H} E={E} k={k} I={I} Is={Is} scales={sd}", flush=True)
         ly = MoeLayer(cfg, scale_dtype=sd, precision=L.PRECISION_W4A8)
-        x = make_input(cfg, 2, tag=3)
-        ws = ly.workspace(2)
-        two, one = torch.empty_like(x), torch.empty_like(x)
+        x = make_input(cfg, 16, tag=3)
+        ws = ly.workspace(16)
         for fn in (ly.forward, ly.block_forward):
-            fn(x, two, ws)
-            for t in range(2):
-                fn(x[t:t + 1], one[t:t + 1], ws)
-            torch.cuda.synchronize()
-            assert torch.isfinite(two.float()).all()
-            assert torch.equal(one.view(torch.int16), two.view(torch.int16)), fn.__name__
+            want, got = torch.empty_like(x), torch.empty_like(x)
+            fn(x, want, ws)
+            for n in (1, 2, 3, 4, 5):
+                for t in range(0, 16, n):
+                    fn(x[t:t + n], got[t:t + n], ws)
+                torch.cuda.synchronize()
+                assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (fn.__name__, n)
+            if fn == ly.forward:
+                check_close(to_np(want), host_copy(oracle, ly).forward_w4a8(to_np(x), 16), "w4a8 16")
