@@ -522,23 +522,44 @@ __global__ __launch_bounds__(64 * WN, 2) void k_expert_gemm(GemmArgs a) {
 
 // ---------------------------------------------------------------------------
 // Router logits for prefill: approx[t][e] = sum_k x[t][k] * w[e][k] (+ bias)
-// on bf16 MFMA, fp32 accumulation.  Block tile: 64 tokens x 128 experts,
-// 4 waves as 2 (tokens) x 2 (experts), each 32 x 64 = 2 x 4 MFMA tiles.  K
-// streams through a 3-stage LDS ring in 64-wide steps (x rows and w rows,
-// 128 bytes each, 16-byte chunk c of row r stored at c ^ (r & 7)).  The
-// blocks after the GEMM tiles compute ||w_e|| (used only as the bound of
-// the canonical refine).
+// on bf16 MFMA, fp32 accumulation.  Block tile: BM tokens x BN experts, 4 waves
+// as 2 (tokens) x 2 (experts).  K streams through an LDS ring of ST stages in
+// 64-wide steps (x rows and w rows, 128 bytes each, 16-byte chunk c of row r
+// stored at c ^ (r & 7)).  The blocks after the GEMM tiles compute ||w_e||
+// (used only as the bound of the canonical refine).
+//
+// A block is a serial chain of H / 64 steps, each a barrier, the DMA issue, the
+// LDS reads and the MFMAs of one wave per SIMD, so a step costs what its tile
+// moves (64 x 128: 0.62 us, 64 x 64: 0.41, 32 x 64: 0.30) and a deeper ring
+// changes nothing (3 and 6 stages: 20.2, 20.6 us).  Hence the smallest tile whose
+// items still have a CU each, and the largest, which reads the least, once none
+// has.  us with 64 x 128 always -> now: E512 H2048 T512 19.5 -> 10.4 (32 x 64),
+// T1024 20.1 -> 11.2, T1500 20.5 -> 13.6 (64 x 64; 32 x 64: 15.9), T2048 20.9 ->
+// 14.9, T4096 23.0 -> 22.1 (64 x 128; 64 x 64: 24.9, 32 x 64: 29.6); E96 H2560 T301
+// 24.4 -> 12.0.
 // ---------------------------------------------------------------------------
-#ifndef RG_BM_
-#define RG_BM_ 64
-#endif
-constexpr int RG_BM = RG_BM_, RG_BN = 128, RG_BK = 64, RG_ST = 3;
-constexpr int RG_MS = RG_BM / 32;  // 16-token MFMA rows per wave
-constexpr int RG_A = RG_BM * RG_BK * 2, RG_B = RG_BN * RG_BK * 2;  // bytes per stage
-constexpr int RG_STAGE = RG_A + RG_B;
-constexpr int RG_DMA = RG_STAGE / (256 * 16);  // per thread per stage: 6
+constexpr int RG_BK = 64;
+constexpr int RG_FILL = 256;  // items that leave no CU idle
 constexpr int RG_NORM_ROWS = 16;                // experts per norm block
 
+template <int BM, int BN, int ST>
+struct RouterGeo {
+  static constexpr int A = BM * RG_BK * 2, STAGE = A + BN * RG_BK * 2;  // bytes
+  static constexpr int DMA = STAGE / (256 * 16);                       // per thread per stage
+  static constexpr int LDS = ST * STAGE;
+  static_assert((ST - 2) * DMA < 64, "vmcnt");
+};
+
+// all but the newest N * D of this wave's DMAs done (n <= N, wave-uniform)
+template <int D, int N>
+__device__ __forceinline__ void wait_stages(int n) {
+  if constexpr (N > 0) {
+    if (n < N) return wait_stages<D, N - 1>(n);
+  }
+  wait_vm<N * D>();
+}
+
+template <int BM, int BN, int ST>
 __global__ __launch_bounds__(256) void k_router_gemm(const uint16_t *__restrict__ x,
                                                      const uint16_t *__restrict__ rw,
                                                      const float *__restrict__ bias,
@@ -546,6 +567,8 @@ __global__ __launch_bounds__(256) void k_router_gemm(const uint16_t *__restrict_
                                                      float *__restrict__ wnorm, int T, int H,
                                                      int E, int n_mt, int n_nt,
                                                      uint32_t *__restrict__ zbuf, int zwords) {
+  using Rg = RouterGeo<BM, BN, ST>;
+  constexpr int MS = BM / 32, NS = BN / 32;  // 16-row MFMA tiles per wave
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -577,80 +600,73 @@ __global__ __launch_bounds__(256) void k_router_gemm(const uint16_t *__restrict_
   }
   const int lb = xcd_remap(blockIdx.x, n_items);
   const int mt = lb / n_nt, nt = lb % n_nt;  // the n_nt expert tiles of a token tile share an XCD
-  const int t0 = mt * RG_BM, e0 = nt * RG_BN;
+  const int t0 = mt * BM, e0 = nt * BN;
   const int wm = wave & 1, wn = wave >> 1;
   const int m16 = lane & 15, q = lane >> 4;
   const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
 
   // DMA sources: slot s = (i*4 + wave)*64 + lane; row s/8, stored chunk s%8
-  const uint8_t *src[RG_DMA];
+  const uint8_t *src[Rg::DMA];
 #pragma unroll
-  for (int i = 0; i < RG_DMA; ++i) {
+  for (int i = 0; i < Rg::DMA; ++i) {
     const int sl = (i * 4 + wave) * 64 + lane;
     const int r = sl >> 3, c = (sl & 7) ^ (r & 7);
-    if (r < RG_BM) {
+    if (r < BM) {
       src[i] = (const uint8_t *)(x + (size_t)min(t0 + r, T - 1) * H) + c * 16;
     } else {
-      src[i] = (const uint8_t *)(rw + (size_t)min(e0 + r - RG_BM, E - 1) * H) + c * 16;
+      src[i] = (const uint8_t *)(rw + (size_t)min(e0 + r - BM, E - 1) * H) + c * 16;
     }
   }
   auto issue = [&](int g) {
-    const uint32_t base = lds0 + (uint32_t)(g % RG_ST) * RG_STAGE;
+    const uint32_t base = lds0 + (uint32_t)(g % ST) * Rg::STAGE;
 #pragma unroll
-    for (int i = 0; i < RG_DMA; ++i)
+    for (int i = 0; i < Rg::DMA; ++i)
       dma16(src[i] + g * (RG_BK * 2), base + (uint32_t)((i * 4 + wave) * 1024));
   };
   const int G = H / RG_BK;
-  issue(0);
-  if (G > 1) issue(1);
-  f32x4 acc[RG_MS][4];
+  for (int g = 0; g < min(ST - 1, G); ++g) issue(g);
+  f32x4 acc[MS][NS];
 #pragma unroll
-  for (int ms = 0; ms < RG_MS; ++ms)
+  for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-    for (int ns = 0; ns < 4; ++ns) acc[ms][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ns = 0; ns < NS; ++ns) acc[ms][ns] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int g = 0; g < G; ++g) {
-    if (g + 2 < G) {
-      issue(g + 2);
-      wait_vm<2 * RG_DMA>();
-    } else if (g + 1 < G) {
-      wait_vm<RG_DMA>();
-    } else {
-      wait_vm<0>();
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    // stage g is there for every wave, and stage g - 1 read by every wave: its
+    // place takes stage g + ST - 1
+    wait_stages<Rg::DMA, ST - 2>(min(ST - 2, G - 1 - g));
     block_barrier();
-    const uint8_t *sa = lds + (g % RG_ST) * RG_STAGE, *sb = sa + RG_A;
+    if (g + ST - 1 < G) issue(g + ST - 1);
+    const uint8_t *sa = lds + (g % ST) * Rg::STAGE, *sb = sa + Rg::A;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {  // two 32-wide MFMA steps
-      u32x4 af[RG_MS], bf[4];
+      u32x4 af[MS], bf[NS];
 #pragma unroll
-      for (int ms = 0; ms < RG_MS; ++ms) {
-        const int r = wm * (RG_BM / 2) + ms * 16 + m16;
+      for (int ms = 0; ms < MS; ++ms) {
+        const int r = wm * (BM / 2) + ms * 16 + m16;
         af[ms] = *(const u32x4 *)(sa + r * 128 + (((4 * s2 + q) ^ (r & 7)) << 4));
       }
 #pragma unroll
-      for (int ns = 0; ns < 4; ++ns) {
-        const int r = wn * 64 + ns * 16 + m16;
+      for (int ns = 0; ns < NS; ++ns) {
+        const int r = wn * (BN / 2) + ns * 16 + m16;
         bf[ns] = *(const u32x4 *)(sb + r * 128 + (((4 * s2 + q) ^ (r & 7)) << 4));
       }
 #pragma unroll
-      for (int ms = 0; ms < RG_MS; ++ms)
+      for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-        for (int ns = 0; ns < 4; ++ns) acc[ms][ns] = mfma_bf16_16x16x32(af[ms], bf[ns], acc[ms][ns]);
+        for (int ns = 0; ns < NS; ++ns) acc[ms][ns] = mfma_bf16_16x16x32(af[ms], bf[ns], acc[ms][ns]);
     }
-    block_barrier();  // stage g may be overwritten by the DMA issued next iteration
   }
   // lane (q, m16) of tile (ms, ns): tokens wm*32 + ms*16 + 4q + r, expert wn*64 + ns*16 + m16
 #pragma unroll
-  for (int ns = 0; ns < 4; ++ns) {
-    const int e = e0 + wn * 64 + ns * 16 + m16;
+  for (int ns = 0; ns < NS; ++ns) {
+    const int e = e0 + wn * (BN / 2) + ns * 16 + m16;
     if (e >= E) continue;
     const float b = bias ? bias[e] : 0.0f;
 #pragma unroll
-    for (int ms = 0; ms < RG_MS; ++ms)
+    for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int t = t0 + wm * (RG_BM / 2) + ms * 16 + 4 * q + r;
+        const int t = t0 + wm * (BM / 2) + ms * 16 + 4 * q + r;
         if (t < T) approx[(size_t)t * E + e] = bias ? acc[ms][ns][r] + b : acc[ms][ns][r];
       }
   }
@@ -685,13 +701,20 @@ hipError_t launch_router_gemm(const void *x, const void *rw, const float *bias, 
                               hipStream_t s) {
   if (T <= 0) return hipSuccess;
   if (H % RG_BK) return hipErrorInvalidValue;
-  const int n_mt = (T + RG_BM - 1) / RG_BM, n_nt = (E + RG_BN - 1) / RG_BN;
   const int n_norm = (E + RG_NORM_ROWS - 1) / RG_NORM_ROWS;
-  const long grid = (long)n_mt * n_nt + n_norm;
-  if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
-  k_router_gemm<<<(unsigned)grid, 256, RG_ST * RG_STAGE, s>>>(
-      (const uint16_t *)x, (const uint16_t *)rw, bias, approx, wnorm, T, H, E, n_mt, n_nt,
-      zbuf, zbuf ? zwords : 0);
+  auto launch = [&](auto kern, int bm, int bn, int lds) {
+    const int n_mt = (T + bm - 1) / bm, n_nt = (E + bn - 1) / bn;
+    kern<<<(unsigned)(n_mt * n_nt + n_norm), 256, lds, s>>>(
+        (const uint16_t *)x, (const uint16_t *)rw, bias, approx, wnorm, T, H, E, n_mt, n_nt,
+        zbuf, zbuf ? zwords : 0);
+  };
+  const long m32 = (T + 31) / 32, m64 = (T + 63) / 64, n64 = (E + 63) / 64;
+  if (m32 * n64 <= RG_FILL)
+    launch(k_router_gemm<32, 64, 4>, 32, 64, RouterGeo<32, 64, 4>::LDS);
+  else if (m64 * n64 <= RG_FILL)
+    launch(k_router_gemm<64, 64, 4>, 64, 64, RouterGeo<64, 64, 4>::LDS);
+  else
+    launch(k_router_gemm<64, 128, 3>, 64, 128, RouterGeo<64, 128, 3>::LDS);
   return hipGetLastError();
 }
 

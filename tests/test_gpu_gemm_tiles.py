@@ -160,3 +160,29 @@ def test_w4a8_gemm_gives_the_decode_rows(torch, H, E, k, I, Is, scales):
         ly.forward(x[:n], y, ws)
         torch.cuda.synchronize()
         assert torch.equal(y.view(torch.int16), want[:n].view(torch.int16)), n
+
+
+@pytest.mark.parametrize("H,E,T", [(128, 96, 257), (256, 512, 511), (256, 512, 1025), (128, 512, 2048),
+                                   (384, 500, 2049), (2560, 64, 300), (4096, 40, 256)])
+def test_router_at_tile_edges(torch, oracle, H, E, T):
+    """The prefill router at the edges of its GEMM tiles (32 x 64, 64 x 64, 64 x
+    128 of tokens x experts, the first and last count of items of each; K of 2
+    to 64 steps): the selection is canonical, so indices are the oracle's, and
+    the weights and gate differ by expf (an ulp on each side), the sum of 6 and a
+    division: below 16 ulps, 2^-19.  Columns with
+    one bias and equal experts make ties, which the smaller index wins."""
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    from test_gpu_parity import host_copy, to_np
+    print(f"[case] router tiles H={H} E={E} T={T}", flush=True)
+    cfg = MoeConfig("rt", H, E, 6, 128, 128, (T,), seed=5)
+    ly = MoeLayer(cfg)
+    rw = ly.t["router_w"].view(E, H)
+    rw[1::7] = rw[0]
+    x = make_input(cfg, T)
+    idx, w, sg, _ = ly.route(x, ly.workspace(T))
+    torch.cuda.synchronize()
+    r_idx, r_w, r_sg, _ = host_copy(oracle, ly).route(to_np(x), T)
+    assert np.array_equal(idx.cpu().numpy(), r_idx)
+    np.testing.assert_allclose(w.cpu().numpy(), r_w, rtol=2.0 ** -19, atol=0)
+    np.testing.assert_allclose(sg.cpu().numpy(), r_sg, rtol=2.0 ** -19, atol=0)
