@@ -28,6 +28,7 @@
 
 #include "moe_common.h"
 #include "moe_dispatch.h"
+#include "moe_gemm_parts.h"
 #include "moe_topk.h"
 #include "moe_internal.h"
 
@@ -131,84 +132,76 @@ __global__ __launch_bounds__(1024) void k_router_mfma(const uint16_t *__restrict
 }
 
 // ---------------------------------------------------------------------------
-// canonical dot: x in registers (lane l holds chunks l, l+64, ...), one
-// router row w; sequential fma in chunk order, then the xor butterfly.
+// Canonical dots of 4 router rows with x in registers (lane l holds chunks l,
+// l + 64, ...): per lane sequential fma in chunk order, then the xor butterfly
+// 32, 16, ..., 1 of every row.  All rows' loads are issued before any math.  The
+// butterfly halves the values at 32 and 16 (permlane swaps: lanes 16 b .. 16 b +
+// 15 end with row b) and goes on inside the 16 lanes on the DPP path, 7 steps for
+// the 4 rows where 24 ds_bpermutes did the same additions.  Returns row lane / 16.
 // ---------------------------------------------------------------------------
+constexpr int SEL_NB = 4;
 template <int CH>
-__device__ __forceinline__ float canon_dot(const u32x4 (&xc)[CH], const uint16_t *w, int lane,
-                                           int nch) {
-  u32x4 wv[CH];
+__device__ __forceinline__ float canon_dot4(const u32x4 (&xc)[CH], const uint16_t *const (&w)[SEL_NB],
+                                            int lane, int nch) {
+  u32x4 wv[SEL_NB][CH];
 #pragma unroll
-  for (int j = 0; j < CH; ++j) {
-    const int c = min(lane + 64 * j, nch - 1);
-    wv[j] = *(const u32x4 *)(w + (size_t)c * 8);
-  }
-  float acc = 0.0f;
+  for (int b = 0; b < SEL_NB; ++b)
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      wv[b][j] = *(const u32x4 *)(w[b] + (size_t)min(lane + 64 * j, nch - 1) * 8);
+  float v[SEL_NB];
+#pragma unroll
+  for (int b = 0; b < SEL_NB; ++b) v[b] = 0.0f;
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
     if (lane + 64 * j < nch) {
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        acc = __builtin_fmaf(__uint_as_float(xc[j][d] << 16), __uint_as_float(wv[j][d] << 16), acc);
-        acc = __builtin_fmaf(__uint_as_float(xc[j][d] & 0xFFFF0000u),
-                             __uint_as_float(wv[j][d] & 0xFFFF0000u), acc);
-      }
-    }
-  }
+        const float lo = __uint_as_float(xc[j][d] << 16), hi = __uint_as_float(xc[j][d] & 0xFFFF0000u);
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) acc = acc + __shfl_xor(acc, m, 64);
-  return acc;
-}
-
-// NB canonical dots at once (loads of all rows issued before any math);
-// rows past nrows repeat the last row and their results are ignored.
-template <int CH, int NB>
-__device__ __forceinline__ void canon_dot_batch(const u32x4 (&xc)[CH], const uint16_t *const (&w)[NB],
-                                                int lane, int nch, float (&out)[NB]) {
-  u32x4 wv[NB][CH];
-#pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int j = 0; j < CH; ++j) {
-      const int c = min(lane + 64 * j, nch - 1);
-      wv[b][j] = *(const u32x4 *)(w[b] + (size_t)c * 8);
-    }
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int j = 0; j < CH; ++j) {
-      if (lane + 64 * j < nch) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          acc = __builtin_fmaf(__uint_as_float(xc[j][d] << 16), __uint_as_float(wv[b][j][d] << 16), acc);
-          acc = __builtin_fmaf(__uint_as_float(xc[j][d] & 0xFFFF0000u),
-                               __uint_as_float(wv[b][j][d] & 0xFFFF0000u), acc);
+        for (int b = 0; b < SEL_NB; ++b) {
+          v[b] = __builtin_fmaf(lo, __uint_as_float(wv[b][j][d] << 16), v[b]);
+          v[b] = __builtin_fmaf(hi, __uint_as_float(wv[b][j][d] & 0xFFFF0000u), v[b]);
         }
       }
     }
-    out[b] = acc;
   }
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1)
-#pragma unroll
-    for (int b = 0; b < NB; ++b) out[b] = out[b] + __shfl_xor(out[b], m, 64);
+  HalveSum<4, 32>::step(v, lane);
+  HalveSum<2, 16>::step(v, lane);
+  float r = v[0];
+  auto mov = [](float f, auto ctrl, auto bank) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(f), __float_as_int(f),
+                                                      decltype(ctrl)::value, 0xF,
+                                                      decltype(bank)::value, false));
+  };
+  using std::integral_constant;
+  r = r + mov(r, integral_constant<int, 0x128>(), integral_constant<int, 0xF>());  // row_ror 8: xor 8
+  // xor 4: row_shl 4 (lane l takes l + 4) into the even quads, row_shr 4 into the odd ones
+  const float up = mov(r, integral_constant<int, 0x104>(), integral_constant<int, 0x5>());
+  const float dn = mov(r, integral_constant<int, 0x114>(), integral_constant<int, 0xA>());
+  r = r + ((lane & 4) ? dn : up);
+  r = r + mov(r, integral_constant<int, 0x4E>(), integral_constant<int, 0xF>());  // xor 2
+  r = r + mov(r, integral_constant<int, 0xB1>(), integral_constant<int, 0xF>());  // xor 1
+  return r;
 }
 
-
 constexpr int SEL_WAVES = 4;
-#ifndef SEL_NB
-#define SEL_NB 4  // candidate rows whose loads are issued together
-#endif
+constexpr int SEL_COOP_MAX_T = 1024;
 
-// COOP (T < GEMM_MIN_T, where one wave per token leaves most of the chip
-// idle and a token's latency is the kernel's): one token per workgroup.
-// Wave 0 takes the approximate top-k and the candidate list, wave 1 writes
-// the MFMA-order copy of x, wave 2 the shared-gate dot, and the candidates'
-// canonical dots are shared by all waves (c3 T=64: the dots were 13 of 25 us
-// per token).
+// One wave per token, SEL_WAVES tokens per workgroup; or COOP (up to
+// SEL_COOP_MAX_T, where one wave per token leaves most of the chip idle and a
+// token's latency is the kernel's): one token per workgroup.  Wave 0 takes the
+// approximate top-k and the candidate list, wave 1 writes the MFMA-order copy of
+// x, and the candidates' canonical dots and the shared gate's are shared by all
+// waves (E512 H2048 k10: T512 16.5 us by one wave per token, 9.5 COOP; T1500 17.1
+// and 18.8).
+// Bound by the latency of its serial parts at few tokens, by the reads of (k + 1)
+// router rows per token through the L2s at many.  With one shuffle chain per row,
+// the gate's dot on its own, x re-read after the top-k and lists of 1024 entries
+// (3 workgroups per CU): T64 17.3 us, T512 16.5, T1500 19.9, T4096 39; H4096 T4096
+// 105.  Now 14.4, 9.4, 17.0, 25.8 and 57.6.
 template <int NV, int CH, bool COOP>
-__global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx,
+__global__ __launch_bounds__(256, CH <= 4 ? 4 : 2) void k_select(const float *__restrict__ approx,
                                                 const float *__restrict__ wnorm,
                                                 const uint16_t *__restrict__ x,
                                                 const uint16_t *__restrict__ rw,
@@ -222,52 +215,53 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
                                                 int k, int H, int has_shared, DispatchOut ds,
                                                 int fused, unsigned long long *cmask,
                                                 int32_t *ccount) {
-  // candidate lists
-  __shared__ int cl[SEL_WAVES][1024];
-  __shared__ float cv[SEL_WAVES][1024];
-  __shared__ uint64_t s_cand[SEL_WAVES][64];
-  __shared__ uint64_t s_sel[SEL_WAVES][16];
+  // candidate lists (E <= 64 NV)
+  constexpr int LISTS = COOP ? 1 : SEL_WAVES;
+  __shared__ int cl[LISTS][64 * NV];
+  __shared__ float cv[LISTS][64 * NV + 1];  // and the shared gate's dot
+  __shared__ uint64_t s_cand[LISTS][64];
+  __shared__ uint64_t s_sel[LISTS][16];
   __shared__ int s_nc;
-  __shared__ float s_sgv;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int t = COOP ? (int)blockIdx.x : (int)blockIdx.x * SEL_WAVES + wave;
   const int sw = COOP ? 0 : wave;  // this wave's LDS lists
   const bool lead = !COOP || wave == 0;
   if (t < T) {
-    // the MFMA-order copy of x (and its group sums) does not depend on the
-    // routing: written first, its latency hides under the selection
+    // the routing's loads first, then the MFMA-order copy of x (and its group
+    // sums), which does not depend on it: its latency hides under the selection
     STRACE(0);
-    if ((xperm || w8.q) && (!COOP || wave == 1))
-      write_xperm(x + (size_t)t * H, xperm, xsum, t, H, lane, nullptr, 1.0f, w8.q, w8.s, w8.sum);
-    STRACE(1);
     const float *ar = approx + (size_t)t * E;
-    // ---- k-th largest approximate logit -------------------------------
+    const uint16_t *xrow = x + (size_t)t * H;
+    const int nch = H >> 3;
     uint32_t key[NV];
-    float wn = 0.0f;
+    float av[NV], wn = 0.0f;
+    u32x4 xc[CH];  // the x row in registers (canonical chunk layout)
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      if (!lead) break;
-      const int e = lane + 64 * i;
-      const float v = ar[min(e, E - 1)];  // unconditional: loads issue together
-      key[i] = e < E ? ordered_key(v) : 0u;
-      wn = fmaxf(wn, e < E ? wnorm[min(e, E - 1)] : 0.0f);
+      const int e = min(lane + 64 * i, E - 1);  // unconditional: loads issue together
+      av[i] = lead ? ar[e] : 0.0f;
+      wn = fmaxf(wn, lead ? wnorm[e] : 0.0f);
     }
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      xc[j] = *(const u32x4 *)(xrow + (size_t)min(lane + 64 * j, nch - 1) * 8);
+    if ((xperm || w8.q) && (!COOP || wave == 1))
+      write_xperm(xrow, xperm, xsum, t, H, lane, nullptr, 1.0f, w8.q, w8.s, w8.sum);
+    STRACE(1);
+    // ---- k-th largest approximate logit -------------------------------
+#pragma unroll
+    for (int i = 0; i < NV; ++i) key[i] = lane + 64 * i < E ? ordered_key(av[i]) : 0u;
     int seli = 0;
     uint32_t selk = 0u;
     if (lead) wave_topk_fast<NV>(key, E, k, lane, seli, selk, s_cand[sw], s_sel[sw]);
     STRACE(2);
-    const uint32_t kth = (uint32_t)__shfl((int)selk, k - 1, 64);
+    const uint32_t kth = (uint32_t)__builtin_amdgcn_readlane((int)selk, k - 1);
     float selv = 0.0f, sgv = 0.0f;
-    const uint16_t *xrow = x + (size_t)t * H;
     {
-      // ---- x row in registers (canonical chunk layout) and its norm ------
-      const int nch = H >> 3;
-      u32x4 xc[CH];
+      // ---- the row's norm (a bound: any order of the additions) -----------
       float xs = 0.0f;
 #pragma unroll
       for (int j = 0; j < CH; ++j) {
-        const int c = min(lane + 64 * j, nch - 1);
-        xc[j] = *(const u32x4 *)(xrow + (size_t)c * 8);
         if (lane + 64 * j < nch) {
 #pragma unroll
           for (int d = 0; d < 4; ++d) {
@@ -277,9 +271,10 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
           }
         }
       }
-      for (int m = 32; m >= 1; m >>= 1) xs += __shfl_xor(xs, m, 64);
-      if (COOP && wave == 2 && gw) s_sgv = canon_dot<CH>(xc, gw, lane, nch);
-      for (int m = 32; m >= 1; m >>= 1) wn = fmaxf(wn, __shfl_xor(wn, m, 64));
+      xs = row16_sum(xs);
+      xs += __shfl_xor(xs, 16, 64);
+      xs += __shfl_xor(xs, 32, 64);
+      wn = __uint_as_float(wave_max_u32(__float_as_uint(wn)));  // norms: not negative
       // ---- candidate threshold --------------------------------------------
       const float lk = key_to_float(kth);
       const float nrm = sqrtf(xs) * wn * 1.0625f;
@@ -304,22 +299,20 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
         nc = s_nc;
       }
       STRACE(3);
-      // ---- canonical logits of the candidates ------------------------------
+      // ---- canonical logits of the candidates, and the shared gate's -------
       {
-        const int cstep = COOP ? SEL_WAVES * SEL_NB : SEL_NB;
-        for (int c0 = COOP ? wave * SEL_NB : 0; c0 < nc; c0 += cstep) {
+        const int nr = nc + (gw ? 1 : 0), cstep = COOP ? SEL_WAVES * SEL_NB : SEL_NB;
+        for (int c0 = COOP ? wave * SEL_NB : 0; c0 < nr; c0 += cstep) {
           const uint16_t *rows[SEL_NB];
-          int ee[SEL_NB];
 #pragma unroll
           for (int b = 0; b < SEL_NB; ++b) {
-            ee[b] = cl[sw][min(c0 + b, nc - 1)];
-            rows[b] = rw + (size_t)ee[b] * H;
+            const int c = min(c0 + b, nr - 1);
+            const int e = __builtin_amdgcn_readfirstlane(cl[sw][max(min(c, nc - 1), 0)]);
+            rows[b] = c < nc ? rw + (size_t)e * H : gw;
           }
-          float v[SEL_NB];
-          canon_dot_batch<CH, SEL_NB>(xc, rows, lane, nch, v);
-#pragma unroll
-          for (int b = 0; b < SEL_NB; ++b)
-            if (lane == 0 && c0 + b < nc) cv[sw][c0 + b] = bias ? v[b] + bias[ee[b]] : v[b];
+          const float v = canon_dot4<CH>(xc, rows, lane, nch);
+          const int c = c0 + (lane >> 4);
+          if ((lane & 15) == 0 && c < nr) cv[sw][c] = bias && c < nc ? v + bias[cl[sw][c]] : v;
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -328,6 +321,10 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
       // ---- top-k among candidates (value desc, expert asc) ----------------
       if (!lead) {
         // helper waves are done
+      } else if (nc < k) {
+        // NaN in the row, the router or its norms: no threshold.  The
+        // approximate selection stands (valid experts).
+        selv = key_to_float(selk);
       } else if (nc <= 64 && k <= 16) {
         // rank of each candidate = candidates above it (unique composite keys)
         auto comp = [&](int i) {
@@ -335,7 +332,7 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
         };
         const uint64_t mine = lane < nc ? comp(lane) : 0ull;
         int rk = 0;
-        for (int j = 0; j < nc; ++j) rk += comp(j) > mine ? 1 : 0;
+        for (int j = 0; j < nc; ++j) rk += readlane_u64(mine, j) > mine ? 1 : 0;
         if (lane < nc && rk < k) s_sel[sw][rk] = ((uint64_t)(uint32_t)lane << 32) | (uint32_t)cl[sw][lane];
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -366,14 +363,15 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
       }
       }
       STRACE(5);
-      if (gw) sgv = COOP ? s_sgv : canon_dot<CH>(xc, gw, lane, nch);
+      if (gw) sgv = cv[sw][nc];
       STRACE(6);
     }
     if (lead) {
-      const float vmax = __shfl(selv, 0, 64);
+      const float vmax = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(selv), 0));
       const float p = lane < k ? expf(selv - vmax) : 0.0f;
       float sum = 0.0f;
-      for (int j = 0; j < k; ++j) sum += __shfl(p, j, 64);
+      for (int j = 0; j < k; ++j)
+        sum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), j));
       if (lane < k) {
         topk_idx[(size_t)t * k + lane] = seli;
         topk_w[(size_t)t * k + lane] = p / sum;
@@ -393,6 +391,7 @@ __global__ __launch_bounds__(256) void k_select(const float *__restrict__ approx
     }
     STRACE(7);
   }
+  if constexpr (!COOP) return;
   if (!fused) return;
   // ---- the last block runs the dispatch ---------------------------------
   __shared__ int is_last;
@@ -443,8 +442,9 @@ hipError_t launch_select(const float *approx, const float *wnorm,
   DispatchOut ds;
   memset(&ds, 0, sizeof ds);
   if (fused) ds = *fused;
-  // one token per workgroup below the GEMM path (k_select, COOP)
-  const bool coop = T < GEMM_MIN_T;
+  // one token per workgroup (k_select, COOP; it alone runs the fused dispatch)
+  if (fused && T > SEL_COOP_MAX_T) return hipErrorInvalidValue;
+  const bool coop = T <= SEL_COOP_MAX_T;
   const unsigned g = coop ? (unsigned)T : (T + SEL_WAVES - 1) / SEL_WAVES;
   const int fz = fused ? 1 : 0;
 #define SEL_CALL(NVV)                                                                          \
