@@ -638,8 +638,8 @@ bool stack_geometry(const ainfer_moe_shape &s, int T, StackGeom *g) {
   if (!expert_geometry(0, s.hidden, s.inter, s.shared_inter, 4, &kbw, &wk, &wr) || kbw != 4)
     return false;
   g->wk_gu = wk;
-  // down: the per-block path's K split at this token count (T <= 2: the
-  // fused expert kernel's KBW 2, else the stand-alone kernels' down_kbw)
+  // down: the per-block path's K split at this token count (T <= 2: KBW 2,
+  // else the stand-alone kernels' down_kbw)
   g->kbw_dn = T <= FUSED_EXPERTS_MAX_T ? 2 : down_kbw_of(s);
   if (!expert_geometry(1, s.hidden, s.inter, s.shared_inter, g->kbw_dn, &kbw, &wk, &wr) ||
       kbw != g->kbw_dn)

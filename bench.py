@@ -62,7 +62,7 @@ def gateup_bytes(cfg, U):
 
 
 def experts_bytes(cfg, U, T):
-    """Algorithmic bytes of the decode expert kernel (k_experts_decode): INT4
+    """Algorithmic bytes of the decode expert kernels: INT4
     nibbles + fp16 scales of gate, up and down for U routed experts and the
     shared expert, plus the bf16 tokens read and the bf16 outputs written."""
     per = lambda I: 3 * (cfg.hidden * I // 2 + cfg.hidden * I // 128 * 2)
@@ -194,7 +194,7 @@ def run_gemv_w4a8(steps, copies=8, M=17408, K=5120):
 
 def run_c3(steps, warmup=5):
     """H4096 E512 k10 I1024 + shared, 64 tokens (the
-    16-token-tile streaming kernels).  One layer is 3.3 GB, far above the
+    4-token-tile streaming kernels).  One layer is 3.3 GB, far above the
     256 MB MALL, so one copy suffices."""
     import torch
     from ainfer_amd.moe import MoeLayer, make_input

@@ -293,8 +293,8 @@ int ainfer_moe_dispatch(const ainfer_moe_shape *shape,
  * aligned; row t*k + j is expert topk_idx[t][j] applied to token t (gate/up,
  * SiLU-mul, down), row T*k + t the shared expert on token t (unused without
  * one).  The kernels and arithmetic of ainfer_moe_forward's expert stage at
- * the same T (for T <= 2 forward fuses the stages and splits K differently;
- * there the rows agree within the layer tolerance).  No reference counterpart
+ * the same T (for T <= 2 forward splits K differently; there the rows agree
+ * within the layer tolerance).  No reference counterpart
  * (the reference is dense); the per-expert MLP is decode_l0.cpp:663-674's. */
 int ainfer_moe_experts(const ainfer_moe_shape *shape,
                        const ainfer_moe_weights *weights, const void *x,
