@@ -9,7 +9,7 @@
 //  k_router_mfma: approximate logits on bf16 MFMA (products exact, fp32
 //    accumulation in the hardware's order) plus the 2-norm of every router
 //    weight row.
-//  k_select: one wave per token.  With L_k the k-th largest approximate
+//  k_select: one wave or one workgroup per token.  With L_k the k-th largest approximate
 //    logit and d >= |approx - exact| + |canonical - exact| for every expert,
 //    any expert whose canonical logit can reach the canonical top-k has
 //    approx >= L_k - 2d (the top-k experts by approx all have canonical >=

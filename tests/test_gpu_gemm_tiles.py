@@ -186,3 +186,28 @@ def test_router_at_tile_edges(torch, oracle, H, E, T):
     assert np.array_equal(idx.cpu().numpy(), r_idx)
     np.testing.assert_allclose(w.cpu().numpy(), r_w, rtol=2.0 ** -19, atol=0)
     np.testing.assert_allclose(sg.cpu().numpy(), r_sg, rtol=2.0 ** -19, atol=0)
+
+
+@pytest.mark.parametrize("T", [33, 300, 1100])
+def test_router_rows_without_a_threshold(torch, oracle, T):
+    """A token whose logits are NaN or infinite has no candidate threshold: its
+    experts are still k distinct valid ones, and every other row is the oracle's."""
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    from test_gpu_parity import host_copy, to_np
+    print(f"[case] router non-finite rows T={T}", flush=True)
+    E, k = 96, 6
+    cfg = MoeConfig("rn", 512, E, k, 128, 128, (T,), seed=6)
+    ly = MoeLayer(cfg)
+    x = make_input(cfg, T)
+    bad = [5, T - 1]
+    good = np.setdiff1d(np.arange(T), bad)
+    r_idx, _, _, _ = host_copy(oracle, ly).route(to_np(x), T)
+    x[5] = float("nan")
+    x[T - 1, 7] = float("inf")
+    idx, _, _, _ = ly.route(x, ly.workspace(T))
+    torch.cuda.synchronize()
+    idx = idx.cpu().numpy()
+    assert np.array_equal(idx[good], r_idx[good])
+    for t in bad:
+        assert idx[t].min() >= 0 and idx[t].max() < E and np.unique(idx[t]).size == k
