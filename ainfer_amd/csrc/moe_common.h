@@ -350,6 +350,11 @@ __device__ __forceinline__ float row_rms_inv(const uint16_t *__restrict__ xr, in
   return rms_inv_finish(tot, emin, xr, H, eps, lane);
 }
 
+// silu(g) * u
+__device__ __forceinline__ float silu_mul(float g, float u) {
+  return g / (1.0f + expf(-g)) * u;
+}
+
 // two floats as packed bf16 (low half: lo), round to nearest even
 // (v_cvt_pk_bf16_f32; for finite values the same bits as f32_to_bf16)
 __device__ __forceinline__ uint32_t bf16x2_bits(float lo, float hi) {

@@ -39,10 +39,6 @@ __device__ __forceinline__ u32x4 ldg_stream(const void *p) {
   return __builtin_nontemporal_load((const u32x4 *)p);
 }
 
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return g / (1.0f + expf(-g)) * u;
-}
-
 __device__ __forceinline__ void dma16(const void *g, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                :

@@ -106,11 +106,16 @@ __device__ __forceinline__ V mfma_bf16(u32x4 a, u32x4 b, V c) {
                                                    __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-// silu(g) * u for the prefill epilogue: the hardware exp2 and reciprocal
-// (about 1 ulp each) instead of expf and an IEEE division, which made the
-// epilogue several times longer than a group of the main loop.  The result is
-// rounded to bf16 (2^-9 relative) right after.  Large |g| behaves: exp2 -> inf
-// gives rcp 0 and g * 0; exp2 -> 0 gives g.
+// silu(g) * u by the hardware exp2 and reciprocal (about 1 ulp each, and the
+// rounding of g log2 e under exp2) instead of silu_mul's expf and division, for
+// tiles of more than 32 tokens in calls of GEMM_MIN_T or more, whose epilogue is
+// VALU-bound: silu_mul there too takes 3% of such layers (us, H2048 E512 k10
+// I512 T4096: 519 -> 535; H2560 E96 k6 I896 T2048: 459 -> 468; H4096 I1024
+// T4096: 1820 -> 1841).  The other tiles wait for their weights, and silu_mul
+// costs them at most 1% (T192 214 -> 215, T1500 286 -> 289, H2560 E96 T301 166.5
+// either way).  An act differs by a few units of its last fp32 place, which its
+// rounding to bf16 hides but for about one value in 65000.
+// Large |g| behaves: exp2 -> inf gives rcp 0 and g * 0; exp2 -> 0 gives g.
 __device__ __forceinline__ float silu_mul_fast(float g, float u) {
   const float e = __builtin_amdgcn_exp2f(g * -1.44269504088896341f);
   return g * __builtin_amdgcn_rcpf(1.0f + e) * u;
@@ -404,27 +409,35 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
       // (perm32_pos), and live in lanes rl and rl ^ 4
       const bool hi4 = (rl & 4) != 0;
       const uint32_t sel0 = pair_sel(hi4, 0), sel1 = pair_sel(hi4, 1);
+      auto stage = [&](auto fast) {
 #pragma unroll
-      for (int ns = 0; ns < NS / 2; ++ns) {
-        // within a 32-aligned block of columns, MFMA order is block-local
-        const int p = perm32_pos(wn * 32 + ns * TM + (rl & ~4));  // the pair's even position
+        for (int ns = 0; ns < NS / 2; ++ns) {
+          // within a 32-aligned block of columns, MFMA order is block-local
+          const int p = perm32_pos(wn * 32 + ns * TM + (rl & ~4));  // the pair's even position
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms)
+          for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-          for (int i = 0; i < NQ; ++i) {
-            float f[4];
+            for (int i = 0; i < NQ; ++i) {
+              float f[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-              f[r] = silu_mul_fast(tot[ms][ns][4 * i + r], tot[ms][ns + NS / 2][4 * i + r]);
-            const uint32_t p01 = bf16x2_bits(f[0], f[1]), p23 = bf16x2_bits(f[2], f[3]);
-            const uint32_t send = hi4 ? p01 : p23, own = hi4 ? p23 : p01;
-            // lane ^ 4 inside each group of 32 lanes (ds_swizzle bit mode)
-            const uint32_t recv = (uint32_t)__builtin_amdgcn_ds_swizzle((int)send, 0x101F);
-            const int row0 = ms * TM + 8 * i + 4 * Q + (hi4 ? 2 : 0);
-            *(uint32_t *)(lds + row0 * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel0);
-            *(uint32_t *)(lds + (row0 + 1) * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel1);
-          }
-      }
+              for (int r = 0; r < 4; ++r) {
+                const float gv = tot[ms][ns][4 * i + r], uv = tot[ms][ns + NS / 2][4 * i + r];
+                f[r] = decltype(fast)::value ? silu_mul_fast(gv, uv) : silu_mul(gv, uv);
+              }
+              const uint32_t p01 = bf16x2_bits(f[0], f[1]), p23 = bf16x2_bits(f[2], f[3]);
+              const uint32_t send = hi4 ? p01 : p23, own = hi4 ? p23 : p01;
+              // lane ^ 4 inside each group of 32 lanes (ds_swizzle bit mode)
+              const uint32_t recv = (uint32_t)__builtin_amdgcn_ds_swizzle((int)send, 0x101F);
+              const int row0 = ms * TM + 8 * i + 4 * Q + (hi4 ? 2 : 0);
+              *(uint32_t *)(lds + row0 * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel0);
+              *(uint32_t *)(lds + (row0 + 1) * OST + p * 2) = __builtin_amdgcn_perm(recv, own, sel1);
+            }
+        }
+      };
+      if (NSUB > 2 && a.T >= GEMM_MIN_T)
+        stage(std::true_type());
+      else
+        stage(std::false_type());
       __syncthreads();
       uint16_t *dst = shared ? a.act_s : a.act;
       float *as = shared ? a.asum_s : a.asum;
