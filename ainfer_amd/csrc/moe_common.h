@@ -219,9 +219,12 @@ __device__ __forceinline__ int xcd_remap(int b, int G) {
   return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
 }
 
+// the prefill GEMM takes an INT4 weight q as the bf16 value q + this
+constexpr float GEMM_NIB_OFFSET = 24.0f;
+
 // MFMA-order copy of one token row (position 8*j+e <- k = 4*e+j inside every
-// 32-element block) and, when xsum is non-null, -136 x its 128-wide group
-// sums (what the prefill GEMM's accumulators start from).
+// 32-element block) and, when xsum is non-null, -GEMM_NIB_OFFSET x its 128-wide
+// group sums (what the prefill GEMM's accumulators start from).
 // RMSNorm applied on the fly (the decode routing kernel at T <= 16, so a
 // block needs no separate RMSNorm launch): the per-token scale and the
 // normalized bf16 values are bit-identical to k_rmsnorm (moe_route.hip).
@@ -434,7 +437,7 @@ __device__ __forceinline__ void write_xperm(const uint16_t *__restrict__ xrow,
           bs += __uint_as_float(in[i2] << 16) + __uint_as_float(in[i2] & 0xFFFF0000u);
         bs += __shfl_xor(bs, 1, 64);
         bs += __shfl_xor(bs, 2, 64);
-        if ((b & 3) == 0) xsum[(size_t)t * (H >> 7) + (b >> 2)] = -136.0f * bs;
+        if ((b & 3) == 0) xsum[(size_t)t * (H >> 7) + (b >> 2)] = -GEMM_NIB_OFFSET * bs;
       }
       if (q8) {
         float m = 0.0f;  // the reference's running max from 0 (exact: any order)

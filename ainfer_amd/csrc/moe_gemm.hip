@@ -1,9 +1,9 @@
 // moe_gemm.hip - grouped INT4 expert GEMM for prefill (bf16 MFMA).
 //
-// Same arithmetic as the decode kernel (moe_expert.hip): weights become bf16
-// 136 + q with one AND-OR per pair, every 128-wide group accumulates from
-// -136 * sum_{k in g} a[m][k] and the group's scale is applied with one fp32
-// fma per output, so the result is sum_g s_g * sum_{k in g} q * a.
+// As in the decode kernel (moe_expert.hip), weights become bf16 values a constant
+// above q (here 24, nib_slice3), every 128-wide group accumulates from -24 *
+// sum_{k in g} a[m][k] and the group's scale is applied with one fp32 fma per
+// output, so the result is sum_g s_g * sum_{k in g} q * a.
 // Restates the reference's INT4 GEMM (ChunkGemm, tools/cmdlist/kernels.cpp:
 // 691-785; gemmMT4, tools/prefill/prefill.cpp:46-129) for bf16 MFMA.
 //
@@ -85,15 +85,27 @@ struct Geo {
 // LDS bank-conflict cycles than c ^ r).
 __device__ __forceinline__ int aswz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
-// Four bf16 pairs 136 + q of k-slice j of a packed 16-byte chunk.  A nibble's
-// two's complement value q is (nibble ^ 8) - 8, and bf16 0x43NN is exactly
-// 128 + NN, so the shifted and masked nibble pair xor'ed with `magic` =
-// 0x43084308 (held in a register) is the pair 136 + q: one v_bitop3_b32 after
-// the shift.
+// Four bf16 pairs 24 + q of k-slice j of a packed 16-byte chunk
+// (GEMM_NIB_OFFSET).  A nibble's two's complement value q is (nibble ^ 8) - 8,
+// and a bf16 between 16 and 32 holds 16 + NN for the four upper bits NN of its
+// mantissa, so the nibble pair shifted there, masked and xor'ed with `magic` =
+// 0x41C041C0 (held in a register) is the pair 24 + q: a shift and one
+// v_bitop3_b32.
+//
+// Why 24: the fp32 sums pass through the offset times sum a, whose rounding is
+// what a dot is off by.  With the nibble in the mantissa's lower four bits
+// (136 + q, one shift in four saved) a gate dot over 2048 columns of variance 1
+// with |q| <= 7 was off by 1.7e-4 to 2.3e-4 (root mean square over dots that are
+// 0 in 64 bits), where the 4-token items, which start anew every 32 columns, are
+// off by 4e-5 to 7e-5; now 1.2e-5 to 1.9e-5.  The shift costs 1 to 2% (us, H2048
+// E512 k10 I512: T192 216 -> 218, T1500 293 -> 296, T4096 516 -> 526; H2560 E96
+// k6 I896 T301 168 -> 169, T2048 461 -> 469; H4096 I1024 T4096 1796 -> 1819).
 __device__ __forceinline__ u32x4 nib_slice3(u32x4 b, int j, uint32_t magic) {
-  const uint32_t mask = 0x000F000Fu;
-  return u32x4{((b[0] >> (4 * j)) & mask) ^ magic, ((b[1] >> (4 * j)) & mask) ^ magic,
-               ((b[2] >> (4 * j)) & mask) ^ magic, ((b[3] >> (4 * j)) & mask) ^ magic};
+  u32x4 r;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+    r[d] = ((j == 0 ? b[d] << 3 : b[d] >> (4 * j - 3)) & 0x00780078u) ^ magic;
+  return r;
 }
 
 // D (TM x TM) += A B: 16 x 16 over 32 k, or 32 x 32 over 16 k
@@ -285,7 +297,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
     // other row; the same for all row tiles, whose rows differ by even numbers)
     uint32_t ssh = ((uint32_t)(brow0 * G) & 1u) * 16u;
     uint32_t magic;
-    asm volatile("v_mov_b32 %0, 0x43084308" : "=v"(magic));
+    asm volatile("v_mov_b32 %0, 0x41C041C0" : "=v"(magic));
     // acc and sprev start at zero, so the scale step of "group -1" adds
     // +0 * +0 to tot's +0 and leaves it unchanged (no branch in the loop)
     acc_t tot[MS][NS], acc[MS][NS];
@@ -331,7 +343,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
         sg[ns] = scale_to_f32<SD>((uint16_t)(*(const uint32_t *)(st + soffl + SO + brow(ns) * 4) >> ssh));
       ssh ^= 16u;
       scale_step();
-      // group sums (-136 sum_k a): the first k-slice accumulates onto them
+      // group sums (-24 sum_k a): the first k-slice accumulates onto them
       acc_t c0[MS];
 #pragma unroll
       for (int ms = 0; ms < MS; ++ms)
@@ -460,7 +472,7 @@ __device__ __forceinline__ void gemm_item(const GemmArgs &a, const int lb, const
         for (int d = 0; d < 4; ++d)
           v += __uint_as_float(out[i][d] << 16) + __uint_as_float(out[i][d] & 0xFFFF0000u);
         v = row16_sum(v);
-        if (c == 0 && row < mcnt) as[(size_t)(pos0 + row) * (N / COLS) + nb] = -136.0f * v;
+        if (c == 0 && row < mcnt) as[(size_t)(pos0 + row) * (N / COLS) + nb] = -GEMM_NIB_OFFSET * v;
       }
     } else {
       constexpr int OST = BN * 2 + 16;

@@ -36,7 +36,7 @@ struct GemmArgs {
   const uint16_t *a_shared;   // MODE 1: act_s [T][Is]
   uint16_t *act, *act_s;      // MODE 0 out
   uint16_t *o;                // MODE 1 out: [Tk + T][H] bf16
-  const float *xsum;          // [T][H/128] -136 x the group sums of x
+  const float *xsum;          // [T][H/128] -GEMM_NIB_OFFSET x the group sums of x
   float *asum, *asum_s;       // [Tk][I/128], [T][Is/128] the same of act (MODE 0 out)
   const int32_t *ptok;
   const int4 *tiles;
@@ -150,7 +150,7 @@ hipError_t launch_router(const void *x, const void *rw, const float *bias, const
 // the last block also runs the dispatch.  approx [T][E] and wnorm [E] are
 // scratch.
 bool router_supported(int H, int E);
-// xsum (may be NULL): [T][H/128] -136 x the group sums of x for the prefill GEMM.
+// xsum (may be NULL): [T][H/128] -GEMM_NIB_OFFSET x the group sums of x for the prefill GEMM.
 hipError_t launch_router_fast(const void *x, const void *rw, const float *bias, const void *gw,
                               float *approx, float *wnorm, int32_t *idx, float *w, float *sg,
                               void *xperm, float *xsum, int T, int H, int E, int k,

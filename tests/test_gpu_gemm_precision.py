@@ -73,3 +73,36 @@ def test_silu_has_the_decode_items_bits(torch, T, crowded):
         assert want.abs().max() > 1
         diff = int((got.view(torch.int16) != want.view(torch.int16)).sum())
         assert diff == 0, (draw, diff)
+
+
+@pytest.mark.parametrize("T", [40, 255, 256, 512, 1024])
+def test_dots_are_as_near_as_the_decode_items(torch, T):
+    """Gate dots that are 0 in 64 bits (every group's second half repeats x and
+    negates the weights), read back as act = silu(e) * 1 = e / 2 of their fp32
+    error e: at 17 tokens and more, in tiles of every height, the mean square is
+    no larger than that of the decode items on the same tokens."""
+    from ainfer_amd.moe import MoeLayer
+    from ainfer_amd.synthetic import MoeConfig
+    print(f"[case] dot error T={T}", flush=True)
+    H, E, k, I = 2048, 64, 8, 256
+    ly = MoeLayer(MoeConfig("dot", H, E, k, I, 0, (T,), seed=3))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    t = ly.t
+    q = torch.randint(-7, 8, (E * I, H // 128, 64), device="cuda", generator=g)
+    t["w_gate"].copy_(pack(torch, torch.cat([q, -q], -1).view(E * I, H)))
+    up = torch.zeros(I, H, dtype=torch.int64, device="cuda")
+    up[:, 127] = 1
+    down = (torch.arange(I, device="cuda")[None] == torch.arange(H, device="cuda")[:, None] % I).long()
+    t["w_up"].copy_(pack(torch, up).repeat(E))
+    t["w_down"].copy_(pack(torch, down).repeat(E))
+    for n in ("s_gate", "s_up", "s_down"):
+        t[n].fill_(1.0)
+    x = torch.randn(T, H // 128, 64, device="cuda", generator=g)
+    x[:, 0, 63] = 1  # column 127: what up reads
+    x = torch.cat([x, x], -1).view(T, H).to(torch.bfloat16)
+    idx = torch.stack([torch.randperm(E, device="cuda", generator=g)[:k] for _ in range(T)]).int()
+    ws = ly.workspace(T)
+    rms = [float(o.double().pow(2).mean().sqrt())
+           for o in (ly.experts(x, idx, ws)[:T * k], decode_rows(torch, ly, x, idx, ws))]
+    print(f"[dot error] T={T} gemm {rms[0]:.2e} items {rms[1]:.2e}", flush=True)
+    assert 0 < rms[0] <= rms[1], rms
