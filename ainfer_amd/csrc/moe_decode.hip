@@ -12,9 +12,10 @@
 //  k_route_decode   workgroups [0, NR): canonical router logits, one
 //                   (one row x 1 or 2 tokens) unit per wave, each stored
 //                   with an sc1 store as ~bits into a key slot of the sync
-//                   region (never 0: ~bits == 0 only for one NaN pattern no
-//                   bf16 product or sum yields); workgroup NR (one wave per
-//                   token) polls its token's slots
+//                   region (never 0: the NaN 0xFFFFFFFF, which no bf16
+//                   product or sum yields but a router bias may hold, is
+//                   stored as 0xFFFFFFFE); workgroup NR (one wave per token)
+//                   polls its token's slots
 //                   until none is 0, clears them, takes the exact top-k, the
 //                   weights and the shared gate, and builds the dispatch
 //                   (tiles of at most DEC_MT tokens) from LDS.  A slot that is
@@ -266,7 +267,9 @@ __global__ __launch_bounds__(W * 64) void k_route_decode(RouteDecodeArgs a) {
             const int r = rbase + i, t = t0 + j;
             if (r >= nrows || t >= T) continue;
             const float v = r < E && a.bias ? acc[i][j] + a.bias[r] : acc[i][j];
-            st_dev(a.slots + (size_t)t * (E + 1) + r, ~__float_as_uint(v));
+            // never 0, which the selection polls away: the one NaN whose ~bits
+            // are 0 is stored as its neighbour
+            st_dev(a.slots + (size_t)t * (E + 1) + r, max(~__float_as_uint(v), 1u));
           }
       }
     }
