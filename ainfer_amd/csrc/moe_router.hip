@@ -200,6 +200,12 @@ constexpr int SEL_COOP_MAX_T = 1024;
 // the gate's dot on its own, x re-read after the top-k and lists of 1024 entries
 // (3 workgroups per CU): T64 17.3 us, T512 16.5, T1500 19.9, T4096 39; H4096 T4096
 // 105.  Now 14.4, 9.4, 17.0, 25.8 and 57.6.
+//
+// LATE_X (more than 512 experts, 1024 < H <= 2048, one wave per token): the row
+// and the norms are loaded after the approximate top-k.  Held through it they take
+// 13 VGPRs more than the 128 of 4 waves per SIMD; whole route, E1024 H2048 k8,
+// spilled / with 3 waves / so: T2048 36.6, 34.1, 33.6 us, T4096 52.6, 54.3, 48.7
+// (E700 H1536: T4096 38.9, 40.6, 35.1).
 template <int NV, int CH, bool COOP>
 __global__ __launch_bounds__(256, CH <= 4 ? 4 : 2) void k_select(const float *__restrict__ approx,
                                                 const float *__restrict__ wnorm,
@@ -217,6 +223,7 @@ __global__ __launch_bounds__(256, CH <= 4 ? 4 : 2) void k_select(const float *__
                                                 int32_t *ccount) {
   // candidate lists (E <= 64 NV)
   constexpr int LISTS = COOP ? 1 : SEL_WAVES;
+  constexpr bool LATE_X = NV > 8 && CH == 4 && !COOP;
   __shared__ int cl[LISTS][64 * NV];
   __shared__ float cv[LISTS][64 * NV + 1];  // and the shared gate's dot
   __shared__ uint64_t s_cand[LISTS][64];
@@ -240,11 +247,14 @@ __global__ __launch_bounds__(256, CH <= 4 ? 4 : 2) void k_select(const float *__
     for (int i = 0; i < NV; ++i) {
       const int e = min(lane + 64 * i, E - 1);  // unconditional: loads issue together
       av[i] = lead ? ar[e] : 0.0f;
-      wn = fmaxf(wn, lead ? wnorm[e] : 0.0f);
+      if (!LATE_X) wn = fmaxf(wn, lead ? wnorm[e] : 0.0f);
     }
+    auto load_x = [&]() {
 #pragma unroll
-    for (int j = 0; j < CH; ++j)
-      xc[j] = *(const u32x4 *)(xrow + (size_t)min(lane + 64 * j, nch - 1) * 8);
+      for (int j = 0; j < CH; ++j)
+        xc[j] = *(const u32x4 *)(xrow + (size_t)min(lane + 64 * j, nch - 1) * 8);
+    };
+    if (!LATE_X) load_x();
     if ((xperm || w8.q) && (!COOP || wave == 1))
       write_xperm(xrow, xperm, xsum, t, H, lane, nullptr, 1.0f, w8.q, w8.s, w8.sum);
     STRACE(1);
@@ -255,6 +265,11 @@ __global__ __launch_bounds__(256, CH <= 4 ? 4 : 2) void k_select(const float *__
     uint32_t selk = 0u;
     if (lead) wave_topk_fast<NV>(key, E, k, lane, seli, selk, s_cand[sw], s_sel[sw]);
     STRACE(2);
+    if (LATE_X) {
+      load_x();
+#pragma unroll
+      for (int i = 0; i < NV; ++i) wn = fmaxf(wn, wnorm[min(lane + 64 * i, E - 1)]);
+    }
     const uint32_t kth = (uint32_t)__builtin_amdgcn_readlane((int)selk, k - 1);
     float selv = 0.0f, sgv = 0.0f;
     {

@@ -163,7 +163,8 @@ def test_w4a8_gemm_gives_the_decode_rows(torch, H, E, k, I, Is, scales):
 
 
 @pytest.mark.parametrize("H,E,T", [(128, 96, 257), (256, 512, 511), (256, 512, 1025), (128, 512, 2048),
-                                   (384, 500, 2049), (2560, 64, 300), (4096, 40, 256)])
+                                   (384, 500, 2049), (2560, 64, 300), (4096, 40, 256),
+                                   (1152, 513, 1025), (2048, 1024, 1030)])
 def test_router_at_tile_edges(torch, oracle, H, E, T):
     """The prefill router at the edges of its GEMM tiles (32 x 64, 64 x 64, 64 x
     128 of tokens x experts, the first and last count of items of each; K of 2
