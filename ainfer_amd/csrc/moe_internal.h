@@ -78,19 +78,29 @@ constexpr int GEMM_MIN_T = 256;
 // Experts as the grouped GEMM or as streaming items of at most DEC_MT tokens,
 // for 16 < T.  The items re-read an expert's weights for every 4 of its
 // tokens; the GEMM reads them once but needs enough items to fill the chip.
-// Measured crossover in tokens per expert (T k / E): 2.6 at H2048 E512 k10
-// I512 (T=160: 225 us items, 210 GEMM; T=96: 175, 188), 1.9 at H4096 I1024, 2
-// to 3 at E64 k8 and E32 k4, 3.2 at E128 k8, 3.5 at H3072 E324 k5 I256; 5 at
-// E8 k2 I4096 and E66 k5 H3584 I128, one of whose stages has fewer than 128
-// items; 12 at E8 k2 I1024 (T=32: 38 us items, 41 GEMM; T=64: 47, 41), where
-// both have.
+// Two lines, in tokens per expert (T k / E), and the GEMM is past both:
+//  - 3.25.  Where both stages have items for every CU the two cross at 2.0
+//    (H4096 E512 k10 I1024; T = 97: 584 us items, 591 GEMM; T = 133: 673, 630), 2.8
+//    (H2048 E512 k10 I512; T = 133: 203, 208; T = 154: 222, 211; and E128 k8 I768),
+//    3.0 (E256 k8 I256) and 3.25 (H3072 E324 k5 I256; T = 194: 143, 147; T = 233:
+//    156, 152).  The line is the largest, so that none of these is slower by the
+//    GEMM; below it the first ones' items are the slower ones, by up to 15%.
+//  - C (1 / gate-up items + 1 / (2 x down items)).  With few items the GEMM waits
+//    for one block's chain of groups per stage, whatever T is (down's weights are
+//    half of gate/up's), while the items only grow with T.  C = the crossover over
+//    that sum: 390 to 500 at H 2048 to 4096 (H3584 E20 k4 I128 crosses at 23: T = 80
+//    51 us items, 56 GEMM; H3584 E66 k5 I128 at 6.4: T = 66 57, 62; H2048 E8 k2 I512
+//    at 17, I4096 at 5.6; H2048 E4 k1 I1024 at 21), 300 to 450 at H 1280 and 1536,
+//    220 to 260 at H1024 (E8 k2 I1024 at 7, E16 k4 I256 at 10), whose chains are
+//    short, 60 to 140 at H512 (E8 k2 I256 at 13, E20 k4 I128 below 4); less where a
+//    shared expert adds items (350 to 410 from H 2048 on).
 inline bool expert_gemm_at(const ainfer_moe_shape &s, int T) {
   if (T >= GEMM_MIN_T) return true;
   if (T <= 16) return false;
   const long E = s.n_experts, slots = (long)T * s.top_k;
   const long gu = E * (s.inter / 128), dn = E * ((s.hidden + 255) / 256);
-  const long quarters = (gu < dn ? gu : dn) >= 128 ? 13 : gu + dn >= 256 ? 20 : 48;
-  return 4 * slots >= quarters * E;
+  const long C = s.hidden <= 512 ? 128 : s.hidden <= 1024 ? 256 : 432;
+  return 4 * slots >= 13 * E && slots * 2 * gu * dn >= C * E * (gu + 2 * dn);
 }
 
 // Rows quantized for the W4A8 GEMM: codes in W8 order (write_xperm,

@@ -91,11 +91,11 @@ def test_expert_rows_at_tile_edges(torch, oracle, H, I, Is, which, scales):
 
 
 # (H, E, k, I, Is) and the token counts either side of the rule that sends the
-# experts to the GEMM: 3.25 tokens per expert, 5 and 12 where the stages have
-# few items
+# experts to the GEMM: 3.25 tokens per expert, and up to about 20 where the
+# stages have few items
 EDGES = [((1024, 64, 8, 256, 256), (25, 26, 64, 65)),
          ((512, 8, 2, 256, 384), (47, 48, 65)),
-         ((3584, 20, 4, 128, 0), (24, 25)),
+         ((3584, 20, 4, 128, 0), (24, 25, 111, 112)),
          ((640, 130, 3, 128, 0), (140, 141))]
 
 
