@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "../../include/ainfer_moe.h"
 
 // Arguments of the grouped expert kernels (one launch covers the routed
@@ -122,14 +124,31 @@ struct W8GemmArgs {
   int T, k, E, H, I, Is;
   int n_nblk;            // set by the launcher
 };
-// The W4A8 GEMM from 2 tokens on, except at decode sizes where its items are few
-// and long: a down product of more than 2048 columns (H2048 E8 k2 I4096, T = 2:
-// 34 us by 16-row GEMV blocks, 45), or fewer than 24 gate/up items (H3584 E66 k5
-// I128, T = 2: 32 and 33; T = 6: 41 and 37).  Else T = 2 to 16 gain 10 to 35%
-// (H2048 E512 k10 I512: T = 4 42 -> 32 us, T = 16 94 -> 79).
+// The W4A8 GEMM or 16-row GEMV blocks, from 2 tokens on.  The GEMM reads a weight
+// once per tile, but where its items are few it waits for one item's chain of
+// groups per stage; the blocks cut rows by 16 (us, blocks then GEMM).
+//  Above 16 tokens the GEMM.  At 2 to 4 (down with the combine in it, intermediate
+//  sizes to W8DC_MAX_K: I4096 H2048 E8 k2 T2 35, 45) from 24 gate/up items on
+//  (H3584 E20 k4 I128 T4 30, 33; H2048 E512 k10 I512 T4 42, 32), and above I256
+//  where gate/up's groups are no more than 0.9 of its items, of the experts that T
+//  tokens hit on average (H4096 E32 k2 I512, 1.4 at T3: 29, 34; H4096 E64 k4 I512,
+//  1.0 at T2: 33, 35, 0.7 at T3: 38, 36).
+//  At 5 to 16 by groups over items, gate/up's + 10 times down's: up to 0.8, or 1.6
+//  at I to 256.  At H2048
+//  E32 k2 I1408 it is 1.2 at T8 (33, 33) and 0.7 at T16 (42, 36); H2048 E64 k2
+//  I1024 0.8 at T8 (30, 32), 0.7 at T10 (34, 33); H4096 E32 k2 I512 1.2 at T5 (33,
+//  38), 0.6 at T12 (43, 42); H4096 E6 k2 I1024 1.8 at T6 (35, 41); H2048 E4 k1
+//  I1024 3.0 (T8 26, 30); H3584 E20 k4 I128 1.9 at T6 (31, 35), 1.5 at T12 (39,
+//  38); H3584 E66 k5 I128 1.3 at T5 (40, 36).
 inline bool w4a8_gemm_at(const ainfer_moe_shape &s, int T) {
   if (T > 16 || T < 2) return T > 1;
-  return s.inter <= 2048 && s.shared_inter <= 2048 && (long)T * s.top_k * (s.inter / 128) >= 24;
+  if (s.inter > 2048 || s.shared_inter > 2048) return false;
+  const int gi = s.inter / 128;
+  const double E = s.n_experts, hit = E * (1.0 - std::pow(1.0 - s.top_k / E, T));
+  const double gu = hit * gi, dn = hit * ((s.hidden + 255) / 256);
+  const double chain = (s.hidden / 128) / gu;
+  if (T <= 4) return (long)T * s.top_k * gi >= 24 && (gi <= 2 || chain <= 0.9);
+  return chain + 10 * gi / dn <= (gi <= 2 ? 1.6 : 0.8);
 }
 hipError_t launch_w4a8_gemm(int mode, int scale_dtype, W8GemmArgs a, int max_tiles,
                             hipStream_t s);

@@ -114,3 +114,26 @@ def test_w4a8_rows_do_not_depend_on_the_call(torch, oracle, H, E, k, I, Is):
                 assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (fn.__name__, n)
             if fn == ly.forward:
                 check_close(to_np(want), host_copy(oracle, ly).forward_w4a8(to_np(x), 16), "w4a8 16")
+
+
+@pytest.mark.parametrize("H,E,k,I,Is", [(2048, 64, 2, 1024, 0), (3584, 20, 4, 128, 128),
+                                        (1024, 24, 3, 512, 256), (640, 40, 2, 384, 0),
+                                        (4096, 64, 4, 512, 128)])
+def test_w4a8_rows_either_side_of_the_gemm_rule(torch, H, E, k, I, Is):
+    """Calls of 2 to 16 tokens go to the GEMM or to 16-row blocks by their items:
+    a token's row has the same bits in all of them."""
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    print(f"[case] w4a8 rule H={H} E={E} k={k} I={I} Is={Is}", flush=True)
+    cfg = MoeConfig("w8rule", H, E, k, I, Is, (17,), seed=14)
+    ly = MoeLayer(cfg, precision=L.PRECISION_W4A8)
+    x = make_input(cfg, 17, tag=4)
+    ws = ly.workspace(17)
+    want = torch.empty_like(x)
+    ly.forward(x, want, ws)  # above 16 tokens: the GEMM
+    for T in range(2, 17):
+        y = torch.full((T, H), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ly.forward(x[:T], y, ws)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want[:T].view(torch.int16)), T
