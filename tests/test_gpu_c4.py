@@ -79,7 +79,7 @@ def test_c4_chained_blocks_real_shape(torch, oracle, c4_layers, T):
 @pytest.mark.parametrize("T", [1, 2, 16])
 def test_c1_block_in_place(torch, oracle, T):
     """block_forward(r, r) is bit-identical to block_forward(r', out) with r'
-    a copy, on the fused expert kernel (T <= 2) and the staged path."""
+    a copy, with the combine in the down kernel (T = 1, 2) and of its own."""
     from ainfer_amd.moe import make_input
     import test_gpu_parity as P
     layer = P.get_layer(torch, "c1")

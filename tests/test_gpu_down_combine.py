@@ -137,3 +137,54 @@ def test_w4a8_rows_either_side_of_the_gemm_rule(torch, H, E, k, I, Is):
         ly.forward(x[:T], y, ws)
         torch.cuda.synchronize()
         assert torch.equal(y.view(torch.int16), want[:T].view(torch.int16)), T
+
+
+@pytest.mark.parametrize("scales", ["fp16", "bf16"])
+@pytest.mark.parametrize("H,E,k,I,Is", [(1024, 12, 3, 2048, 0), (512, 10, 4, 256, 1280),
+                                        (1024, 6, 2, 1280, 2048), (256, 20, 16, 4096, 4096)])
+def test_two_tokens_with_a_long_k(torch, oracle, H, E, k, I, Is, scales):
+    """Two tokens with an expert above 1024 columns: gate/up, down and the combine
+    in one launch whose workgroups meet through counters (the first three shapes;
+    LDS leaves the last one three launches, and gives its T = 1 down + combine 16
+    waves of 8 runs).  Every sum has the order of the one-token call's, so the
+    rows are that call's bit for bit, shared experts (two tokens of one expert) and
+    the residual included; calls follow each other on one workspace, whose
+    counters end at zero.  Then, with every wait made to give up at once from the
+    host, the outputs are NaN and the check reports it."""
+    import ctypes as C
+    from ainfer_amd import _lib as L
+    from ainfer_amd.moe import MoeLayer, _ptr, _stream, make_input
+    from ainfer_amd.synthetic import MoeConfig
+    what = f"H={H} E={E} k={k} I={I} Is={Is} {scales} T=2"
+    print(f"[case] {what}", flush=True)
+    cfg = MoeConfig("two", H, E, k, I, Is, (2,), seed=15)
+    ly = MoeLayer(cfg, scale_dtype=L.SCALE_FP16 if scales == "fp16" else L.SCALE_BF16)
+    hl = host_copy(oracle, ly)
+    ws = ly.workspace(2)
+    for tag in range(4):
+        x = make_input(cfg, 2, tag=tag)
+        if tag == 3:
+            x[1] = x[0]  # every expert has both tokens
+        for fn in (ly.forward, ly.block_forward):
+            y, one = torch.full_like(x, float("nan")), torch.empty_like(x)
+            fn(x, y, ws)
+            for t in (0, 1):
+                fn(x[t:t + 1], one[t:t + 1], ws)
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), one.view(torch.int16)), (what, tag, fn.__name__)
+            if fn == ly.forward:
+                check_close(to_np(y), hl.forward(to_np(x), 2), what)
+        assert ly.workspace_check(ws) == L.OK
+    try:
+        L.check(L.lib().ainfer_moe_debug_spin_limit(0))
+        ly.forward(x, y, ws)
+        torch.cuda.synchronize()
+    finally:
+        L.check(L.lib().ainfer_moe_debug_spin_limit(1 << 20))
+    assert torch.isnan(y.float()).all()
+    assert ly.workspace_check(ws) == L.ERR_SYNC
+    L.check(L.lib().ainfer_moe_workspace_init(C.byref(ly.shape), _ptr(ws), ws.numel(), _stream(None)))
+    ly.block_forward(x, y, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), one.view(torch.int16))
+    assert ly.workspace_check(ws) == L.OK

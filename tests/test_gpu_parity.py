@@ -303,8 +303,8 @@ def test_block_forward_fused_norm(torch, oracle, mode):
     code path for T = 1..4).  At T = 3 to 16 every later stage is the one
     T = 17 runs (4-token tiles, per-token arithmetic), and T = 17 normalizes
     with the separate RMSNorm kernel: each token's output must be equal bit
-    for bit (T = 5 and 8: both normalize with the separate kernel).  T = 1 and 2 run the fused expert kernel, whose down items split
-    K differently, so there the check is the oracle's block within tolerance
+    for bit (T = 5 and 8: both normalize with the separate kernel).  At T = 1 and 2
+    down splits K differently (two k-groups to a sum), so there the check is the oracle's block within tolerance
     (as at every T)."""
     from ainfer_amd import _lib as L
     from ainfer_amd.moe import MoeLayer, make_input
@@ -351,9 +351,8 @@ def test_zero_tokens_and_errors(torch, oracle):
 @pytest.mark.parametrize("name,T", [("c1", 1), ("c1", 16), ("c1", 300), ("c3", 64)])
 def test_forward_parity_bf16_scales(torch, oracle, name, T):
     """The reference's own scale dtype (bf16, binfer.py:76-91) through every
-    expert path: the fused decode kernel (T=1), the staged decode kernels
-    (T=16), the prefill GEMM with small-expert tiles (T=300) and the
-    16-token-tile kernels (c3, T=64)."""
+    expert path: down with the combine in it (T=1), the streaming items
+    (T=16, and c3 T=64) and the grouped GEMM (T=300)."""
     from ainfer_amd import _lib as L
     from ainfer_amd.moe import MoeLayer, make_input
     from ainfer_amd.synthetic import CONFIGS
@@ -517,7 +516,7 @@ def test_stage_entries_compose_to_forward(torch, oracle, name, T):
     """ainfer_moe_route -> ainfer_moe_experts -> ainfer_moe_combine: within
     the layer tolerance of the oracle at every T, bit-identical to
     ainfer_moe_forward where forward runs the same expert kernels (T >= 3;
-    at T <= 2 it fuses the stages), and with the residual bit-identical to
+    at T <= 2 down splits K differently), and with the residual bit-identical to
     block_forward where that normalizes with the separate kernel (T > 4)."""
     from ainfer_amd.moe import make_input, rmsnorm
     print(f"[case] stage entries {name} T={T}", flush=True)
