@@ -490,7 +490,7 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
   a.a_shared = at<uint16_t>(ws, L.xperm);
   a.act = at<uint16_t>(ws, L.act);
   a.act_s = at<uint16_t>(ws, L.act_s);
-  HIP_TRY(launch_expert_stream(0, s->scale_dtype, a, max_tiles, kbw, RG_GATE_UP, st));
+  HIP_TRY(launch_expert_stream(0, s->scale_dtype, a, max_tiles, kbw, st));
   pc->end(4);
   // down + combine
   a.w0 = w->w_down;
@@ -504,7 +504,7 @@ int run_experts(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const La
   a.a_routed = at<uint16_t>(ws, L.act);
   a.a_shared = at<uint16_t>(ws, L.act_s);
   a.o = at<uint16_t>(ws, L.o);
-  HIP_TRY(launch_expert_stream(1, s->scale_dtype, a, max_tiles, kbw_down, RG_DOWN, st));
+  HIP_TRY(launch_expert_stream(1, s->scale_dtype, a, max_tiles, kbw_down, st));
   pc->end(5);
   return AINFER_OK;
 }
@@ -562,7 +562,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
       return AINFER_OK;
     }
     pc->kernel_events();
-    HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, mtb, 4, DEC_RG_GATE_UP, st));
+    HIP_TRY(launch_expert_stream(0, s->scale_dtype, gu, mtb, 4, st));
     pc->end(4);
     if (down_combine_at(*s, T)) {
       int kbw, wk, wr;
@@ -573,7 +573,7 @@ int do_forward(const ainfer_moe_shape *s, const ainfer_moe_weights *w, const voi
       pc->end(5);
       return AINFER_OK;
     }
-    HIP_TRY(launch_expert_stream(1, s->scale_dtype, dn, mtb, kbw_dn, DEC_RG_DOWN, st));
+    HIP_TRY(launch_expert_stream(1, s->scale_dtype, dn, mtb, kbw_dn, st));
     pc->end(5);
     HIP_TRY(combine(d, L));
     pc->end(6);

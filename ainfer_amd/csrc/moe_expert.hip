@@ -28,14 +28,14 @@ namespace {
 
 constexpr int MAX_WAVES = 16;  // 1024 threads
 
-template <int SD, int KBW, int RG, int MT, int MODE>
+template <int SD, int KBW, int RG, int MODE>
 __global__ __launch_bounds__(1024) void k_expert_lds(ExpertArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tile_id = blockIdx.x / a.n_slabs, slab = blockIdx.x % a.n_slabs;
   int n_tiles;
   const int4 t = sload_tile(a.tiles, a.n_tiles, tile_id, n_tiles);
   if (tile_id >= n_tiles) return;
-  expert_lds_item<SD, KBW, RG, MT, MODE, false, false, true>(a, t, slab, lds);
+  expert_lds_item<SD, KBW, RG, DEC_MT, MODE, false, false, true>(a, t, slab, lds);
 }
 
 }  // namespace
@@ -73,7 +73,7 @@ bool expert_geometry(int mode, int H, int I, int Is, int pref_kbw, int *KBW, int
 
 hipEvent_t g_kev_start = nullptr, g_kev_stop = nullptr;
 
-template <int SD, int MODE, int RG>
+template <int SD, int MODE>
 void launch_kbw(int kbw, unsigned grid, int threads, size_t lds, const ExpertArgs &a,
                 hipStream_t s) {
   auto go = [&](auto kern) {
@@ -85,23 +85,13 @@ void launch_kbw(int kbw, unsigned grid, int threads, size_t lds, const ExpertArg
       kern<<<grid, threads, lds, s>>>(a);
     }
   };
+  constexpr int RG = stream_rg(MODE);
   if (kbw == 1)
-    go(k_expert_lds<SD, 1, RG, DEC_MT, MODE>);
+    go(k_expert_lds<SD, 1, RG, MODE>);
   else if (kbw == 2)
-    go(k_expert_lds<SD, 2, RG, DEC_MT, MODE>);
+    go(k_expert_lds<SD, 2, RG, MODE>);
   else
-    go(k_expert_lds<SD, 4, RG, DEC_MT, MODE>);
-}
-
-template <int SD, int MODE>
-void launch_rg(int rg, int kbw, unsigned grid, int threads, size_t lds, const ExpertArgs &a,
-               hipStream_t s) {
-  if (rg == 1)
-    launch_kbw<SD, MODE, 1>(kbw, grid, threads, lds, a, s);
-  else if (rg == 2)
-    launch_kbw<SD, MODE, 2>(kbw, grid, threads, lds, a, s);
-  else
-    launch_kbw<SD, MODE, 4>(kbw, grid, threads, lds, a, s);
+    go(k_expert_lds<SD, 4, RG, MODE>);
 }
 
 void set_expert_launch_events(hipEvent_t start, hipEvent_t stop) {
@@ -110,9 +100,9 @@ void set_expert_launch_events(hipEvent_t start, hipEvent_t stop) {
 }
 
 hipError_t launch_expert_stream(int mode, int scale_dtype, ExpertArgs a, int max_tiles,
-                                int pref_kbw, int rg, hipStream_t s) {
+                                int pref_kbw, hipStream_t s) {
   if (max_tiles <= 0) return hipSuccess;
-  if (rg != 1 && rg != 2 && rg != 4) return hipErrorInvalidValue;
+  const int rg = stream_rg(mode);
   int kbw;
   if (!expert_geometry(mode, a.H, a.I, a.Is, pref_kbw, &kbw, &a.WK, &a.WR))
     return hipErrorInvalidValue;
@@ -126,14 +116,14 @@ hipError_t launch_expert_stream(int mode, int scale_dtype, ExpertArgs a, int max
   if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
   if (mode == 0) {
     if (scale_dtype == AINFER_SCALE_FP16)
-      launch_rg<AINFER_SCALE_FP16, 0>(rg, kbw, (unsigned)grid, threads, lds, a, s);
+      launch_kbw<AINFER_SCALE_FP16, 0>(kbw, (unsigned)grid, threads, lds, a, s);
     else
-      launch_rg<AINFER_SCALE_BF16, 0>(rg, kbw, (unsigned)grid, threads, lds, a, s);
+      launch_kbw<AINFER_SCALE_BF16, 0>(kbw, (unsigned)grid, threads, lds, a, s);
   } else {
     if (scale_dtype == AINFER_SCALE_FP16)
-      launch_rg<AINFER_SCALE_FP16, 1>(rg, kbw, (unsigned)grid, threads, lds, a, s);
+      launch_kbw<AINFER_SCALE_FP16, 1>(kbw, (unsigned)grid, threads, lds, a, s);
     else
-      launch_rg<AINFER_SCALE_BF16, 1>(rg, kbw, (unsigned)grid, threads, lds, a, s);
+      launch_kbw<AINFER_SCALE_BF16, 1>(kbw, (unsigned)grid, threads, lds, a, s);
   }
   return hipGetLastError();
 }

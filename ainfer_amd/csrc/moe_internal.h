@@ -212,20 +212,11 @@ hipError_t launch_combine_norm(const uint16_t *o, const int32_t *inv, const floa
 // polls a bounded device wait makes before it gives up (sets the workspace's
 // error word); ainfer_moe_debug_spin_limit changes it for tests
 extern int g_spin_max;
-// false when the shape has no wave geometry (more than 8 waves along K)
+// false when the shape has no wave geometry (more than 16 waves along K)
 bool expert_geometry(int mode, int H, int I, int Is, int pref_kbw, int *KBW, int *WK,
                      int *WR);
-// mode 0: gate/up + SiLU-mul; mode 1: down.  max_tiles bounds
-// the tile list.
-// pref_kbw: preferred 128-wide k-groups per wave (1, 2 or 4).
-#ifndef RG_GATE_UP
-#define RG_GATE_UP 1
-#endif
-#ifndef RG_DOWN
-#define RG_DOWN 2
-#endif
-// the same for the decode tiles (T > FUSED_EXPERTS_MAX_T), and the down
-// items' preferred k-groups per wave
+// the streaming items: 16-row groups per wave that share one load of the token
+// rows (gate/up, down), and down's preferred k-groups per wave
 #ifndef DEC_RG_GATE_UP
 #define DEC_RG_GATE_UP 1
 #endif
@@ -235,12 +226,14 @@ bool expert_geometry(int mode, int H, int I, int Is, int pref_kbw, int *KBW, int
 #ifndef DEC_KBW_DOWN
 #define DEC_KBW_DOWN 2
 #endif
-// rg: 16-row groups per wave (1, 2 or 4) sharing one load of the token rows;
-// The next decode gate/up launch of launch_expert_stream (the DEC_MT items)
-// goes through hipExtLaunchKernel with these start/stop events (one shot).
+constexpr int stream_rg(int mode) { return mode == 0 ? DEC_RG_GATE_UP : DEC_RG_DOWN; }
+// The next gate/up launch of launch_expert_stream goes through hipExtLaunchKernel
+// with these start/stop events (one shot).
 void set_expert_launch_events(hipEvent_t start, hipEvent_t stop);
+// mode 0: gate/up + SiLU-mul; mode 1: down.  max_tiles bounds the tile list.
+// pref_kbw: preferred 128-wide k-groups per wave (1, 2 or 4).
 hipError_t launch_expert_stream(int mode, int scale_dtype, ExpertArgs a, int max_tiles,
-                                int pref_kbw, int rg, hipStream_t s);
+                                int pref_kbw, hipStream_t s);
 
 // LDS bytes per wave of a decode expert item (moe_expert_item.h): its A
 // rows (MT x KBW * 256 B), its scales (KBW >= 2: one dword DMA per 256 B),

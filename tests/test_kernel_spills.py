@@ -41,9 +41,10 @@ def spills(tmp_path):
     return out
 
 
-def test_no_selection_kernel_spills(tmp_path):
+def test_no_kernel_spills(tmp_path):
+    """All but the persistent stack, whose phases share one register budget."""
     if not LIB.exists() or not READELF.exists():
         pytest.skip("library or llvm-readelf missing")
-    found = {k: n for k, n in spills(tmp_path).items() if "k_select" in k}
-    assert len(found) == 40  # 5 expert counts x 4 widths x 2 forms
-    assert not {k: n for k, n in found.items() if n}
+    found = spills(tmp_path)
+    assert sum("k_select" in k for k in found) == 40  # 5 expert counts x 4 widths x 2 forms
+    assert not {k: n for k, n in found.items() if n and "k_decode_stack" not in k}
