@@ -721,7 +721,8 @@ int ainfer_moe_validate(const ainfer_moe_shape *s) {
   if (s->group != 128) return AINFER_ERR_SHAPE;
   if (s->precision != AINFER_PRECISION_W4A16 && s->precision != AINFER_PRECISION_W4A8)
     return AINFER_ERR_SHAPE;
-  // K of every expert product <= 4096 (the prefill GEMM's tables hold 32 groups)
+  // K of every expert product <= 4096: the row kernels hold a row of 64 lanes x 8
+  // chunks in registers, and the GEMMs' token offsets (T <= 4096 rows) are 32-bit
   if (s->hidden < 128 || s->hidden % 128 || s->hidden > 4096) return AINFER_ERR_SHAPE;
   if (s->inter < 128 || s->inter % 128 || s->inter > 4096) return AINFER_ERR_SHAPE;
   if (s->shared_inter < 0 || s->shared_inter % 128 || s->shared_inter > 4096)

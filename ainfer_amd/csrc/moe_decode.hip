@@ -1,13 +1,15 @@
-// moe_decode.hip - the decode routing kernel (T <= 16 tokens), the fused
-// expert kernel (T = 2) and the one-token down + combine kernel.
+// moe_decode.hip - the decode routing kernel (T <= 16 tokens), the down + combine
+// kernel (down_combine_at: T = 1, and up to 4 tokens with at most 1024
+// intermediate columns) and the fused expert kernel (T = 2 beyond that, where
+// decode_geometry allows it).
 //
 // Measured on MI355X: a dependent kernel launch costs about 2.5 us, a flag
 // handed from one workgroup to another through device memory about 0.8 us,
 // same-address device atomics serialise at about 11 ns each, and an
 // agent-scope release or acquire fence (a whole-L2 write-back or
-// invalidate) about 20 ns, serialised.  So at T = 2 the layer is two kernels
-// whose stages meet through counters that few workgroups touch, with data
-// handed over by sc1 stores and loads instead of fences (moe_common.h):
+// invalidate) about 20 ns, serialised.  So what meets inside a kernel meets
+// through slots and counters that few workgroups touch, with data handed over by
+// sc1 stores and loads instead of fences (moe_common.h):
 //
 //  k_route_decode   workgroups [0, NR): canonical router logits, one
 //                   (one row x 1 or 2 tokens) unit per wave, each stored
@@ -31,9 +33,11 @@
 //                   (token, slab) sums the token's k + 1 rows of that slab in
 //                   slot order (the combine).
 //
-// At T = 1 the gate/up items run in a launch of their own (k_expert_lds), then
-// k_down_combine_t1: each workgroup owns 8 output rows of every selected
-// expert, so the combine is an LDS exchange and no counter is needed.
+//  k_down_combine   after the gate/up items (k_expert_lds, a launch of their
+//                   own): each workgroup owns 8 or 16 output rows of every
+//                   selected expert, so the combine is an LDS exchange and no
+//                   counter is needed.
+// Every other call runs k_expert_lds twice and k_combine.
 //
 // A wait only ever names work of lower workgroup index, and workgroups are
 // dispatched in index order, so every awaited workgroup is already running.

@@ -9,32 +9,34 @@
 //
 // Block tile: at most 64 tokens (one expert tile of the dispatch) x 256
 // weight rows (MODE 0 takes 128 gate rows and the matching 128 up rows, MODE
-// 1 256 down rows), K in 128-wide groups.  4 waves along the rows; a wave
-// owns 64 x 64 = 4 x 4 tiles of v_mfma_f32_16x16x32_bf16.  16-token subtiles
-// past the tile's count cost no MFMA, A read or A copy, so one kernel serves
-// experts of one token (bound by streaming their weights) and of thousands
-// (bound by the loop's issue).
+// 1 256 down rows), K in 128-wide groups.  4 waves along the rows, each all the
+// tile's tokens x 64 rows: 2 x 2 tiles of v_mfma_f32_32x32x16_bf16 at 33 to 64
+// tokens, 1 x 2 at 17 to 32, 1 x 4 of 16x16x32 up to 16.  16-token subtiles past
+// the tile's count are not copied, and cost MFMAs only as the missing partner of
+// a third one, so one kernel serves experts of one token (bound by streaming
+// their weights) and of thousands (bound by the loop's issue).
 //
-// Why 64 tokens and 4 waves: two such blocks fit a CU (76 KB of LDS each, 2
-// waves per SIMD together), so one block's table loads, barriers and epilogue
+// Why 64 tokens and 4 waves: two such blocks fit a CU (80 KB of LDS each, 2
+// waves per SIMD together), so one block's prologue, barriers and epilogue
 // run under the other's main loop, and a tile holds little padding.  Against
 // one block of 8 waves on 128-token tiles with the experts of at most 32
 // tokens in a 16-token streaming kernel (whole layer, H2048 E512 k10 I512):
 // T = 1500 576 -> 319 us, T = 4096 Zipf 578 -> 477, 4 x 4096 2822 -> 2209;
-// H2560 E96 k6 I896 T = 301 381 -> 191 us.
+// H2560 E96 k6 I896 T = 301 381 -> 191 us.  With the steps since then (32-wide
+// MFMAs, a third stage, scales on the ring) 297, 435, 2065 and 167.
 //
-// Data movement: a 2-stage LDS ring per block, one barrier per group.  Each
-// stage holds one group of the token rows (64 x 256 B, already in MFMA
-// order) and of the raw INT4 weight rows (64 B each).  Both arrive by
-// global->LDS DMA (global_load_lds_dwordx4: lane i of a wave lands at
-// M0 + 16 i), one group ahead of the math, with no staging registers.  The
+// Data movement: an LDS ring of 2 stages, 3 up to 32 tokens, one barrier per
+// group.  Each stage holds one group of the token rows (256 B each, already in
+// MFMA order), of the raw INT4 weight rows (64 B each), the dword of each weight
+// row that holds its scale, and the token rows' group sums (for x from k_select,
+// for act from this kernel's MODE 0 epilogue).  All of it arrives by global->LDS
+// DMA (global_load_lds_dwordx4 and _dword: lane i of a wave lands at M0 + 16 i or
+// 4 i), one or two groups ahead of the math, with no staging registers.  The
 // DMA is issued from inline asm and its completion tracked with explicit
 // vmcnt waits, so the compiler's conservative waits do not serialise the
 // ring.  Rows are swizzled in 16-byte chunks (A: chunk c of row r at
 // c ^ aswz(r); B: chunk q at q ^ bswz(r)) so that the lanes reading 16 rows
-// at one column hit distinct bank groups.  Scales and the group sums
-// sum_{k in g} a (for x from k_select, for act from this kernel's MODE 0
-// epilogue) are copied to LDS tables 16 groups at a time.
+// at one column hit distinct bank groups.
 #include <type_traits>
 
 #include "moe_common.h"
@@ -681,7 +683,7 @@ __global__ __launch_bounds__(256) void k_router_gemm(const uint16_t *__restrict_
         for (int ns = 0; ns < NS; ++ns) acc[ms][ns] = mfma_bf16_16x16x32(af[ms], bf[ns], acc[ms][ns]);
     }
   }
-  // lane (q, m16) of tile (ms, ns): tokens wm*32 + ms*16 + 4q + r, expert wn*64 + ns*16 + m16
+  // lane (q, m16) of tile (ms, ns): tokens wm BM/2 + 16 ms + 4 q + r, expert wn BN/2 + 16 ns + m16
 #pragma unroll
   for (int ns = 0; ns < NS; ++ns) {
     const int e = e0 + wn * (BN / 2) + ns * 16 + m16;

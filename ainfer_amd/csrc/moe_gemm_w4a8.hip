@@ -1,5 +1,5 @@
-// moe_gemm_w4a8.hip - the layer's expert GEMVs in W4A8 for more than 16
-// tokens, as a grouped int8 MFMA GEMM.
+// moe_gemm_w4a8.hip - the layer's expert GEMVs in W4A8 from 2 tokens on
+// (w4a8_gemm_at, moe_internal.h), as a grouped int8 MFMA GEMM.
 //
 // Arithmetic: Int4Gemv's (tools/cmdlist/kernels.cpp:148-201) per (token,
 // expert), bit for bit: the group dot gs = sum q * x exact in int32, its term

@@ -250,8 +250,8 @@ constexpr int DEC_MT = 4;  // token rows of the streaming items' tiles
 constexpr int FUSED_DISPATCH_MAX_T = 64;
 
 
-// ---- decode layer in two launches (moe_decode.hip), T <= DECODE_MAX_T ----
-// (every logit in the canonical order; above, approximate logits and the
+// ---- decode layer (moe_decode.hip), T <= DECODE_MAX_T ----
+// (routed by k_route_decode: every logit in the canonical order; above, approximate logits and the
 // canonical ones of the candidates)
 constexpr int DECODE_MAX_T = 16;
 // ainfer_moe_block_forward folds the RMSNorm into the decode routing kernel
@@ -315,7 +315,7 @@ hipError_t launch_act_quant_i8(const void *x, int x_dtype, int T, int K, int8_t 
                                hipStream_t s);
 hipError_t launch_int4_gemv_i8(const uint8_t *P, const void *S, int scale_dtype, const int8_t *xq,
                                const float *sq, int M, int K, int T, float *y, hipStream_t s);
-// 0 when the shape has no decode geometry (the staged path is used then)
+// 0 when the shape has no geometry for k_experts_decode (T = 2 then takes three launches)
 int decode_geometry(const ainfer_moe_shape &s, DecodeGeom *g);
 // router logits + top-k + weights + shared gate + x in MFMA order, and the
 // dispatch (tiles of DEC_MT tokens) when ds != NULL

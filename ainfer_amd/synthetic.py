@@ -1,6 +1,6 @@
 """Synthetic MoE layer configurations and their seeds.
 
-The five configurations are the benchmark's (BASELINE.json configs[0..4]).
+The five configurations are the benchmark's.
 Every tensor is a pure function of (config seed, layer, tensor id): element i
 of a tensor is drawn by the counter-based generator of ainfer_moe_fill, so
 the GPU fill and the CPU oracle's fill produce the same bits.

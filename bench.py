@@ -5,7 +5,7 @@ Headline (the JSON line's `value`): config c4, the 60-block decode step at 1
 token -- microseconds per token of the whole step (each block: RMSNorm ->
 MoE layer H4096, 512 experts, top-10, I1024 + shared expert, INT4 g128 fp16
 scales -> residual add; 200 GB of weights resident).  It is the largest
-BASELINE config that fits one GPU.  `details` adds c4 at 8 tokens, c1 decode
+configuration that fits one GPU.  `details` adds c4 at 8 tokens, c1 decode
 at 1/4/16 tokens, the c2 prefill (4096 tokens, Zipf(1.1) routing) in tokens/s
 and % of bf16 MFMA peak, c3 (64 tokens) and the W4A8 GEMV.
 
@@ -193,7 +193,7 @@ def run_gemv_w4a8(steps, copies=8, M=17408, K=5120):
 
 
 def run_c3(steps, warmup=5):
-    """H4096 E512 k10 I1024 + shared, 64 tokens (the
+    """Config c3: H4096 E512 k10 I1024 + shared, 64 tokens (the
     4-token-tile streaming kernels).  One layer is 3.3 GB, far above the
     256 MB MALL, so one copy suffices."""
     import torch
@@ -226,7 +226,7 @@ def run_c3(steps, warmup=5):
 
 
 def run_c4(steps, tokens=(1, 8), warmup=3, keep_layer0=False, stack=True):
-    """60 blocks of config 3 (RMSNorm -> MoE -> residual),
+    """Config c4: 60 blocks of c3's layer (RMSNorm -> MoE -> residual),
     one decode step = all 60 blocks in sequence on a bf16 residual stream,
     200 GB of weights resident.  The step is one ainfer_moe_stack_forward
     call (the layers' kernels replayed; from T = 5 on each layer's combine

@@ -294,7 +294,10 @@ int ainfer_moe_dispatch(const ainfer_moe_shape *shape,
  * SiLU-mul, down), row T*k + t the shared expert on token t (unused without
  * one).  The kernels and arithmetic of ainfer_moe_forward's expert stage at
  * the same T (for T <= 2 forward splits K differently; there the rows agree
- * within the layer tolerance).  No reference counterpart
+ * within the layer tolerance).  Between calls of different T a token's rows
+ * agree within that tolerance, not bit for bit: above 16 tokens the size of the
+ * call decides between the decode items (one order of additions from T = 3 on)
+ * and the grouped GEMM.  No reference counterpart
  * (the reference is dense); the per-expert MLP is decode_l0.cpp:663-674's. */
 int ainfer_moe_experts(const ainfer_moe_shape *shape,
                        const ainfer_moe_weights *weights, const void *x,
